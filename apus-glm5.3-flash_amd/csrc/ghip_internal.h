@@ -41,6 +41,16 @@ hipError_t ghip_launch_bf16_linear(const uint16_t *w, const uint16_t *x,
                                    uint16_t *y, size_t M, size_t O, size_t K,
                                    const hipEvent_t *ev, hipStream_t st);
 
+/* BF16-weight GEMM on MFMA for more rows than the GEMV passes take: K % 64
+ * == 0, 16-byte aligned w and x (ghip_bf16_gemm_fits). One launch, no
+ * workspace. e0/e1: NULL or timing events. */
+int ghip_bf16_gemm_fits(size_t M, size_t N, size_t K, const void *w, const void *x);
+hipError_t ghip_launch_bf16_gemm(const uint16_t *w, const uint16_t *x, uint16_t *y, size_t M,
+                                 size_t N, size_t K, uint32_t n_cu, hipEvent_t e0,
+                                 hipEvent_t e1, hipStream_t st);
+/* Raise its dynamic-LDS limits (once per process). */
+hipError_t ghip_bf16_gemm_init(void);
+
 /* K3 MoE decode workspace: the SwiGLU activations h handed from the
  * gate/up phase to the down phase as words of two bf16 values (the even
  * row in bits 0..15), in two buffers that alternate between launches: the
