@@ -19,7 +19,8 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
 C_SRCS = ["ghip_backend.c", "ghip_synth.c", "ghip_container.c"]
-HIP_SRCS = ["k_linear.hip", "k_gemm_bf16.hip", "k_moe.hip", "k_moe_prefill.hip", "k_synth.hip"]
+HIP_SRCS = ["k_linear.hip", "k_gemm_bf16.hip", "k_rows.hip",
+            "k_moe.hip", "k_moe_prefill.hip", "k_synth.hip"]
 
 INC = ["-I" + os.path.join(ROOT, "include"), "-I" + CSRC]
 CFLAGS = ["-std=c11", "-O2", "-Wall", "-Wextra", "-fPIC", "-ffp-contract=off",
@@ -74,7 +75,8 @@ def resource_usage(out):
 # kernels whose remarks must be present: if the compiler stops emitting the
 # resource-usage remarks, or words them differently, the gate would see
 # nothing and pass, so their absence fails the build instead
-REQUIRED_KERNELS = ("k_moe_decode", "k_pf_gemm", "k_fp8_gemv_stream", "k_fp8_gemm", "k_bf16_gemm")
+REQUIRED_KERNELS = ("k_moe_decode", "k_pf_gemm", "k_fp8_gemv_stream", "k_fp8_gemm", "k_bf16_gemm",
+                    "k_rows_gemm")
 
 
 def check_resources(usage, required=REQUIRED_KERNELS):

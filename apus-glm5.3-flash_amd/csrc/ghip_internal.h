@@ -48,8 +48,24 @@ int ghip_bf16_gemm_fits(size_t M, size_t N, size_t K, const void *w, const void 
 hipError_t ghip_launch_bf16_gemm(const uint16_t *w, const uint16_t *x, uint16_t *y, size_t M,
                                  size_t N, size_t K, uint32_t n_cu, hipEvent_t e0,
                                  hipEvent_t e1, hipStream_t st);
+/* Its estimated time in microseconds (the dispatch compares it). */
+float ghip_bf16_gemm_estimate(size_t M, size_t N, size_t K, uint32_t n_cu);
 /* Raise its dynamic-LDS limits (once per process). */
 hipError_t ghip_bf16_gemm_init(void);
+
+/* Weight-streaming linear for a few activation rows: bf != 0 BF16 weights (K
+ * % 64 == 0), else FP8 codes (K % 128 == 0) with scales and exact_dev as
+ * ghip_launch_fp8_linear; 16-byte aligned w and x (ghip_rows_fits). One
+ * launch, no workspace. e0/e1: NULL or timing events. The estimate is in
+ * microseconds. */
+int ghip_rows_fits(int bf, size_t M, size_t N, size_t K, const void *w, const void *x);
+float ghip_rows_estimate(int bf, size_t M, size_t N, size_t K, uint32_t n_cu);
+hipError_t ghip_launch_rows(int bf, const void *w, const float *scales, const uint16_t *x,
+                            uint16_t *y, size_t M, size_t N, size_t K,
+                            const uint32_t *exact_dev, uint32_t n_cu, hipEvent_t e0,
+                            hipEvent_t e1, hipStream_t st);
+/* Raise its dynamic-LDS limits (once per process). */
+hipError_t ghip_rows_init(void);
 
 /* K3 MoE decode workspace: the SwiGLU activations h handed from the
  * gate/up phase to the down phase as words of two bf16 values (the even

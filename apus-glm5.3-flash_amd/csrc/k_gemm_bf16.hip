@@ -255,7 +255,7 @@ static const BgTile bg_tiles[] = {
  * caches and the clock; measured 29.1 against 27.5 us with 160 of 256 CUs
  * busy, 35.1 with all). The estimate is within 10% of the measured time over
  * M = 32..2048, N = 288..8192 for every shape. */
-static const BgTile *bg_pick(size_t M, size_t N, uint32_t n_cu) {
+static const BgTile *bg_pick(size_t M, size_t N, uint32_t n_cu, double *est) {
     const BgTile *best = nullptr;
     double bc = 0.0;
     for (const BgTile &t : bg_tiles) {
@@ -267,6 +267,7 @@ static const BgTile *bg_pick(size_t M, size_t N, uint32_t n_cu) {
             bc = c;
         }
     }
+    *est = bc;
     return best;
 }
 
@@ -279,11 +280,22 @@ extern "C" int ghip_bf16_gemm_fits(size_t M, size_t N, size_t K, const void *w, 
         && ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & 15) == 0;
 }
 
+/* Estimated microseconds: 3 + the pick's stages scaled to K (600 x 4096: 29.1
+ * us at K = 4096, 17.1 at 2048), and no less than the weights at 5.7 TB/s
+ * (LM head, M = 12: 225 us). */
+extern "C" float ghip_bf16_gemm_estimate(size_t M, size_t N, size_t K, uint32_t n_cu) {
+    double est = 0.0;
+    (void)bg_pick(M, N, n_cu, &est);
+    const double t = (est - 2.0) * (double)K / 4096.0, hbm = 2.0 * (double)N * (double)K / 5.7e6;
+    return (float)(3.0 + (t > hbm ? t : hbm));
+}
+
 extern "C" hipError_t ghip_launch_bf16_gemm(const uint16_t *w, const uint16_t *x, uint16_t *y,
                                             size_t M, size_t N, size_t K, uint32_t n_cu,
                                             hipEvent_t e0, hipEvent_t e1, hipStream_t st) {
     if (!ghip_bf16_gemm_fits(M, N, K, w, x) || n_cu == 0) return hipErrorInvalidValue;
-    const BgTile *t = bg_pick(M, N, n_cu);
+    double est = 0.0;
+    const BgTile *t = bg_pick(M, N, n_cu, &est);
     const size_t mt = (M + t->bm - 1) / t->bm, nt = (N + t->bn - 1) / t->bn;
     t->launch((uint32_t)(mt * nt), t->lds, st, e0, e1, w, x, y, (uint32_t)M, (uint32_t)N,
               (uint32_t)K, (uint32_t)mt);

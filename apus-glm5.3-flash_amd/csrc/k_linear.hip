@@ -2,33 +2,27 @@
  * k_linear.hip — gfx950 kernels for the dense FP8-block path:
  *   K1  k_dequant16 / k_dequant_any : FP8-E4M3 + F32 128x128 scales -> BF16,
  *       bit-exact vs c/fp8blk.h:115-136 (apus_fp8blk_rows_scalar).
- *   K2  k_fp8_gemv : decode / MTP-verify GEMV (M <= 4 per launch) with the
- *       dequant fused in registers and the k reduction on MFMA
+ *   K2  k_fp8_gemv_stream : decode / MTP-verify GEMV (M <= 4, many weight
+ *       rows) with the dequant fused in registers and the k reduction on MFMA
  *       (v_mfma_f32_16x16x32_bf16), the composition of c/gdsa.h:525-534
- *       (dequant -> bf16 -> fp32-accumulated GEMM -> RNE bf16).
- *   k_fp8_linear_any / k_bf16_linear_any : shape-general fallbacks (ceil
- *       shapes, K not a multiple of 64) with the exact integer decode.
+ *       (dequant -> bf16 -> fp32-accumulated GEMM -> RNE bf16). Other row
+ *       counts and shapes: k_rows.hip, k_moe_prefill.hip (k_fp8_gemm) and,
+ *       for BF16 weights, k_rows.hip and k_gemm_bf16.hip.
+ *   k_fp8_linear_any / k_bf16_linear_any : shape-general fallbacks (K not a
+ *       multiple of 128 / 64, unaligned operands) with the exact integer
+ *       decode.
  *   k_nan_scan : flags the out-of-contract NaN codes 0x7F/0xFF so callers
  *       can select the exact decode for such weights.
  *
- * GEMV tiling (K2). A workgroup owns 16 consecutive output rows; its NW
- * waves split K into 128-wide chunks (one scale block; wave w takes chunks
- * w, w+NW, ...). Per chunk, lane l loads 32 codes of row (l % 16) at k
- * offset 32*(l / 16) (two 16-byte loads; a wave covers 16 full 128-byte
- * lines), dequantizes them to four bf16x8 operands and issues four MFMAs
- * whose A operand is x staged in LDS. The MFMA k-slot
- * to k mapping is any permutation used identically for A and B, so the
- * result is an exact-product fp32 sum in a different order than the
+ * The MFMA k-slot to k mapping is any permutation used identically for A and
+ * B, so a result is an exact-product fp32 sum in a different order than the
  * reference's sequential k: a tolerance-class result, per the contract.
- * Partial sums of the NW waves are combined in LDS in a fixed order, so the
- * output is deterministic run to run.
+ * Partial sums of waves are combined in LDS in a fixed order, so outputs are
+ * deterministic run to run.
  */
 #include "ghip_device.h"
 #include <type_traits>
 #include "ghip_internal.h"
-
-#define GEMV_NW 8          /* waves per workgroup (k split) */
-#define GEMV_U 4           /* 128-wide chunks (2 loads each) per batch */
 
 /* ------------------------------------------------------------------------ */
 /* K1: dequant                                                              */
@@ -84,97 +78,6 @@ __global__ __launch_bounds__(256) void k_nan_scan(
         for (size_t i = (nv << 4) + threadIdx.x; i < n; i += 256)
             hit |= ((p[i] & 0x7fu) == 0x7fu);
     if (hit) atomicOr(flag, 1u);
-}
-
-/* ------------------------------------------------------------------------ */
-/* K2: FP8 GEMV, M <= 4, K % 128 == 0                                       */
-/* ------------------------------------------------------------------------ */
-
-/* One batch of a wave's chunk loads: chunks c0, c0 + NW, ... (GEMV_U of
- * them). The first batch is issued before x is staged so the two latencies
- * overlap. */
-__device__ __forceinline__ void gemv16_fetch(const uint8_t *__restrict__ wr,
-                                             uint32_t nch, uint32_t c0,
-                                             ghip_chunk *buf) {
-    /* unconditional (chunk clamped; the compute loop skips c >= nch) so the
-     * waitcnt pass sees a fixed number of loads */
-#pragma unroll
-    for (int u = 0; u < GEMV_U; u++) {
-        uint32_t c = min(c0 + u * GEMV_NW, nch - 1u);
-        buf[u] = ghip_chunk_load(wr + (size_t)c * 128);
-    }
-}
-
-/* buf holds the first batch on entry and is refilled in place. */
-/* sc holds the first batch's scales (fetched with the weights). */
-template <bool EXACT>
-__device__ __forceinline__ ghip_f32x4 gemv16_rows(
-    const uint8_t *__restrict__ wr, const float *__restrict__ srow,
-    const uint16_t *xa, uint32_t nch, uint32_t wv, ghip_chunk (&buf)[GEMV_U],
-    const float (&sc)[GEMV_U]) {
-    ghip_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (uint32_t c0 = wv; c0 < nch; c0 += GEMV_NW * GEMV_U) {
-        float s2[GEMV_U];
-        if (c0 != wv) {
-            gemv16_fetch(wr, nch, c0, buf);
-#pragma unroll
-            for (int u = 0; u < GEMV_U; u++) s2[u] = srow[min(c0 + u * GEMV_NW, nch - 1u)];
-        } else {
-#pragma unroll
-            for (int u = 0; u < GEMV_U; u++) s2[u] = sc[u];
-        }
-#pragma unroll
-        for (int u = 0; u < GEMV_U; u++) {
-            uint32_t c = c0 + u * GEMV_NW;
-            if (c < nch) ghip_chunk_mfma<EXACT>(buf[u], s2[u], xa + c * 128, acc);
-        }
-    }
-    return acc;
-}
-
-template <int M>
-__global__ __launch_bounds__(GEMV_NW * 64, 4) void k_fp8_gemv(
-    const uint8_t *__restrict__ W, const float *__restrict__ S,
-    const uint16_t *__restrict__ X, uint16_t *__restrict__ Y, uint32_t O,
-    uint32_t K, uint32_t nkb, const uint32_t *__restrict__ exact_flag) {
-    extern __shared__ __align__(16) uint16_t xs[];     /* M x K */
-    __shared__ float red[GEMV_NW][M][16];
-    const uint32_t tid = threadIdx.x, lane = tid & 63;
-    const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t row0 = blockIdx.x * 16u;
-    const uint32_t n = lane & 15u, g = lane >> 4;
-    const uint32_t row = min(row0 + n, O - 1u);
-    const uint8_t *wr = W + (size_t)row * K + 32u * g;
-    const uint32_t nch = K >> 7;
-    /* this wave's x slices first, then the weights, then the slices into
-     * LDS (ghip_wstage_*: no workgroup barrier) */
-    ghip_stage stx;
-    ghip_wstage_load(stx, X, M, K, nch, wv, GEMV_NW, lane);
-    ghip_chunk pre[GEMV_U];
-    gemv16_fetch(wr, nch, wv, pre);
-    const float *srow = S + (size_t)(row0 >> 7) * nkb;
-    float sc[GEMV_U];
-#pragma unroll
-    for (int u = 0; u < GEMV_U; u++) sc[u] = srow[min(wv + u * GEMV_NW, nch - 1u)];
-    const bool exact = exact_flag != nullptr && *exact_flag != 0u;
-    ghip_wstage_store(stx, xs, X, M, K, nch, wv, GEMV_NW, lane);
-    /* MFMA A row i = lane % 16 is token m; rows m >= M only feed output
-     * rows that are discarded, so they read row M-1 instead of zeros. */
-    const uint16_t *xa = xs + (size_t)min(n, (uint32_t)M - 1u) * K + 32u * g;
-    ghip_f32x4 acc = exact ? gemv16_rows<true>(wr, srow, xa, nch, wv, pre, sc)
-                           : gemv16_rows<false>(wr, srow, xa, nch, wv, pre, sc);
-    if (g == 0) {
-#pragma unroll
-        for (int i = 0; i < M; i++) red[wv][i][n] = acc[i];
-    }
-    __syncthreads();
-    if (tid < (uint32_t)M * 16u) {
-        uint32_t m = tid >> 4, nn = tid & 15u;
-        float s = 0.0f;
-#pragma unroll
-        for (int w = 0; w < GEMV_NW; w++) s += red[w][m][nn];
-        if (row0 + nn < O) Y[(size_t)m * O + row0 + nn] = (uint16_t)ghip_bf16_bits(s);
-    }
 }
 
 /* ------------------------------------------------------------------------ */
@@ -268,39 +171,35 @@ extern "C" hipError_t ghip_launch_nan_scan(const uint8_t *codes, size_t n,
 }
 
 /* ------------------------------------------------------------------------ */
-/* K2 streaming: persistent FP8 / BF16 GEMV, register-load chunk streams   */
+/* K2: persistent FP8 GEMV, M <= 4, x staged once, weights streamed         */
 /* ------------------------------------------------------------------------ */
 
 #define GS_NW 8                  /* waves per workgroup */
 /* LDS chunk slots per wave: a chunk is written from registers and read
- * back in the MFMA layout while the next ones are in flight: two for FP8
- * weights (measured: one 13.8 us, two 12.3, three 12.6 on config 1), three
- * for BF16 (the LM head: two 226 us, three 208) */
-#define GS_R 3
+ * back in the MFMA layout while the next one is in flight (measured on
+ * 16384 x 4096: one 13.8 us, two 12.3, three 12.6) */
+#define GS_R 2
+#define GS_X_MAX (48u * 1024u)   /* most bytes of x staged (K <= 6144 at M = 4) */
 #define GS_LDS (144u * 1024u)    /* dynamic LDS limit of the streaming GEMV */
 
 /* Y[m, rows] for M <= 4 token rows. A row group (16 weight rows) is split
- * over KS waves along K (KS in {2, 8}); a workgroup pass covers 8 / KS row
- * groups, passes run over the groups persistently (grid <= CUs). Each wave
- * streams its chunks (16 rows x 128 bytes: 128 FP8 codes with one scale
- * block, or 64 BF16 weights when BF) through registers: two 16-byte loads
- * per lane in a whole-line pattern (load i: rows 8i + lane / 8, piece lane
- * % 8), two chunks in flight, each chunk written to a wave-private 2-slot
- * LDS area (lane l's bytes at 16 l, piece p of row r at p ^ ((r >> 1) & 7))
- * and read back in the MFMA layout, dequantized in registers (FP8) and
- * reduced on MFMA with the token rows of x (staged once per workgroup) as
- * the A operand: A row i = lane % 16 is token min(i, M-1), rows past M feed
- * output rows that are discarded. The KS partial sums of a group are added
- * in LDS in a fixed order (deterministic). BF: the BF16 GEMV of the
- * bf16_gemm hook (c/bf16.h:712-767), no scales; lane 16g + n holds row n,
- * weights [16g, 16g + 16) of the chunk, two v_mfma_f32_16x16x32_bf16 with
- * x at the same k. */
-template <int M, int KS, bool BF = false>
+ * over two waves along K; a workgroup pass covers 4 row groups, passes run
+ * over the groups persistently (one workgroup per CU). Each wave streams its
+ * chunks (16 rows x 128 codes, one scale block) through registers: two
+ * 16-byte loads per lane in a whole-line pattern (load i: rows 8i + lane /
+ * 8, piece lane % 8), two chunks in flight, each chunk written to a
+ * wave-private LDS slot (lane l's bytes at 16 l, piece p of row r at p ^
+ * ((r >> 1) & 7)) and read back in the MFMA layout, dequantized in registers
+ * and reduced on MFMA with the token rows of x (staged once per workgroup)
+ * as the A operand: A row i = lane % 16 is token min(i, M-1), rows past M
+ * feed output rows that are discarded. The two partial sums of a group are
+ * added in LDS in a fixed order (deterministic). */
+template <int M>
 __global__ __launch_bounds__(GS_NW * 64, 1) void k_fp8_gemv_stream(
     const uint8_t *__restrict__ W, const float *__restrict__ S,
     const uint16_t *__restrict__ X, uint16_t *__restrict__ Y, uint32_t O,
     uint32_t K, const uint32_t *__restrict__ exact_flag) {
-    constexpr uint32_t GPP = GS_NW / KS;             /* row groups per pass */
+    constexpr uint32_t KS = 2, GPP = GS_NW / KS;     /* K splits, row groups per pass */
     extern __shared__ __attribute__((aligned(1024))) uint8_t gsl[];
     __shared__ float red[GPP][KS][M][16];
     uint16_t *xs = (uint16_t *)gsl;
@@ -309,40 +208,33 @@ __global__ __launch_bounds__(GS_NW * 64, 1) void k_fp8_gemv_stream(
     const uint32_t n = lane & 15u, g = lane >> 4;
     uint8_t *ring = gsl + (((size_t)M * K * 2u + 1023u) & ~(size_t)1023u) +
                     wv * (GS_R * 2048u);
-    /* chunk = 128 bytes of each of 16 rows; row stride in bytes */
-    const uint32_t KB = BF ? 2u * K : K;
-    const uint32_t nch = KB >> 7, nkb = K >> 7;
+    const uint32_t nch = K >> 7, nkb = K >> 7;
     const uint32_t part = wv % KS, slot = wv / KS;
     const uint32_t c0 = part * nch / KS, c1 = (part + 1) * nch / KS, nc = c1 - c0;
     const uint32_t groups = (O + 15) / 16, passes = (groups + GPP - 1) / GPP;
-    const uint16_t *xa = xs + (size_t)min(n, (uint32_t)M - 1u) * K + (BF ? 16u : 32u) * g;
+    const uint16_t *xa = xs + (size_t)min(n, (uint32_t)M - 1u) * K + 32u * g;
     /* pass ps's row group of this wave: its rows and load offsets (a
      * partial last group re-reads row O-1, outputs discarded) */
     auto rows_of = [&](uint32_t ps) {
-        return W + (size_t)(ps * GPP + slot) * 16u * KB;
+        return W + (size_t)(ps * GPP + slot) * 16u * K;
     };
     auto offs_of = [&](uint32_t ps) {
-        return ghip_cdma_offsets(lane, KB, min(15u, O - 1u - (ps * GPP + slot) * 16u));
+        return ghip_cdma_offsets(lane, K, min(15u, O - 1u - (ps * GPP + slot) * 16u));
     };
-    /* NA chunks in flight: chunk t's two 16-byte pieces in register set
-     * t % NA ((ra0, ra1), (rb0, rb1), (rc0, rc1)) and LDS slot t % NA */
-    constexpr uint32_t NA = BF ? 3u : 2u;
-    ghip_u32x4 ra0, ra1, rb0, rb1, rc0, rc1;
-    /* the first NA chunks of a pass, always all loaded (chunk indices
+    /* two chunks in flight: chunk t's two 16-byte pieces in register set t % 2
+     * ((ra0, ra1), (rb0, rb1)) and LDS slot t % 2 */
+    ghip_u32x4 ra0, ra1, rb0, rb1;
+    /* the first two chunks of a pass, always both loaded (chunk indices
      * clamped): a fixed count of loads in flight, in a fixed order */
     auto prefetch = [&](const uint8_t *rows, const ghip_cdma &d) {
         ghip_rl_load(rows, d, min(c0, nch - 1u), ra0, ra1);
         __builtin_amdgcn_sched_barrier(0);
         ghip_rl_load(rows, d, min(c0 + 1u, nch - 1u), rb0, rb1);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (NA == 3u) {
-            ghip_rl_load(rows, d, min(c0 + 2u, nch - 1u), rc0, rc1);
-            __builtin_amdgcn_sched_barrier(0);
-        }
     };
     /* x into LDS without delaying the weight stream: x goes by direct DMA
-     * (1 KB pieces dealt to the waves, lanes past x re-read its last vector
-     * into the 1 KB-rounded x region) ahead of the first pass's 2 NA chunk
+     * (1 K pieces dealt to the waves, lanes past x re-read its last vector
+     * into the 1 K-rounded x region) ahead of the first pass's four chunk
      * loads, so waiting until no more than those are in flight means this
      * wave's x pieces have landed */
     {
@@ -350,95 +242,62 @@ __global__ __launch_bounds__(GS_NW * 64, 1) void k_fp8_gemv_stream(
         for (uint32_t c = wv; c < nxc; c += GS_NW)
             ghip_dma16(X + (size_t)min(c * 64u + lane, nvec - 1u) * 8u, gsl + c * 1024u);
         const uint32_t grp0 = min(blockIdx.x * GPP + slot, groups - 1u);
-        prefetch(W + (size_t)grp0 * 16u * KB,
-               ghip_cdma_offsets(lane, KB, min(15u, O - 1u - grp0 * 16u)));
-        GHIP_VMCNT(2 * NA);
+        prefetch(W + (size_t)grp0 * 16u * K,
+               ghip_cdma_offsets(lane, K, min(15u, O - 1u - grp0 * 16u)));
+        GHIP_VMCNT(4);
     }
     /* a bare barrier: __syncthreads() would also wait for the chunk loads
      * (its workgroup-scope release waits for every load in flight) */
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    const bool exact = !BF && exact_flag != nullptr && *exact_flag != 0u;
+    const bool exact = exact_flag != nullptr && *exact_flag != 0u;
     for (uint32_t ps = blockIdx.x; ps < passes; ps += gridDim.x) {
         const uint32_t grp = ps * GPP + slot;
         const bool live = grp < groups;
         if (live) {
-            /* a wave with no chunks (K < KS * 128) contributes zeros */
+            /* a wave with no chunks (K < 256) contributes zeros */
             const uint32_t row0 = grp * 16;
             const uint8_t *rows = rows_of(ps);
             const ghip_cdma d = offs_of(ps);
-            const float *srow = BF ? nullptr : S + (size_t)(row0 >> 7) * nkb;
+            const float *srow = S + (size_t)(row0 >> 7) * nkb;
             if (ps != blockIdx.x) prefetch(rows, d);
             ghip_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            /* chunk t: its registers into LDS slot t % NA, the registers
-             * refilled with chunk t + NA (REFILL), the chunk read back in
+            /* chunk t: its registers into LDS slot t % 2, the registers
+             * refilled with chunk t + 2 (REFILL), the chunk read back in
              * the MFMA layout with this lane's activations and the scale */
             auto step = [&](auto refill_c, uint32_t t, ghip_u32x4 &v0, ghip_u32x4 &v1,
                             uint8_t *buf) {
                 ghip_rl_store(buf, lane, v0, v1);
                 if constexpr (decltype(refill_c)::value) {
                     __builtin_amdgcn_sched_barrier(0);
-                    ghip_rl_load(rows, d, c0 + t + NA, v0, v1);
+                    ghip_rl_load(rows, d, c0 + t + 2u, v0, v1);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 const uint32_t c = c0 + t;
                 const ghip_chunk cw = ghip_cdma_read(buf, n, g);
-                if constexpr (BF) {
-                    const ghip_bf16x8 *a = (const ghip_bf16x8 *)(xa + c * 64u);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        a[0], __builtin_bit_cast(ghip_bf16x8, cw.lo), acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        a[1], __builtin_bit_cast(ghip_bf16x8, cw.hi), acc, 0, 0, 0);
-                } else {
-                    ghip_bf16x8 a4[4];
-                    ghip_read_a4(xa + c * 128u, a4);
-                    const float sc = ghip_sload(srow, c);
-                    if (exact) ghip_chunk_mfma_a<true>(cw, sc, a4, acc);
-                    else ghip_chunk_mfma_a<false>(cw, sc, a4, acc);
-                }
+                ghip_bf16x8 a4[4];
+                ghip_read_a4(xa + c * 128u, a4);
+                const float sc = ghip_sload(srow, c);
+                if (exact) ghip_chunk_mfma_a<true>(cw, sc, a4, acc);
+                else ghip_chunk_mfma_a<false>(cw, sc, a4, acc);
             };
             using RF = std::true_type;
             using NR = std::false_type;
             uint32_t t = 0;
-            if constexpr (NA == 2u) {
-                for (; t + 3u < nc; t += 2) {
-                    step(RF{}, t, ra0, ra1, ring);
-                    step(RF{}, t + 1u, rb0, rb1, ring + 2048u);
-                }
-                if (nc - t == 3u) {
-                    step(RF{}, t, ra0, ra1, ring);
-                    step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
-                    step(NR{}, t + 2u, ra0, ra1, ring);
-                } else if (nc - t == 2u) {
-                    step(NR{}, t, ra0, ra1, ring);
-                    step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
-                } else if (nc - t == 1u) {
-                    step(NR{}, t, ra0, ra1, ring);
-                }
-            } else {
-                for (; t + 5u < nc; t += 3) {
-                    step(RF{}, t, ra0, ra1, ring);
-                    step(RF{}, t + 1u, rb0, rb1, ring + 2048u);
-                    step(RF{}, t + 2u, rc0, rc1, ring + 4096u);
-                }
-                const uint32_t rem = nc - t;
-                if (rem == 5u) {
-                    step(RF{}, t, ra0, ra1, ring);
-                    step(RF{}, t + 1u, rb0, rb1, ring + 2048u);
-                    step(NR{}, t + 2u, rc0, rc1, ring + 4096u);
-                    step(NR{}, t + 3u, ra0, ra1, ring);
-                    step(NR{}, t + 4u, rb0, rb1, ring + 2048u);
-                } else if (rem == 4u) {
-                    step(RF{}, t, ra0, ra1, ring);
-                    step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
-                    step(NR{}, t + 2u, rc0, rc1, ring + 4096u);
-                    step(NR{}, t + 3u, ra0, ra1, ring);
-                } else {
-                    if (rem > 0u) step(NR{}, t, ra0, ra1, ring);
-                    if (rem > 1u) step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
-                    if (rem > 2u) step(NR{}, t + 2u, rc0, rc1, ring + 4096u);
-                }
+            for (; t + 3u < nc; t += 2) {
+                step(RF{}, t, ra0, ra1, ring);
+                step(RF{}, t + 1u, rb0, rb1, ring + 2048u);
+            }
+            if (nc - t == 3u) {
+                step(RF{}, t, ra0, ra1, ring);
+                step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
+                step(NR{}, t + 2u, ra0, ra1, ring);
+            } else if (nc - t == 2u) {
+                step(NR{}, t, ra0, ra1, ring);
+                step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
+            } else if (nc - t == 1u) {
+                step(NR{}, t, ra0, ra1, ring);
             }
             if (g == 0) {
 #pragma unroll
@@ -472,40 +331,24 @@ static size_t gs_lds(size_t M, size_t K) {
 }
 
 template <int M>
-static hipError_t launch_gemv_m(const uint8_t *codes, const float *scales,
-                                const uint16_t *x, uint16_t *y, size_t O,
-                                size_t K, const uint32_t *exact_dev,
+static hipError_t launch_gemv_m(const uint8_t *codes, const float *scales, const uint16_t *x,
+                                uint16_t *y, size_t O, size_t K, const uint32_t *exact_dev,
                                 hipEvent_t ev0, hipEvent_t ev1, hipStream_t st) {
-    const size_t groups = (O + 15) / 16;
-    if (g_gs_ncu && gs_lds(M, K) <= GS_LDS) {
-        const size_t lds = gs_lds(M, K);
-        if ((groups + 3) / 4 >= g_gs_ncu) {          /* KS = 2: 4 groups a pass */
-            uint32_t g = (uint32_t)((groups + 3) / 4);
-            if (g > g_gs_ncu) g = g_gs_ncu;
-            GHIP_LAUNCH(ev0, ev1, (k_fp8_gemv_stream<M, 2>), dim3(g), dim3(GS_NW * 64),
-                        lds, st, codes, scales, x, y, (uint32_t)O, (uint32_t)K, exact_dev);
-        } else {                                       /* KS = 8: 1 group a pass */
-            uint32_t g = (uint32_t)groups;
-            if (g > g_gs_ncu) g = g_gs_ncu;
-            GHIP_LAUNCH(ev0, ev1, (k_fp8_gemv_stream<M, 8>), dim3(g), dim3(GS_NW * 64),
-                        lds, st, codes, scales, x, y, (uint32_t)O, (uint32_t)K, exact_dev);
-        }
-        return hipGetLastError();
-    }
-    size_t lds = (size_t)M * K * 2;
-    uint32_t nkb = (uint32_t)((K + 127) / 128);
-    uint32_t g = (uint32_t)groups;
-    GHIP_LAUNCH(ev0, ev1, k_fp8_gemv<M>, dim3(g), dim3(GEMV_NW * 64), lds, st,
-                codes, scales, x, y, (uint32_t)O, (uint32_t)K, nkb, exact_dev);
+    GHIP_LAUNCH(ev0, ev1, k_fp8_gemv_stream<M>, dim3(g_gs_ncu), dim3(GS_NW * 64), gs_lds(M, K), st,
+                codes, scales, x, y, (uint32_t)O, (uint32_t)K, exact_dev);
     return hipGetLastError();
 }
 
-/* Rows of X from which the FP8 linear runs as one GEMM (below: GEMV passes
- * of <= 4 rows, each reading the weights once). */
+/* Rows of X from which the MFMA GEMM (N % 256 == 0) is considered. */
 #define GHIP_GEMM_MIN_M 16
 
-/* Largest dynamic LDS the GEMV stages x into (per workgroup). */
-#define GEMV_LDS_MAX (48u * 1024u)
+/* Estimated microseconds of ghip_launch_fp8_gemm below 256 rows (two
+ * launches, K split): 11 + the weights at 6 TB/s + 0.04 a row. Measured q_a
+ * 1536 x 4096 14.6 us at M = 64, o_proj 4096 x 16384 22.2 at 16 and 31.4 at
+ * 128, q_b 16384 x 1536 20.5 at 96. */
+static float fp8_gemm_estimate(size_t M, size_t O, size_t K) {
+    return 11.0f + (float)((double)O * (double)K / 6.0e6) + 0.04f * (float)M;
+}
 
 extern "C" hipError_t ghip_launch_fp8_linear(const uint8_t *codes,
                                              const float *scales,
@@ -519,9 +362,7 @@ extern "C" hipError_t ghip_launch_fp8_linear(const uint8_t *codes,
         return hipErrorInvalidValue;
     /* timing events: start on the first launch, stop on the last */
     hipEvent_t ev0 = ev ? ev[0] : nullptr, ev1 = ev ? ev[1] : nullptr;
-    bool fast = (K % 128 == 0) && (((uintptr_t)codes & 15) == 0)
-             && (((uintptr_t)x & 15) == 0) && K * 2 <= GEMV_LDS_MAX;
-    if (!fast) {
+    if (!g_gs_ncu || !ghip_rows_fits(0, M, O, K, codes, x)) {
         uint32_t nkb = (uint32_t)((K + 127) / 128);
         size_t items = M * O;
         if (items > 0xffffffffull * 4) return hipErrorInvalidValue;
@@ -530,57 +371,24 @@ extern "C" hipError_t ghip_launch_fp8_linear(const uint8_t *codes,
                     (uint32_t)O, (uint32_t)K, nkb);
         return hipGetLastError();
     }
-    /* from GHIP_GEMM_MIN_M rows on, the weights are read once by the MFMA
-     * GEMM instead of once per group of <= 4 rows */
-    if (M >= GHIP_GEMM_MIN_M && g_gs_ncu && ghip_fp8_gemm_fits(M, O, K, codes, x, y))
+    /* up to 4 rows against enough weight rows that every wave holds a row
+     * group for half of K: x staged once in LDS (16384 x 4096, M = 1: 11.6 us
+     * against 12.0 with x streamed beside the weights; 16384 x 1536: 5.9
+     * against 6.2; below that many rows the streamed form is as good or
+     * better, 7000 x 2048 4.9 against 6.0) */
+    if (M <= 4 && (O + 63) / 64 >= g_gs_ncu && M * K * 2 <= GS_X_MAX) {
+        switch (M) {
+        case 4: return launch_gemv_m<4>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
+        case 3: return launch_gemv_m<3>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
+        case 2: return launch_gemv_m<2>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
+        default: return launch_gemv_m<1>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
+        }
+    }
+    if (M >= GHIP_GEMM_MIN_M && ghip_fp8_gemm_fits(M, O, K, codes, x, y)
+        && (M >= 256 || fp8_gemm_estimate(M, O, K) < ghip_rows_estimate(0, M, O, K, g_gs_ncu)))
         return ghip_launch_fp8_gemm(codes, scales, x, y, M, O, K, exact_dev, g_gs_ncu, ev,
                                     st);
-    /* m-groups of up to 4 rows, each as large as the x staging allows */
-    size_t m0 = 0;
-    while (m0 < M) {
-        size_t mc = M - m0;
-        if (mc > 4) mc = 4;
-        while (mc > 1 && mc * K * 2 > GEMV_LDS_MAX) mc--;
-        const uint16_t *xm = x + m0 * K;
-        uint16_t *ym = y + m0 * O;
-        hipEvent_t a = m0 == 0 ? ev0 : nullptr, b = m0 + mc == M ? ev1 : nullptr;
-        hipError_t e;
-        switch (mc) {
-        case 4: e = launch_gemv_m<4>(codes, scales, xm, ym, O, K, exact_dev, a, b, st); break;
-        case 3: e = launch_gemv_m<3>(codes, scales, xm, ym, O, K, exact_dev, a, b, st); break;
-        case 2: e = launch_gemv_m<2>(codes, scales, xm, ym, O, K, exact_dev, a, b, st); break;
-        default: e = launch_gemv_m<1>(codes, scales, xm, ym, O, K, exact_dev, a, b, st); break;
-        }
-        if (e != hipSuccess) return e;
-        m0 += mc;
-    }
-    return hipSuccess;
-}
-
-/* Rows of X from which the BF16 linear runs as one GEMM: its shortest launch
- * takes 15.4 us at K = 4096, two GEMV passes (M <= 8) 13.3 us at N = 4096 and
- * 8.7 at N = 288, three 19 and 13. */
-#define GHIP_BF16_GEMM_MIN_M 9
-
-template <int M>
-static hipError_t launch_bf16_gemv_m(const uint16_t *w, const uint16_t *x, uint16_t *y,
-                                     size_t O, size_t K, hipEvent_t ev0, hipEvent_t ev1,
-                                     hipStream_t st) {
-    const size_t groups = (O + 15) / 16;
-    const size_t lds = gs_lds(M, K);
-    const uint8_t *wb = (const uint8_t *)w;
-    if ((groups + 3) / 4 >= g_gs_ncu) {              /* KS = 2: 4 groups a pass */
-        uint32_t g = (uint32_t)((groups + 3) / 4);
-        if (g > g_gs_ncu) g = g_gs_ncu;
-        GHIP_LAUNCH(ev0, ev1, (k_fp8_gemv_stream<M, 2, true>), dim3(g), dim3(GS_NW * 64),
-                    lds, st, wb, nullptr, x, y, (uint32_t)O, (uint32_t)K, nullptr);
-    } else {                                           /* KS = 8: 1 group a pass */
-        uint32_t g = (uint32_t)groups;
-        if (g > g_gs_ncu) g = g_gs_ncu;
-        GHIP_LAUNCH(ev0, ev1, (k_fp8_gemv_stream<M, 8, true>), dim3(g), dim3(GS_NW * 64),
-                    lds, st, wb, nullptr, x, y, (uint32_t)O, (uint32_t)K, nullptr);
-    }
-    return hipGetLastError();
+    return ghip_launch_rows(0, codes, scales, x, y, M, O, K, exact_dev, g_gs_ncu, ev0, ev1, st);
 }
 
 extern "C" hipError_t ghip_launch_bf16_linear(const uint16_t *w,
@@ -590,34 +398,19 @@ extern "C" hipError_t ghip_launch_bf16_linear(const uint16_t *w,
     if (M == 0 || O == 0) return hipSuccess;
     if (K == 0 || O > 0x7fffffffu || K > 0x7fffffffu || M > 0x7fffffffu)
         return hipErrorInvalidValue;
-    /* timing events: start on the first launch, stop on the last */
     hipEvent_t ev0 = ev ? ev[0] : nullptr, ev1 = ev ? ev[1] : nullptr;
-    /* from GHIP_BF16_GEMM_MIN_M rows on, one GEMM that reads the weights once */
-    if (M >= GHIP_BF16_GEMM_MIN_M && g_gs_ncu && ghip_bf16_gemm_fits(M, O, K, w, x))
-        return ghip_launch_bf16_gemm(w, x, y, M, O, K, g_gs_ncu, ev0, ev1, st);
-    /* the streaming MFMA GEMV, in groups of <= 4 token rows (each reading
-     * the weights once), when the shape and alignment allow */
-    if (g_gs_ncu && K % 64 == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & 15) == 0
-        && gs_lds(1, K) <= GS_LDS) {
-        size_t m0 = 0;
-        while (m0 < M) {
-            size_t mc = M - m0;
-            if (mc > 4) mc = 4;
-            while (mc > 1 && gs_lds(mc, K) > GS_LDS) mc--;
-            const uint16_t *xm = x + m0 * K;
-            uint16_t *ym = y + m0 * O;
-            hipEvent_t a = m0 == 0 ? ev0 : nullptr, b = m0 + mc == M ? ev1 : nullptr;
-            hipError_t e;
-            switch (mc) {
-            case 4: e = launch_bf16_gemv_m<4>(w, xm, ym, O, K, a, b, st); break;
-            case 3: e = launch_bf16_gemv_m<3>(w, xm, ym, O, K, a, b, st); break;
-            case 2: e = launch_bf16_gemv_m<2>(w, xm, ym, O, K, a, b, st); break;
-            default: e = launch_bf16_gemv_m<1>(w, xm, ym, O, K, a, b, st); break;
-            }
-            if (e != hipSuccess) return e;
-            m0 += mc;
-        }
-        return hipSuccess;
+    if (g_gs_ncu) {
+        /* the weight-streaming form reads the weights once per row tile, the
+         * GEMM's tiles share them: whichever is estimated faster (4096 x
+         * 4096: 12.3 against 15.5 us at M = 64, 20.2 against 15.9 at 96) */
+        const bool rows = ghip_rows_fits(1, M, O, K, w, x);
+        if (ghip_bf16_gemm_fits(M, O, K, w, x)
+            && (!rows || ghip_bf16_gemm_estimate(M, O, K, g_gs_ncu)
+                             < ghip_rows_estimate(1, M, O, K, g_gs_ncu)))
+            return ghip_launch_bf16_gemm(w, x, y, M, O, K, g_gs_ncu, ev0, ev1, st);
+        if (rows)
+            return ghip_launch_rows(1, w, nullptr, x, y, M, O, K, nullptr, g_gs_ncu, ev0, ev1,
+                                    st);
     }
     size_t items = M * O;
     if (items > 0xffffffffull * 4) return hipErrorInvalidValue;
@@ -626,25 +419,15 @@ extern "C" hipError_t ghip_launch_bf16_linear(const uint16_t *w,
     return hipGetLastError();
 }
 
-template <int M>
-static hipError_t gs_attr(void) {
-    const void *ks[4] = {(const void *)k_fp8_gemv_stream<M, 2>,
-                         (const void *)k_fp8_gemv_stream<M, 8>,
-                         (const void *)k_fp8_gemv_stream<M, 2, true>,
-                         (const void *)k_fp8_gemv_stream<M, 8, true>};
-    for (int i = 0; i < 4; i++) {
-        hipError_t e = hipFuncSetAttribute(ks[i], hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           GS_LDS);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
-}
-
 extern "C" hipError_t ghip_linear_init(uint32_t n_cu) {
+    const void *ks[4] = {(const void *)k_fp8_gemv_stream<1>, (const void *)k_fp8_gemv_stream<2>,
+                         (const void *)k_fp8_gemv_stream<3>, (const void *)k_fp8_gemv_stream<4>};
     hipError_t e;
-    if ((e = gs_attr<1>()) != hipSuccess || (e = gs_attr<2>()) != hipSuccess
-        || (e = gs_attr<3>()) != hipSuccess || (e = gs_attr<4>()) != hipSuccess)
-        return e;
+    for (int i = 0; i < 4; i++)
+        if ((e = hipFuncSetAttribute(ks[i], hipFuncAttributeMaxDynamicSharedMemorySize, GS_LDS))
+            != hipSuccess)
+            return e;
+    if ((e = ghip_rows_init()) != hipSuccess) return e;
     if ((e = ghip_bf16_gemm_init()) != hipSuccess) return e;
     g_gs_ncu = n_cu;
     return hipSuccess;

@@ -700,7 +700,7 @@ def bench_bf16_gemv(lib, pkg, rt, steps, warmup, M=1, copies=2):
     for i in range(warmup):
         step(i)
     ms = timed(rt, st, step, warmup, steps)
-    kname = "k_fp8_gemv_stream<%d, 2, true>" % min(M, 4)
+    kname = "k_rows_gemm"
     kt = kernel_times(lib, rt, step, warmup + steps, steps, 2, {kname: (0, 1)})
     nbytes = N * K * 2 + M * K * 2 + M * N * 2
     return {"ms_per_step": ms, "value": nbytes / (ms * 1e-3) / 1e9,

@@ -15,13 +15,13 @@ from tolerance import assert_close
 pytestmark = pytest.mark.gpu
 
 # (M, N, K): the tile the launcher picks on 256 CUs
-SHAPES = [(9, 64, 64), (33, 200, 576), (100, 300, 1088),     # 64 x 64
+SHAPES = [(65, 8000, 64), (250, 2005, 128), (130, 4100, 1088),  # 64 x 64
           (64, 20000, 192), (320, 4000, 448),                 # 64 x 128
           (600, 4096, 320),                                   # 192 x 64
           (1023, 4095, 128), (1024, 4096, 704),               # 128 x 128
           (1100, 4104, 256),                                  # 192 x 128
           (2047, 4096, 320),                                  # 256 x 128
-          (2048, 8200, 192)]                                  # 256 x 256
+          (2048, 8185, 192)]                                  # 256 x 256
 
 
 def run(ghip, w, x, pad):
@@ -51,8 +51,8 @@ def test_bf16_gemm_tiles(ghip, M, N, K):
 def test_bf16_gemm_unaligned_y(ghip):
     """y two bytes off a 16-byte boundary: the same values by 2-byte stores."""
     rng = np.random.default_rng(11)
-    w = O.f32_to_bf16(rng.uniform(-4, 4, (264, 256)).astype(np.float32))
-    x = O.f32_to_bf16(rng.uniform(-4, 4, (70, 256)).astype(np.float32))
+    w = O.f32_to_bf16(rng.uniform(-4, 4, (2056, 256)).astype(np.float32))
+    x = O.f32_to_bf16(rng.uniform(-4, 4, (250, 256)).astype(np.float32))
     assert np.array_equal(run(ghip, w, x, 1), run(ghip, w, x, 8))
 
 
@@ -60,7 +60,7 @@ def test_bf16_gemm_not_finite(ghip):
     """An infinity and a NaN reach exactly their own row or column (rows past
     M and N re-read the last one and are not stored)."""
     rng = np.random.default_rng(12)
-    M, N, K = 70, 100, 128
+    M, N, K = 250, 2050, 128
     w = O.f32_to_bf16(rng.uniform(1, 4, (N, K)).astype(np.float32))
     x = O.f32_to_bf16(rng.uniform(1, 4, (M, K)).astype(np.float32))
     x[M - 1, 5], w[N - 1, 7] = 0x7F80, 0x7FC0                       # +inf, NaN
