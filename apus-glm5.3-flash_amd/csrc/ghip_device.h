@@ -13,8 +13,9 @@
  *     v_cvt_pk_bf16_f32 (RNE). Used for weights with no NaN code; the GPU
  *     gate (tests/test_gpu_dequant.py) checks it on every finite code x
  *     scale corners, including subnormal products.
- *   - EXACT: integer decode (NaN codes -> +-480, as the reference) and the
- *     integer RNE narrow. Used when a matrix holds a 0x7F/0xFF code.
+ *   - EXACT: the same with the NaN codes replaced by +-480 (as the
+ *     reference). Used when a matrix holds a 0x7F/0xFF code. The dequant
+ *     entry's exact form is all integer (ghip_deq4_int).
  */
 #ifndef GHIP_DEVICE_H
 #define GHIP_DEVICE_H
@@ -57,30 +58,42 @@ __device__ __forceinline__ float ghip_e4m3_exact(uint32_t c) {
 typedef unsigned int ghip_u32x2 __attribute__((ext_vector_type(2)));
 
 /* Four codes of one dword -> four dequantized bf16 packed in two dwords
- * (element j in bits [16*(j&1), +16) of dword j/2). */
+ * (element j in bits [16*(j&1), +16) of dword j/2). EXACT: the hardware
+ * convert gives a NaN for the two NaN codes only; the minimum of |value| and
+ * 480 picks the number there, and the sign comes from the code (a compare per
+ * code would cost a mask register each: 80 to 290 of them spilled in the
+ * unrolled GEMV and GEMM bodies). */
 template <bool EXACT>
 __device__ __forceinline__ ghip_u32x2 ghip_deq4(uint32_t d, float s) {
-    ghip_u32x2 r;
+    typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+    ghip_f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8((int)d, false);
+    ghip_f32x2 b = __builtin_amdgcn_cvt_pk_f32_fp8((int)d, true);
     if (EXACT) {
-        uint32_t b0 = ghip_bf16_bits(ghip_e4m3_exact(d & 0xffu) * s);
-        uint32_t b1 = ghip_bf16_bits(ghip_e4m3_exact((d >> 8) & 0xffu) * s);
-        uint32_t b2 = ghip_bf16_bits(ghip_e4m3_exact((d >> 16) & 0xffu) * s);
-        uint32_t b3 = ghip_bf16_bits(ghip_e4m3_exact(d >> 24) * s);
-        r[0] = b0 | (b1 << 16);
-        r[1] = b2 | (b3 << 16);
-    } else {
-        ghip_f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8((int)d, false);
-        ghip_f32x2 b = __builtin_amdgcn_cvt_pk_f32_fp8((int)d, true);
-        typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-        bf2 p, q;
-        p[0] = (__bf16)(a[0] * s);
-        p[1] = (__bf16)(a[1] * s);
-        q[0] = (__bf16)(b[0] * s);
-        q[1] = (__bf16)(b[1] * s);
-        r[0] = __builtin_bit_cast(uint32_t, p);
-        r[1] = __builtin_bit_cast(uint32_t, q);
+        auto fix = [](float v, uint32_t sign) {
+            return __builtin_copysignf(__builtin_fminf(__builtin_fabsf(v), 480.0f),
+                                       __uint_as_float(sign));
+        };
+        a[0] = fix(a[0], d << 24);
+        a[1] = fix(a[1], d << 16);
+        b[0] = fix(b[0], d << 8);
+        b[1] = fix(b[1], d);
     }
-    return r;
+    bf2 p, q;
+    p[0] = (__bf16)(a[0] * s);
+    p[1] = (__bf16)(a[1] * s);
+    q[0] = (__bf16)(b[0] * s);
+    q[1] = (__bf16)(b[1] * s);
+    return (ghip_u32x2){__builtin_bit_cast(uint32_t, p), __builtin_bit_cast(uint32_t, q)};
+}
+
+/* The same by the integer decode and the integer RNE narrow, which passes a
+ * NaN product's bits through as the reference does. */
+__device__ __forceinline__ ghip_u32x2 ghip_deq4_int(uint32_t d, float s) {
+    uint32_t b0 = ghip_bf16_bits(ghip_e4m3_exact(d & 0xffu) * s);
+    uint32_t b1 = ghip_bf16_bits(ghip_e4m3_exact((d >> 8) & 0xffu) * s);
+    uint32_t b2 = ghip_bf16_bits(ghip_e4m3_exact((d >> 16) & 0xffu) * s);
+    uint32_t b3 = ghip_bf16_bits(ghip_e4m3_exact(d >> 24) * s);
+    return (ghip_u32x2){b0 | (b1 << 16), b2 | (b3 << 16)};
 }
 
 /* 16 codes (one 16-byte load) -> 8 dwords of packed bf16: lo holds codes

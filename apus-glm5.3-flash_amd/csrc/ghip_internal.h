@@ -195,6 +195,17 @@ hipError_t ghip_launch_moe_prefill(const GhipBank *bank, const uint16_t *x,
                                    const GhipMoePrefillWs *ws,
                                    const hipEvent_t *ev, hipStream_t st);
 
+/* The products of a prefill whose tiles mostly hold a few rows: mode 0 gate/up
+ * + SwiGLU (act = x, rows gathered by perm[s] / topk; out = H), mode 1 down
+ * (act = H, out = O), over the tile list of the permutation. e0/e1: NULL or
+ * timing events. fits: whether its 32-bit offsets hold T tokens, P pairs. */
+int ghip_moe_rows_fits(const GhipBank *bank, size_t T, size_t P);
+hipError_t ghip_launch_moe_rows(int mode, const GhipBank *bank, const uint16_t *act,
+                                const int32_t *perm, const uint32_t *tiles,
+                                const uint32_t *hdr, uint32_t topk, float limit,
+                                uint16_t *out, uint32_t n_cu, hipEvent_t e0,
+                                hipEvent_t e1, hipStream_t st);
+
 /* Dense FP8-block GEMM on MFMA (the prefill tile body): Y [M, N] =
  * bf16(X [M, K] . dequant(W [N, K])^T). Shapes it takes: N % 256 == 0,
  * K % 128 == 0, K <= 16384, 16-byte aligned codes, X and Y

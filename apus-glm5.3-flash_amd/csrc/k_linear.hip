@@ -43,7 +43,14 @@ __global__ __launch_bounds__(256) void k_dequant16(
         float sc = s[(size_t)(o >> 7) * nkb + (k0 >> 7)];
         ghip_u32x4 v = *(const ghip_u32x4 *)(w + (size_t)o * K + k0);
         ghip_u32x4 r0, r1;
-        ghip_deq16_u32<EXACT>(v, sc, r0, r1);
+        if (EXACT) {
+            const ghip_u32x2 a = ghip_deq4_int(v[0], sc), b = ghip_deq4_int(v[1], sc);
+            const ghip_u32x2 e = ghip_deq4_int(v[2], sc), f = ghip_deq4_int(v[3], sc);
+            r0 = (ghip_u32x4){a[0], a[1], b[0], b[1]};
+            r1 = (ghip_u32x4){e[0], e[1], f[0], f[1]};
+        } else {
+            ghip_deq16_u32<false>(v, sc, r0, r1);
+        }
         ghip_u32x4 *dst = (ghip_u32x4 *)(out + (size_t)o * K + k0);
         dst[0] = r0;
         dst[1] = r1;

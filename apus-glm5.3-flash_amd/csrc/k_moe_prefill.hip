@@ -12,20 +12,25 @@
  *   k_pf_scan     one workgroup: exclusive offsets per (chunk, expert), the
  *                 expert-sorted row ranges and the tile list.
  *   k_pf_scatter  stable scatter (token order inside each expert).
- *   k_pf_gemm<0, NW>  gate/up: H[s] = SwiGLU(bf16(x Wg^T), bf16(x Wu^T)) for the
+ *                 Up to 1024 pairs: k_pf_permute, all three in one launch.
+ *   k_pf_gemm<0, ·> gate/up: H[s] = SwiGLU(bf16(x Wg^T), bf16(x Wu^T)) for the
  *                 sorted pair rows s of each tile; x rows gathered by token.
- *   k_pf_gemm<1, NW>  down: O[s] = bf16(H[s] Wd^T).
+ *   k_pf_gemm<1, ·> down: O[s] = bf16(H[s] Wd^T).
+ *                 Few rows an expert: k_moe_rows.hip's streams instead.
  *   k_pf_combine  out[t] = ascending-expert, bf16-per-add sum of
  *                 bf16(O[s] * w) over the token's pairs (c/gmoe.h:307-320).
  *
- * GEMM tile (both modes). A workgroup of 4 waves (NW = 4) owns one tile of
- * up to 256 expert-sorted rows and one column block; K is walked in
- * 64-wide stages (half an F32 scale block). Each wave owns two 32-column
- * weight slots (gate and up columns [c, c+32) in mode 0, so the SwiGLU
- * epilogue is lane-local; two 128-apart down column groups in mode 1) for
- * all tile rows, accumulating 2 x NRB v_mfma_f32_32x32x16_bf16 blocks.
- * With NW = 8 (two waves per SIMD) the same tile is split into two row
- * halves, so one wave's MFMAs run while the other issues its DMA. Both
+ * GEMM tile (both modes). A workgroup of 8 waves, two per SIMD so that one
+ * wave's MFMAs run while the other waits or dequantizes, owns one tile of up
+ * to 256 expert-sorted rows and one column block; K is walked in 64-wide
+ * stages (half an F32 scale block). Each wave owns two 32-column weight slots
+ * (gate and up columns [c, c+32) in mode 0, so the SwiGLU epilogue is
+ * lane-local; two 128-apart down column groups in mode 1) in
+ * v_mfma_f32_32x32x16_bf16 blocks: for half of a full tile's rows, or, for
+ * tiles of up to 128 rows in the queued form, for all rows and half of each
+ * stage's k (every weight dequantized once); tiles of up to 16 rows there are
+ * weight streams (pf_rows_tile). The dense GEMM runs the same body with 4
+ * waves, each over all the tile's rows. Both
  * operands stream HBM -> LDS by direct DMA (global_load_lds) through a ring
  * of stages, the activation rows gathered by token in mode 0; the FP8 codes
  * are dequantized in registers when read from LDS, bit-exact
@@ -132,8 +137,9 @@ __device__ __forceinline__ uint32_t pf_block_scan(uint32_t v, uint32_t *sh) {
 
 /* One workgroup of 1024 threads, thread e = expert e. cnt becomes the
  * exclusive start offset (in the expert-sorted order) of each (chunk,
- * expert); tiles[] = {expert, first sorted row, rows, NaN-code flag of the
- * expert (nan_flags[e] != 0; 0 without nan_flags)}; hdr gets the tile
+ * expert); tiles[] = {expert, first sorted row, rows, flags: 1 = the expert
+ * has NaN codes (nan_flags[e] != 0; 0 without nan_flags), 2 = it has more
+ * than one tile}; hdr gets the tile
  * count and the number of valid pairs. */
 __global__ __launch_bounds__(1024) void k_pf_scan(
     uint32_t *__restrict__ cnt, uint32_t nch, uint32_t E,
@@ -158,7 +164,7 @@ __global__ __launch_bounds__(1024) void k_pf_scan(
     const uint32_t base = pf_block_scan(tot, sh) - tot;
     const uint32_t tb = pf_block_scan(nt, sh) - nt;
     if (e < E) {
-        const uint32_t nanf = nan_flags && nan_flags[e] ? 1u : 0u;
+        const uint32_t nanf = (nan_flags && nan_flags[e] ? 1u : 0u) | (nt > 1u ? 2u : 0u);
         uint32_t run = base;
         for (uint32_t c0 = 0; c0 < nch; c0 += 16) {
             uint32_t v[16];
@@ -216,6 +222,88 @@ __global__ __launch_bounds__(1024) void k_pf_scatter(
         pos[p] = (int32_t)s;
     } else if (p < P) {
         pos[p] = -1;
+    }
+}
+
+/* The whole permutation of at most PF_CHUNK pairs in one launch (one
+ * workgroup): what the header fill, k_pf_count, k_pf_scan and k_pf_scatter do
+ * in four, with the histogram and the expert starts in LDS, and the same
+ * results. At these sizes each of the four launches costs its ~4.5 us however
+ * little it does (T = 12 at top-8: 20 us of 353). */
+__global__ __launch_bounds__(1024) void k_pf_permute(
+    const int32_t *__restrict__ idx, uint32_t P, uint32_t topk, uint32_t topk_p, uint32_t E,
+    const uint32_t *__restrict__ nan_flags, uint4 *__restrict__ tiles,
+    int32_t *__restrict__ perm, int32_t *__restrict__ pos, uint32_t *__restrict__ hdr,
+    uint32_t *__restrict__ serr) {
+    extern __shared__ uint32_t pm[];                    /* starts [Ep], counts [16][Ep] */
+    __shared__ uint32_t sh[16], bad;
+    const uint32_t Ep = E + (topk_p - topk), tid = threadIdx.x, w = tid >> 6, lane = tid & 63u;
+    uint32_t *start = pm, *wcnt = pm + Ep;
+    for (uint32_t i = tid; i < 16u * Ep; i += 1024u) wcnt[i] = 0;
+    if (tid == 0) bad = 0;
+    __syncthreads();
+    /* ids as k_pf_count takes them: out of range flagged and dropped, a
+     * repeat of an earlier slot of the token dropped */
+    int32_t e = -1;
+    if (tid < P) {
+        const uint32_t t = tid / topk_p, j = tid - t * topk_p;
+        e = j < topk ? idx[(size_t)t * topk + j] : (int32_t)E;
+        if (j < topk) {
+            if (e < 0 || (uint32_t)e >= E) {
+                e = -1;
+                bad = 1;
+            } else {
+                for (uint32_t jj = 0; jj < j; jj++)
+                    if (idx[(size_t)t * topk + jj] == e) {
+                        e = -1;
+                        break;
+                    }
+            }
+        }
+    }
+    /* rank among the wave's pairs of the same expert, as k_pf_scatter */
+    uint32_t rank = 0;
+    uint64_t todo = __ballot(e >= 0);
+    while (todo) {
+        const int lead = __builtin_ctzll(todo);
+        const int32_t e0 = __builtin_amdgcn_readlane(e, lead);
+        const uint64_t m = __ballot(e == e0);
+        if (e == e0) rank = __popcll(m & ((1ull << lane) - 1ull));
+        if (lane == (uint32_t)lead) wcnt[w * Ep + e0] = __popcll(m);
+        todo &= ~m;
+    }
+    __syncthreads();
+    /* thread x: expert x's rows, as k_pf_scan */
+    uint32_t tot = 0;
+    if (tid < Ep)
+#pragma unroll
+        for (uint32_t v = 0; v < 16; v++) tot += wcnt[v * Ep + tid];
+    const uint32_t nt = (tot + PF_BM - 1) / PF_BM;
+    const uint32_t base = pf_block_scan(tot, sh) - tot;
+    const uint32_t tb = pf_block_scan(nt, sh) - nt;
+    if (tid < Ep) {
+        const uint32_t nanf = (nan_flags && nan_flags[tid] ? 1u : 0u) | (nt > 1u ? 2u : 0u);
+        start[tid] = base;
+        for (uint32_t i = 0; i < nt; i++) {
+            const uint32_t r0 = i * PF_BM;
+            tiles[tb + i] = make_uint4(tid, base + r0, tot - r0 < PF_BM ? tot - r0 : PF_BM, nanf);
+        }
+    }
+    if (tid < PF_HDR_WORDS && tid != PF_HDR_NTILES && tid != PF_HDR_NPAIRS)
+        hdr[tid] = tid == PF_HDR_ERR ? bad : 0u;
+    if (tid == 1023) {
+        hdr[PF_HDR_NTILES] = tb + nt;
+        hdr[PF_HDR_NPAIRS] = base + tot;
+    }
+    if (tid == 0 && bad && serr) atomicOr(serr, 2u);
+    __syncthreads();
+    if (e >= 0) {
+        for (uint32_t v = 0; v < w; v++) rank += wcnt[v * Ep + e];
+        const uint32_t s = start[e] + rank;
+        perm[s] = (int32_t)tid;
+        pos[tid] = (int32_t)s;
+    } else if (tid < P) {
+        pos[tid] = -1;
     }
 }
 
@@ -298,6 +386,110 @@ struct PfTile {
     float limit;                  /* K: row stride; KS: k span of this tile */
 };
 
+/* The end of a KG = 2 tile body: each K group hands the other half of its
+ * sums over through LDS and finishes registers [8 kg, 8 kg + 8) of every row
+ * block, i.e. rows 16 kg .. 16 kg + 15 of it, so both groups share the
+ * epilogue. group 0's sum + group 1's, whichever wave adds. Rows, columns and
+ * staging as in pf_tile's own epilogue. */
+template <int MODE, int NRB>
+__device__ __forceinline__ void pf_epilogue_kg(const PfTile &t, uint8_t *lds,
+                                               const ghip_f32x16 (&a0)[NRB],
+                                               const ghip_f32x16 (&a1)[NRB], uint32_t kg,
+                                               uint32_t cw, uint32_t lane) {
+    const uint32_t n = lane & 31u, h = lane >> 5;
+    float v0[NRB][8], v1[NRB][8];
+    __builtin_amdgcn_s_waitcnt(0xc07f);            /* lgkmcnt(0): ring reads done */
+    __builtin_amdgcn_s_barrier();
+    ghip_f32x4 *mine = (ghip_f32x4 *)lds + (size_t)(kg * 4u + cw) * (NRB * 4u * 64u) + lane;
+    const ghip_f32x4 *theirs =
+        (const ghip_f32x4 *)lds + (size_t)((kg ^ 1u) * 4u + cw) * (NRB * 4u * 64u) + lane;
+#pragma unroll
+    for (int rb = 0; rb < NRB; rb++)
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            ghip_f32x4 g0, g1;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int i = 4 * q + k;
+                g0[k] = kg ? a0[rb][i] : a0[rb][8 + i];
+                g1[k] = kg ? a1[rb][i] : a1[rb][8 + i];
+                v0[rb][i] = kg ? a0[rb][8 + i] : a0[rb][i];
+                v1[rb][i] = kg ? a1[rb][8 + i] : a1[rb][i];
+            }
+            mine[(rb * 4 + q) * 64] = g0;
+            mine[(rb * 4 + 2 + q) * 64] = g1;
+        }
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int rb = 0; rb < NRB; rb++)
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const ghip_f32x4 g0 = theirs[(rb * 4 + q) * 64], g1 = theirs[(rb * 4 + 2 + q) * 64];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                v0[rb][4 * q + k] = v0[rb][4 * q + k] + g0[k];
+                v1[rb][4 * q + k] = v1[rb][4 * q + k] + g1[k];
+            }
+        }
+    if constexpr (MODE == 2) {
+        const uint32_t c0 = t.cb0 + 32u * cw + n, c1 = t.cb1 + 32u * cw + n;
+#pragma unroll
+        for (int rb = 0; rb < NRB; rb++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const uint32_t r = rb * 32u + 16u * kg + 8u * (i >> 2) + 4u * h + (i & 3);
+                if (r < t.rows) {
+                    float *of = t.outf + (size_t)(t.row0 + r) * t.N;
+                    of[c0] = v0[rb][i];
+                    of[c1] = v1[rb][i];
+                }
+            }
+        return;
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);            /* own reads of the exchange */
+    __builtin_amdgcn_s_barrier();
+    constexpr uint32_t RB = MODE == 0 ? 64u : 128u;
+    uint8_t *sw = lds + (kg * 4u + cw) * (NRB * 16u * RB);
+#pragma unroll
+    for (int rb = 0; rb < NRB; rb++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const uint32_t r = rb * 16u + 8u * (i >> 2) + 4u * h + (i & 3);
+            if (MODE == 0) {
+                const uint32_t pr = r ^ ((r >> 2) & 1u);
+                *(uint16_t *)(sw + pr * 64u + n * 2u) = pf_swiglu(v0[rb][i], v1[rb][i], t.limit);
+            } else {
+                const uint32_t x = ((r >> 2) & 1u) * 64u;
+                *(uint16_t *)(sw + r * 128u + ((n * 2u) ^ x)) = pf_bf16_bits(v0[rb][i]);
+                *(uint16_t *)(sw + r * 128u + ((64u + n * 2u) ^ x)) = pf_bf16_bits(v1[rb][i]);
+            }
+        }
+    __builtin_amdgcn_s_waitcnt(0xc07f);            /* the wave's own LDS writes */
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t p = lane & 3u;
+    if (MODE == 0) {
+        uint16_t *ob = t.out + (size_t)t.row0 * t.N + t.cb0 + 32u * cw + 8u * p;
+#pragma unroll
+        for (int j = 0; j < NRB; j++) {
+            const uint32_t rr = (lane >> 2) + 16u * j, prr = rr ^ ((rr >> 2) & 1u);
+            const uint32_t m = 32u * j + 16u * kg + (lane >> 2);
+            const ghip_u32x4 v = *(const ghip_u32x4 *)(sw + prr * 64u + p * 16u);
+            if (m < t.rows) *(ghip_u32x4 *)(ob + (size_t)m * t.N) = v;
+        }
+    } else {
+        const uint32_t gs = (lane >> 2) & 1u;
+        uint16_t *ob = t.out + (size_t)t.row0 * t.N + (gs ? t.cb1 : t.cb0) + 32u * cw + 8u * p;
+#pragma unroll
+        for (int j = 0; j < 2 * NRB; j++) {
+            const uint32_t rr = (lane >> 3) + 8u * j, x = ((rr >> 2) & 1u) * 64u;
+            const uint32_t m = 32u * (j >> 1) + 16u * kg + (rr & 15u);
+            const ghip_u32x4 v = *(const ghip_u32x4 *)(sw + rr * 128u + ((gs * 64u + p * 16u) ^ x));
+            if (m < t.rows) *(ghip_u32x4 *)(ob + (size_t)m * t.N) = v;
+        }
+    }
+}
+
 /* The tile body for tiles of at most NRB 32-row blocks (rows past NRB*32
  * are neither loaded nor computed; rows past `rows` inside the last block
  * repeat the last row: computed, never stored).
@@ -319,7 +511,8 @@ struct PfTile {
  * (b) is followed by MFMA work that hides the latency of the next stage's
  * first LDS reads. Scales come from the per-tile table in LDS (sct: one
  * {slot 0, slot 1} pair per 128-wide k block), not from memory. */
-template <int MODE, int NRB, bool EXACT, int NW, int NRBC = 0, int H0 = 0>
+template <int MODE, int NRB, bool EXACT, int NW, int NRBC = 0, int H0 = 0, int KG = 1,
+          bool WBOK = true>
 __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
                                         ghip_f32x2 *sct) {
     /* NW = 4 waves (one per SIMD) or 8 (two per SIMD). Wave wv computes
@@ -329,16 +522,24 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
      * a 1-block tile loads its A rows twice, so every wave issues the same
      * count: identical bytes to the same LDS place). */
     static_assert(NW == 4 || NW == 8, "4 or 8 waves");
+    /* KG = 2 (8 waves, at most 4 row blocks): instead of the tile's rows the
+     * two halves of the waves split each stage's four MFMA steps (wave half kg
+     * takes steps 2 kg and 2 kg + 1 of every row block), so two waves share a
+     * SIMD and one's dequant and waits run under the other's MFMAs while
+     * every weight is still dequantized once. The two halves' sums meet in LDS
+     * at the end (pf_epilogue_kg). */
+    static_assert(KG == 1 || (KG == 2 && NW == 8 && NRB <= 4 && NRBC == 0), "K groups");
     /* NRBC, H0 (8 waves, 8-block layout only): this wave computes NRBC row
      * blocks and the first row half holds H0 -- a tile of 7 blocks runs its
      * second half on 3 (no MFMAs on the empty fourth block), with loads,
      * LDS layout and barriers unchanged */
-    constexpr uint32_t NRBL = NW == 8 ? (NRB >= 2 ? NRB / 2 : 1) : NRB;
+    constexpr bool RH = NW == 8 && KG == 1;      /* row halves */
+    constexpr uint32_t NRBL = RH ? (NRB >= 2 ? NRB / 2 : 1) : NRB;
     constexpr uint32_t NRBW = NRBC > 0 ? (uint32_t)NRBC : NRBL;   /* computed here */
     constexpr uint32_t HB0 = H0 > 0 ? (uint32_t)H0 : NRBL;        /* first half */
     static_assert(NRBC == 0 || (NW == 8 && NRB == 8 && NRBW <= HB0 && HB0 <= 4),
                   "short row halves: 8-wave, 8-block layout");
-    constexpr uint32_t QA = NW == 8 && NRB < 2 ? 8 : 4 * NRB;
+    constexpr uint32_t QA = NW == 8 ? (4 * NRB + 7) / 8 * 8 : 4 * NRB;
     constexpr uint32_t NA = QA / NW;              /* A loads per wave per stage */
     constexpr uint32_t NWL = 16 / NW;             /* weight loads per wave per stage */
     constexpr uint32_t LPS = NA + NWL;            /* DMA loads per wave per stage */
@@ -351,7 +552,7 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
      * each, so every load instruction reads 8 whole lines instead of 16
      * half lines) through their own 2-block ring after the 3-stage A ring,
      * filling all 160 KB; the scales come by scalar loads (no table) */
-    constexpr bool WB = NW == 8 && NRB == 8 && MODE < 2 && !EXACT;
+    constexpr bool WB = WBOK && NW == 8 && NRB == 8 && MODE < 2 && !EXACT;
     constexpr uint32_t STG = WB ? ASTG : ASTG + PF_W_STAGE;
     constexpr uint32_t NS = WB ? 3u : (PF_RING / STG < 8 ? PF_RING / STG : 8);
     constexpr uint32_t NWW = WB ? (PF_WB / 1024) / NW : 0;  /* block loads per wave */
@@ -364,7 +565,7 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
     asm volatile("" : "+v"(tid));
     const uint32_t lane = tid & 63;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t cw = wv & 3u, hr = NW == 8 ? wv >> 2 : 0u;
+    const uint32_t cw = wv & 3u, hr = RH ? wv >> 2 : 0u, kg = KG == 2 ? wv >> 2 : 0u;
     const uint32_t n = lane & 31, h = lane >> 5;
     const uint32_t K = t.K, nst = t.KS / PF_BK;
 
@@ -386,7 +587,7 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
     uint32_t aofs[NA], alds[NA];
 #pragma unroll
     for (int i = 0; i < (int)NA; i++) {
-        const uint32_t q = wv + NW * i, qq = NW == 8 && NRB < 2 ? (q & 3u) : q;
+        const uint32_t q = wv + NW * i, qq = q < 4u * NRB ? q : q - 4u * NRB;
         alds[i] = qq * 1024u;
         const uint32_t r = 8 * qq + (lane >> 3);
         const uint32_t rc = r < t.rows ? r : t.rows - 1;
@@ -480,7 +681,7 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
     uint32_t aoff[4], boff0[2];
 #pragma unroll
     for (int s = 0; s < 4; s++)
-        aoff[s] = n * 128 + 16 * (((4 * h) | s) ^ ((n >> 1) & 7));
+        aoff[s] = n * 128 + 16 * (((4 * h) | ((s + 2 * kg) & 3)) ^ ((n >> 1) & 7));
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         if constexpr (WB) {
@@ -489,7 +690,7 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
             const uint32_t ph = ((2 * h + u) ^ ((n >> 1) & 7)) * 16;
             boff0[u] = (64 * cw + n) * 128 + ph;
         } else {
-            const uint32_t ph = ((2 * h + u) ^ ((n >> 2) & 3)) * 16;
+            const uint32_t ph = ((2 * h + (KG == 2 ? kg : u)) ^ ((n >> 2) & 3)) * 16;
             boff0[u] = ASTG + (64 * cw + n) * 64 + ph;
         }
     }
@@ -502,7 +703,9 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
 
     ghip_f32x16 a0[NRBW], a1[NRBW];
     /* this wave's first row block in the stage's A rows */
-    const uint32_t arow0 = NW == 8 && NRB >= 2 ? hr * HB0 * 32u * 128u : 0u;
+    const uint32_t arow0 = RH && NRB >= 2 ? hr * HB0 * 32u * 128u : 0u;
+    /* MFMA steps of a stage this wave computes, and its code pieces per slot */
+    constexpr int ST = KG == 2 ? 2 : 4, NU = KG == 2 ? 1 : 2;
 #pragma unroll
     for (int rb = 0; rb < (int)NRBW; rb++)
 #pragma unroll
@@ -545,7 +748,7 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
         const uint8_t *sb0 = bsrc(0);
         if constexpr (!WB) sc = sct[0];
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
+        for (int u = 0; u < NU; u++) {
             q0[u] = *(const ghip_u32x4 *)(sb0 + boff0[u]);
             q1[u] = *(const ghip_u32x4 *)(sb0 + boff0[u] + BD);
         }
@@ -568,7 +771,7 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
         const uint8_t *st = lds + (j % NS) * STG;
         const uint32_t ld = j + NS - 1;
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
+        for (int s = 0; s < ST; s++) {
             if constexpr (WB) {
                 /* an even stage issues weight block j/2 + 1 (steps 0, 1)
                  * ahead of stage j + 2's A rows (steps 2, 3), so waiting for
@@ -579,11 +782,11 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
                 if (REFILL && s == 3) issue_a(std::integral_constant<int, 1>{}, j + 2u);
             } else {
                 if (REFILL && s == 0) issue_part(std::integral_constant<int, 0>{}, ld, ld);
-                if (REFILL && s == 1) issue_part(std::integral_constant<int, 1>{}, ld, ld);
-                if (REFILL && s == 2) issue_part(std::integral_constant<int, 2>{}, ld, ld);
-                if (REFILL && s == 3) issue_part(std::integral_constant<int, 3>{}, ld, ld);
+                if (REFILL && s == (KG == 2 ? 0 : 1)) issue_part(std::integral_constant<int, 1>{}, ld, ld);
+                if (REFILL && s == (KG == 2 ? 1 : 2)) issue_part(std::integral_constant<int, 2>{}, ld, ld);
+                if (REFILL && s == ST - 1) issue_part(std::integral_constant<int, 3>{}, ld, ld);
             }
-            if (s < 3) {
+            if (s < ST - 1) {
                 /* step s+1 of this stage: A rows from LDS, B codes already
                  * in registers */
                 const int u = (s + 1) >> 1, v = 2 * ((s + 1) & 1);
@@ -626,7 +829,7 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
                     sc = sct[(j + 1) >> 1];
                 }
 #pragma unroll
-                for (int u = 0; u < 2; u++) {
+                for (int u = 0; u < NU; u++) {
                     q0[u] = *(const ghip_u32x4 *)(sbn + (boff0[u] ^ bx));
                     q1[u] = *(const ghip_u32x4 *)(sbn + (boff0[u] ^ bx) + BD);
                 }
@@ -643,7 +846,7 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
             }
             /* interleave the next step's LDS reads and dequant (and, at a
              * stage boundary, the DMA refill) between this step's MFMAs */
-            if (s == 3 && NEXT) {
+            if (s == ST - 1 && NEXT) {
                 /* 5 + NRB LDS reads (scales, B codes, A rows), then the
                  * dequant of the next step's B */
 #pragma unroll
@@ -654,7 +857,7 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
                     if (i >= 3 && i < 3 + (int)NRBW) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                     if (i >= (NW == 8 ? 3 : 5)) __builtin_amdgcn_sched_group_barrier(0x002, 4, 0); /* VALU */
                 }
-            } else if (s < 3) {
+            } else if (s < ST - 1) {
 #pragma unroll
                 for (int i = 0; i < 2 * (int)NRBW; i++) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -692,6 +895,10 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
 
     /* epilogue: lane (n, h), register i of row block rb holds output row
      * rowbase + rb*32 + 8*(i/4) + 4*h + i%4, column n of each slot */
+    if constexpr (KG == 2) {
+        pf_epilogue_kg<MODE, NRB>(t, lds, a0, a1, kg, cw, lane);
+        return;
+    }
     const uint32_t rowbase = hr * HB0 * 32;
     if constexpr (MODE == 2) {
         const uint32_t c0 = t.cb0 + 32 * cw + n, c1 = t.cb1 + 32 * cw + n;
@@ -763,26 +970,144 @@ __device__ __forceinline__ void pf_tile(const PfTile &t, uint8_t *lds,
     }
 }
 
+/* A tile of at most 16 rows, as a weight stream: wave w of 8
+ * owns 32 weight rows (16 gate and the same 16 up rows in mode 0, 32 down
+ * rows in mode 1) over all of K and walks their 128-wide k blocks with two in
+ * flight, each loaded with its part of the tile's activation rows into
+ * registers (whole lines), passed through a wave-private LDS area into the
+ * layout of v_mfma_f32_16x16x32_bf16 and dequantized once. No barrier in the
+ * stream and nothing to reduce. The stage loop of pf_tile dequantizes the
+ * same bytes against 32-row blocks that are mostly padding and meets at a
+ * barrier a stage: 288 experts at T = 128 1292 -> 1132 us (6.2 TB/s). */
+template <int MODE>
+__device__ __forceinline__ void pf_rows_tile(const PfTile &t, uint8_t *lds) {
+    uint32_t tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const uint32_t lane = tid & 63u;
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t n = lane & 15u, g = lane >> 4;
+    const uint32_t K = t.K, nch = K >> 7;
+    uint8_t *xs = lds + wv * 8192u, *ws = xs + 4096u;
+    const uint32_t col = MODE == 0 ? t.cb0 + 16u * wv : t.cb0 + 32u * wv;
+    const uint8_t *w0 = t.w0 + (size_t)col * K;
+    const uint8_t *w1 = MODE == 0 ? t.w1 + (size_t)col * K : w0 + (size_t)16u * K;
+    const float *s0 = MODE == 1 && wv >= 4u ? t.sr1 : t.sr0, *s1 = MODE == 0 ? t.sr1 : s0;
+    const ghip_cdma d = ghip_cdma_offsets(lane, K);
+    uint32_t xo[4];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; u++) {
+        const uint32_t r = 4u * u + (lane >> 4), rc = t.row0 + min(r, t.rows - 1u);
+        const uint32_t src = MODE == 0 ? (uint32_t)t.perm[rc] / t.topk : rc;
+        xo[u] = src * K * 2u + 16u * ((lane & 15u) ^ (r & 15u));
+    }
+    struct Set {
+        ghip_u32x4 x[4], a0, a1, b0, b1;
+        float sa, sb;
+    };
+    Set r0, r1;
+    auto load = [&](Set &r, uint32_t c) {
+        const uint8_t *xc = (const uint8_t *)t.act + (size_t)c * 256u;
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) r.x[u] = *(const ghip_u32x4 *)(xc + xo[u]);
+        ghip_rl_load(w0, d, c, r.a0, r.a1);
+        ghip_rl_load(w1, d, c, r.b0, r.b1);
+        /* the scales as vector loads, in order with the codes: a scalar load
+         * would make every LDS wait of the step wait for it */
+        r.sa = __uint_as_float(__hip_atomic_load((const uint32_t *)s0 + c, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_WORKGROUP));
+        r.sb = MODE == 0 ? __uint_as_float(__hip_atomic_load((const uint32_t *)s1 + c,
+                                                             __ATOMIC_RELAXED,
+                                                             __HIP_MEMORY_SCOPE_WORKGROUP))
+                         : r.sa;
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    ghip_f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+    auto step = [&](Set &r, auto refill_c, uint32_t c) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) *(ghip_u32x4 *)(xs + u * 1024u + lane * 16u) = r.x[u];
+        ghip_rl_store(ws, lane, r.a0, r.a1);
+        ghip_rl_store(ws + 2048u, lane, r.b0, r.b1);
+        const float fa = r.sa, fb = r.sb;
+        if constexpr (decltype(refill_c)::value) {
+            __builtin_amdgcn_sched_barrier(0);
+            load(r, c + 2u);
+        }
+        const ghip_chunk ca = ghip_cdma_read(ws, n, g), cb = ghip_cdma_read(ws + 2048u, n, g);
+        ghip_bf16x8 wa[4], wb[4];
+        ghip_deq16<false>(ca.lo, fa, wa[0], wa[1]);
+        ghip_deq16<false>(ca.hi, fa, wa[2], wa[3]);
+        ghip_deq16<false>(cb.lo, fb, wb[0], wb[1]);
+        ghip_deq16<false>(cb.hi, fb, wb[2], wb[3]);
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            const ghip_bf16x8 xv = *(const ghip_bf16x8 *)(xs + n * 256u + 16u * ((4u * g + i) ^ n));
+            acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv, wa[i], acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv, wb[i], acc1, 0, 0, 0);
+        }
+    };
+    using RF = std::true_type;
+    using NR = std::false_type;
+    load(r0, 0u);
+    load(r1, nch > 1u ? 1u : 0u);
+    /* every wave holds its item before thread 0 publishes the next one */
+    __builtin_amdgcn_s_barrier();
+    uint32_t c = 0;
+    for (; c + 3u < nch; c += 2u) {
+        step(r0, RF{}, c);
+        step(r1, RF{}, c + 1u);
+    }
+    if (nch - c == 3u) {
+        step(r0, RF{}, c);
+        step(r1, NR{}, c + 1u);
+        step(r0, NR{}, c + 2u);
+    } else if (nch - c == 2u) {
+        step(r0, NR{}, c);
+        step(r1, NR{}, c + 1u);
+    } else {
+        step(r0, NR{}, c);
+    }
+    /* lane (g, n), register i: tile row 4g + i, column n */
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) {
+        const uint32_t m = 4u * g + i;
+        if (m < t.rows) {
+            uint16_t *o = t.out + (size_t)(t.row0 + m) * t.N + col + n;
+            if (MODE == 0) {
+                o[0] = pf_swiglu(acc0[i], acc1[i], t.limit);
+            } else {
+                o[0] = pf_bf16_bits(acc0[i]);
+                o[16] = pf_bf16_bits(acc1[i]);
+            }
+        }
+    }
+}
+
 /* MODE 0: act = x [T, dim], rows gathered by token (perm[s] / topk);
  *         out = H [P, inter] (sorted rows), SwiGLU epilogue.
  * MODE 1: act = H [P, inter] (sorted rows); out = O [P, dim] (sorted rows),
  *         bf16 expert outputs.
- * Grid: G (multiple of 8) workgroups of NW * 64 threads, one per CU. The
- * body is chosen once per tile: 8, 4, 2 or 1 row blocks (the smallest that
- * holds the tile), or the exact-decode body for an expert with NaN codes.
+ * Grid: G (multiple of 8) workgroups of 512 threads, one per CU. The body is
+ * chosen once per tile by its row blocks, or the exact-decode body for an
+ * expert with NaN codes.
  *
  * Items (tile, column block) are grouped by XCD: XCD x owns tiles x, x + 8,
  * ... and its workgroups share each tile's column blocks, so a tile's
- * gathered activation rows are read into one L2. With NW = 8 (routings
- * that fill tiles: items of one size) an XCD's workgroups take its items
- * round-robin. With NW = 4 (sparse routings: tiles of 1 to 256 rows, items
- * of very different cost) they take them from the XCD's queue, a counter
- * in hdr that every grab bumps, and, once it is empty, from the other XCDs'
- * queues in turn: no workgroup idles while another still holds a backlog.
+ * gathered activation rows are read into one L2. FULL (routings that fill
+ * tiles: items of one size): an XCD's workgroups take its items round-robin,
+ * the bodies split a tile's rows between the two wave halves, and full tiles
+ * take their weights in 128-wide blocks. Else (sparse routings: tiles of 1 to
+ * 256 rows, items of very different cost) they take them from the XCD's
+ * queue, a counter in hdr that every grab bumps, and, once it is empty, from
+ * the other XCDs' queues in turn: no workgroup idles while another still
+ * holds a backlog; tiles of up to 128 rows split each stage's k between the
+ * wave halves instead of the rows, which dequantizes every weight once, and
+ * tiles of up to 16 rows are weight streams. Against one wave per SIMD over
+ * all rows (288 experts, top-8): T = 512 1381 -> 1269 us, T = 2048 1712 ->
+ * 1651 and, Zipf 1.1, 1867 -> 1773, T = 4096 2311 -> 2240.
  * A grab past a queue's end moves on to the next queue, so every workgroup
  * leaves the loop after at most one failed grab per queue. */
-template <int MODE, int NW>
-__global__ __launch_bounds__(NW * 64, 1) void k_pf_gemm(
+template <int MODE, bool FULL>
+__global__ __launch_bounds__(512, 1) void k_pf_gemm(
     GhipBank bank, const uint16_t *__restrict__ act,
     const int32_t *__restrict__ perm, const uint4 *__restrict__ tiles,
     uint32_t *__restrict__ hdr, uint32_t nblk, uint32_t topk,
@@ -798,7 +1123,7 @@ __global__ __launch_bounds__(NW * 64, 1) void k_pf_gemm(
     const uint32_t items = ntx * nblk;
     const uint32_t K = MODE == 0 ? bank.dim : bank.inter;
     const uint32_t nkb = K >> 7;
-    constexpr bool DYN = NW == 4;
+    constexpr bool DYN = !FULL;
     constexpr uint32_t NONE = 0xffffffffu;
     /* dynamic items: thread 0 grabs (queue y, index i) and publishes the
      * tile index * nblk + column block in s_item (NONE when every queue is
@@ -867,23 +1192,38 @@ __global__ __launch_bounds__(NW * 64, 1) void k_pf_gemm(
         }
         /* the tile's scale table is filled by the body and made visible by
          * its prologue barrier (the previous item's trailing barrier ordered
-         * all reads of the old table); td.w = the expert's NaN-code flag */
+         * all reads of the old table); td.w: the flags of k_pf_scan */
         ghip_f32x2 *sct = (ghip_f32x2 *)(pf_lds + PF_RING);
         const uint32_t nrb = (t.rows + 31) >> 5;
-        if (td.w) pf_tile<MODE, PF_RB, true, NW>(t, pf_lds, sct);
-        else if (NW == 8 && nrb == 7) {
-            /* 7 blocks: the second row half computes 3 (same loads) */
-            if constexpr (NW == 8) {
-                if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >> 2)
-                    pf_tile<MODE, 8, false, NW, 3, 4>(t, pf_lds, sct);
-                else
-                    pf_tile<MODE, 8, false, NW, 4, 4>(t, pf_lds, sct);
+        const bool half1 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >> 2;
+        if (td.w & 1u) pf_tile<MODE, PF_RB, true, 8>(t, pf_lds, sct);
+        else if constexpr (FULL) {
+            if (nrb == 7) {
+                /* 7 blocks: the second row half computes 3 (same loads) */
+                if (half1) pf_tile<MODE, 8, false, 8, 3, 4>(t, pf_lds, sct);
+                else pf_tile<MODE, 8, false, 8, 4, 4>(t, pf_lds, sct);
             }
+            else if (nrb > 4) pf_tile<MODE, 8, false, 8>(t, pf_lds, sct);
+            else if (nrb > 2) pf_tile<MODE, 4, false, 8>(t, pf_lds, sct);
+            else if (nrb > 1) pf_tile<MODE, 2, false, 8>(t, pf_lds, sct);
+            else              pf_tile<MODE, 1, false, 8>(t, pf_lds, sct);
+        } else {
+            if (nrb > 6) pf_tile<MODE, 8, false, 8, 0, 0, 1, false>(t, pf_lds, sct);
+            else if (nrb > 4) pf_tile<MODE, 8, false, 8, 3, 3, 1, false>(t, pf_lds, sct);
+            else if (td.w & 2u) {
+                /* an expert's last tile beside full ones: which of its tokens
+                 * come here depends on the tokens' order, so their sums take
+                 * the full tiles' order (row halves, k ascending) */
+                if (nrb > 2) pf_tile<MODE, 4, false, 8>(t, pf_lds, sct);
+                else if (nrb > 1) pf_tile<MODE, 2, false, 8>(t, pf_lds, sct);
+                else pf_tile<MODE, 1, false, 8>(t, pf_lds, sct);
+            }
+            else if (nrb > 3) pf_tile<MODE, 4, false, 8, 0, 0, 2>(t, pf_lds, sct);
+            else if (nrb > 2) pf_tile<MODE, 3, false, 8, 0, 0, 2>(t, pf_lds, sct);
+            else if (nrb > 1) pf_tile<MODE, 2, false, 8, 0, 0, 2>(t, pf_lds, sct);
+            else if (t.rows > 16) pf_tile<MODE, 1, false, 8, 0, 0, 2>(t, pf_lds, sct);
+            else              pf_rows_tile<MODE>(t, pf_lds);
         }
-        else if (nrb > 4) pf_tile<MODE, 8, false, NW>(t, pf_lds, sct);
-        else if (nrb > 2) pf_tile<MODE, 4, false, NW>(t, pf_lds, sct);
-        else if (nrb > 1) pf_tile<MODE, 2, false, NW>(t, pf_lds, sct);
-        else              pf_tile<MODE, 1, false, NW>(t, pf_lds, sct);
         if constexpr (DYN) {
             /* every wave has read s_item (the body holds barriers) */
             if (threadIdx.x == 0) s_item = grab();
@@ -1142,42 +1482,61 @@ extern "C" hipError_t ghip_launch_moe_prefill(const GhipBank *bank,
     hipEvent_t e4 = ev ? ev[4] : nullptr, e5 = ev ? ev[5] : nullptr;
     hipEvent_t e6 = ev ? ev[6] : nullptr, e7 = ev ? ev[7] : nullptr;
     hipError_t e;
-    if ((e = ghip_launch_fill_u32(ws->hdr, PF_HDR_WORDS, 0u, st)) != hipSuccess) return e;
-    GHIP_LAUNCH(e0, nullptr, k_pf_count, dim3(nch), dim3(1024), Ep * 4, st, idx,
-                (uint32_t)P, (uint32_t)topk, topk_p, E, ws->cnt, ws->eid, ws->hdr,
-                bank->err);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_pf_scan, dim3(1), dim3(1024), 0, st, ws->cnt, nch, Ep,
-                       bank->nan_flags, (uint4 *)ws->tiles, ws->hdr);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    GHIP_LAUNCH(nullptr, e1, k_pf_scatter, dim3(nch), dim3(1024), 16 * Ep * 4, st,
-                ws->eid, (uint32_t)P, Ep, ws->cnt, ws->perm, ws->pos);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if (P <= PF_CHUNK) {
+        GHIP_LAUNCH(e0, e1, k_pf_permute, dim3(1), dim3(1024), 17 * Ep * 4, st, idx, (uint32_t)P,
+                    (uint32_t)topk, topk_p, E, bank->nan_flags, (uint4 *)ws->tiles, ws->perm,
+                    ws->pos, ws->hdr, bank->err);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    } else {
+        if ((e = ghip_launch_fill_u32(ws->hdr, PF_HDR_WORDS, 0u, st)) != hipSuccess) return e;
+        GHIP_LAUNCH(e0, nullptr, k_pf_count, dim3(nch), dim3(1024), Ep * 4, st, idx,
+                    (uint32_t)P, (uint32_t)topk, topk_p, E, ws->cnt, ws->eid, ws->hdr,
+                    bank->err);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        hipLaunchKernelGGL(k_pf_scan, dim3(1), dim3(1024), 0, st, ws->cnt, nch, Ep,
+                           bank->nan_flags, (uint4 *)ws->tiles, ws->hdr);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        GHIP_LAUNCH(nullptr, e1, k_pf_scatter, dim3(nch), dim3(1024), 16 * Ep * 4, st,
+                    ws->eid, (uint32_t)P, Ep, ws->cnt, ws->perm, ws->pos);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
     const size_t lds = PF_LDS, lds8 = PF_LDS_WB;
     (void)mt;
     const uint32_t g0 = ws->n_cu, g1 = ws->n_cu;
-    /* two waves per SIMD when the tiles are mostly full (on average at
-     * least half a 256-row tile per expert): one wave's MFMAs cover the
-     * other's DMA issue; sparse routings (mostly short tiles) keep one wave
-     * per SIMD, which wastes no MFMAs on a half-empty row split */
+    /* Which products. Tiles mostly full (on average at least half a 256-row
+     * tile per expert): the static full-tile form. Few rows an expert (on
+     * average at most one, or little work in all): weight streams in small
+     * items, which the tile form's 1 MB items and long launches cannot match
+     * (288 experts of 4096/2048, top-8: T = 12 351 against 364 us, T = 32
+     * 698 against 691, T = 64 1000 against 979; 64 of 2048/1024, 6 + shared:
+     * T = 32, 2.8 GFLOP, 87 against 102 us, T = 64, 5.6 GFLOP, 118 against
+     * 114). Else the queued form. */
     const bool full = P >= (size_t)Ep * (PF_BM / 2);
-    if (full)
-        GHIP_LAUNCH(e2, e3, (k_pf_gemm<0, 8>), dim3(g0), dim3(512), lds8, st, *bank,
+    const bool few = !full && ghip_moe_rows_fits(bank, T, P)
+                  && (P <= Ep || 6.0 * (double)P * dim * inter <= 3e9);
+    if (few) {
+        if ((e = ghip_launch_moe_rows(0, bank, x, ws->perm, ws->tiles, ws->hdr, topk_p, limit,
+                                      ws->h, ws->n_cu, e2, e3, st)) != hipSuccess
+            || (e = ghip_launch_moe_rows(1, bank, ws->h, ws->perm, ws->tiles, ws->hdr, topk_p,
+                                         limit, ws->o, ws->n_cu, e4, e5, st)) != hipSuccess)
+            return e;
+    } else if (full) {
+        GHIP_LAUNCH(e2, e3, (k_pf_gemm<0, true>), dim3(g0), dim3(512), lds8, st, *bank,
                     x, ws->perm, (const uint4 *)ws->tiles, ws->hdr, inter / 128,
                     topk_p, limit, ws->h);
-    else
-        GHIP_LAUNCH(e2, e3, (k_pf_gemm<0, 4>), dim3(g0), dim3(256), lds, st, *bank,
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        GHIP_LAUNCH(e4, e5, (k_pf_gemm<1, true>), dim3(g1), dim3(512), lds8, st, *bank,
+                    ws->h, ws->perm, (const uint4 *)ws->tiles, ws->hdr, dim / 256,
+                    topk_p, limit, ws->o);
+    } else {
+        GHIP_LAUNCH(e2, e3, (k_pf_gemm<0, false>), dim3(g0), dim3(512), lds, st, *bank,
                     x, ws->perm, (const uint4 *)ws->tiles, ws->hdr, inter / 128,
                     topk_p, limit, ws->h);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    if (full)
-        GHIP_LAUNCH(e4, e5, (k_pf_gemm<1, 8>), dim3(g1), dim3(512), lds8, st, *bank,
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        GHIP_LAUNCH(e4, e5, (k_pf_gemm<1, false>), dim3(g1), dim3(512), lds, st, *bank,
                     ws->h, ws->perm, (const uint4 *)ws->tiles, ws->hdr, dim / 256,
                     topk_p, limit, ws->o);
-    else
-        GHIP_LAUNCH(e4, e5, (k_pf_gemm<1, 4>), dim3(g1), dim3(256), lds, st, *bank,
-                    ws->h, ws->perm, (const uint4 *)ws->tiles, ws->hdr, dim / 256,
-                    topk_p, limit, ws->o);
+    }
     if ((e = hipGetLastError()) != hipSuccess) return e;
     const size_t nblk_c = T * (size_t)((dim + 2047) / 2048);
     GHIP_LAUNCH(e6, e7, k_pf_combine, dim3((uint32_t)nblk_c), dim3(256),
@@ -1352,11 +1711,12 @@ extern "C" hipError_t ghip_pf_scratch_ws(int device, size_t pairs, uint32_t n_ex
 }
 
 extern "C" hipError_t ghip_moe_prefill_init(void) {
-    const void *ks[5] = {(const void *)k_pf_gemm<0, 8>, (const void *)k_pf_gemm<0, 4>,
-                         (const void *)k_pf_gemm<1, 8>, (const void *)k_pf_gemm<1, 4>,
+    const void *ks[6] = {(const void *)k_pf_permute,
+                         (const void *)k_pf_gemm<0, true>, (const void *)k_pf_gemm<0, false>,
+                         (const void *)k_pf_gemm<1, true>, (const void *)k_pf_gemm<1, false>,
                          (const void *)k_fp8_gemm};
-    const int lds[5] = {PF_LDS_WB, PF_LDS, PF_LDS_WB, PF_LDS, PF_LDS};
-    for (int i = 0; i < 5; i++) {
+    const int lds[6] = {17 * PF_MAXE * 4, PF_LDS_WB, PF_LDS, PF_LDS_WB, PF_LDS, PF_LDS};
+    for (int i = 0; i < 6; i++) {
         hipError_t e = hipFuncSetAttribute(ks[i], hipFuncAttributeMaxDynamicSharedMemorySize,
                                            lds[i]);
         if (e != hipSuccess) return e;

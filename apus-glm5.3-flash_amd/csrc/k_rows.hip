@@ -32,27 +32,6 @@
 #define RW_NW 8                  /* waves per workgroup */
 #define RW_LDS_MAX (160u * 1024u)
 
-/* Exact decode (NaN codes are +-480, c/num.h:136-141) on the hardware
- * convert: |value| is a NaN for those codes only, and the minimum with 480
- * picks the number; the sign comes from the code. */
-
-__device__ __forceinline__ void rw_deq16_exact(ghip_u32x4 c, float s, ghip_bf16x8 &b0, ghip_bf16x8 &b1) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const ghip_f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)c[q], false);
-        const ghip_f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)c[q], true);
-        const float f[4] = {lo[0], lo[1], hi[0], hi[1]};
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const float v = __builtin_copysignf(__builtin_fminf(__builtin_fabsf(f[j]), 480.0f),
-                                                __uint_as_float(c[q] << (24 - 8 * j)));
-            const __bf16 r = (__bf16)(v * s);
-            if (q < 2) b0[4 * q + j] = r;
-            else b1[4 * (q - 2) + j] = r;
-        }
-    }
-}
-
 /* LDS: each wave's SL slots of x and weights; the partial sums reuse it */
 template <bool BF, int MR, int NT, int SL>
 __host__ __device__ constexpr uint32_t rw_wave_lds() {
@@ -177,8 +156,8 @@ __global__ __launch_bounds__(RW_NW * 64, 1) void k_rows_gemm(
 #pragma unroll
                 for (int b = 0; b < NT; b++) {
                     if (exact) {
-                        rw_deq16_exact(cw[b].lo, sc, w4[b][0], w4[b][1]);
-                        rw_deq16_exact(cw[b].hi, sc, w4[b][2], w4[b][3]);
+                        ghip_deq16<true>(cw[b].lo, sc, w4[b][0], w4[b][1]);
+                        ghip_deq16<true>(cw[b].hi, sc, w4[b][2], w4[b][3]);
                     } else {
                         ghip_deq16<false>(cw[b].lo, sc, w4[b][0], w4[b][1]);
                         ghip_deq16<false>(cw[b].hi, sc, w4[b][2], w4[b][3]);

@@ -1,0 +1,105 @@
+"""The forms a routed-MoE prefill launch takes (csrc/k_moe_prefill.hip,
+csrc/k_moe_rows.hip) at the row counts where each can go wrong, every output
+against the oracle's per-token loop (tests/tolerance.py): the weight streams
+of few rows, the queued tile form's bodies (streams up to 16 rows, k split
+between the wave halves up to 128, row halves above), the one-launch
+permutation and its limits, and experts with NaN codes in each."""
+import numpy as np
+import pytest
+
+import oracle as O
+import gpu_util as G
+from tolerance import assert_close_combined
+from test_gpu_moe import open_store, random_slabs
+from test_gpu_prefill import floor_of, prefill
+
+pytestmark = pytest.mark.gpu
+
+
+def routing_of(rows, rng):
+    """[T, k] ids that give expert e rows[e] rows (the rest repeats, dropped)."""
+    T, k = max(rows), max(1, max(sum(r > t for r in rows) for t in range(max(rows))))
+    idx = np.empty((T, k), np.int32)
+    for t in range(T):
+        mine = list(rng.permutation([e for e, r in enumerate(rows) if r > t]))
+        idx[t] = mine + [mine[0]] * (k - len(mine))
+    return idx
+
+
+def floor(slabs, dim, inter, x, idx, w, eo):
+    """Every row is checked, with as few as one expert a token, so the floor is
+    the one of the full-size checks: the combine's sum of |terms|, or, where
+    an expert's down products cancel, its own terms carried through the
+    weights -- a one-ulp step of one h_i (2^-8 |h_i| at most) moves that
+    output by up to 2^-8 |h_i wd_i|, however small the sum."""
+    return np.maximum(floor_of(eo, w, idx),
+                      O.moe_expert_floor(slabs, dim, inter, x, idx, w, threads=16))
+
+
+def check(ghip, dim, inter, rows, nan):
+    """One store and routing; k <= 16 slots a token."""
+    E = len(rows)
+    rng = np.random.default_rng(sum(rows) + dim)
+    slabs = random_slabs(E, dim, inter, rng, nan_codes_in=nan)
+    s = open_store(ghip, E, dim, inter)
+    try:
+        for e, sl in enumerate(slabs):
+            assert ghip.apus_ghip_store_put(s, e, O.ptr(sl), sl.nbytes) == 0
+        idx = routing_of(rows, rng)
+        T, k = idx.shape
+        assert k <= 16
+        w = rng.uniform(0.02, 0.6, (T, k)).astype(np.float32)
+        x = O.f32_to_bf16((rng.standard_normal((T, dim)) *
+                           rng.uniform(0.5, 4.0, (T, 1))).astype(np.float32))
+        out = prefill(ghip, s, x, idx, w, host=False)
+        want, eo = O.moe_forward(slabs, dim, inter, x, idx, w, want_expert_out=True, threads=16)
+        assert_close_combined(out, want, floor(slabs, dim, inter, x, idx, w, eo), "%s" % (rows,))
+        assert np.array_equal(out, prefill(ghip, s, x, idx, w, host=False))
+    finally:
+        ghip.apus_ghip_store_close(s)
+
+
+@pytest.mark.parametrize("dim,inter,rows", [
+    (256, 128, [1]), (512, 384, [1, 15, 16, 17, 0, 31, 32, 33, 48]),
+    (256, 256, [260, 3, 0, 16]), (1024, 128, [5] * 16)])
+def test_prefill_streams(ghip, dim, inter, rows):
+    """Little work: the weight streams, in passes of 16 rows."""
+    check(ghip, dim, inter, rows, nan=(len(rows) - 1,))
+
+
+@pytest.mark.parametrize("rows", [
+    [1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128],
+    [129, 159, 160, 161, 191, 192, 193, 223, 0, 8, 9, 40, 41, 70, 0, 100],
+    [224, 225, 255, 256, 257, 20, 0, 0, 0, 4, 7, 300, 50, 10, 16, 80]])
+def test_prefill_queued_bodies(ghip, rows):
+    """Sparse tiles with enough work for the queued form (more than 3 GFLOP,
+    under 128 rows an expert): each body's row remainders; the experts with
+    NaN codes take the exact one."""
+    dim, inter = 1024, 1024
+    assert 6.0 * sum(rows) * dim * inter > 3e9 and sum(rows) > len(rows)
+    T, k = routing_of(rows, np.random.default_rng(0)).shape
+    assert T * k < 128 * len(rows) * 16
+    check(ghip, dim, inter, rows + [0] * max(0, (T * k) // 127 + 1 - len(rows)), nan=(1, 4, 13))
+
+
+def test_prefill_permutation_limit(ghip):
+    """1024 pairs are sorted in one launch, 1025 in four: the same results for
+    the tokens both have. Up to 1024 experts."""
+    dim, inter, E = 256, 128, 1000
+    rng = np.random.default_rng(6)
+    slab = random_slabs(1, dim, inter, rng)[0]
+    s = open_store(ghip, E, dim, inter)
+    try:
+        for e in range(E):
+            assert ghip.apus_ghip_store_put(s, e, O.ptr(slab), slab.nbytes) == 0
+        x = O.f32_to_bf16(rng.standard_normal((1025, dim)).astype(np.float32))
+        idx = rng.integers(0, E, (1025, 1)).astype(np.int32)
+        w = rng.uniform(0.02, 0.6, (1025, 1)).astype(np.float32)
+        a = prefill(ghip, s, x[:1024], idx[:1024], w[:1024], host=False)
+        b = prefill(ghip, s, x, idx, w, host=False)
+        assert np.array_equal(a, b[:1024])
+        want, eo = O.moe_forward([slab] * E, dim, inter, x, idx, w, want_expert_out=True,
+                                 threads=16)
+        assert_close_combined(b, want, floor([slab] * E, dim, inter, x, idx, w, eo), "1025 pairs")
+    finally:
+        ghip.apus_ghip_store_close(s)
