@@ -19,7 +19,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
 C_SRCS = ["ghip_backend.c", "ghip_synth.c", "ghip_container.c"]
-HIP_SRCS = ["k_linear.hip", "k_gemm_bf16.hip", "k_rows.hip",
+HIP_SRCS = ["k_dequant.hip", "k_linear.hip", "k_gemm_bf16.hip", "k_rows.hip",
             "k_moe.hip", "k_moe_rows.hip", "k_moe_prefill.hip", "k_synth.hip"]
 
 INC = ["-I" + os.path.join(ROOT, "include"), "-I" + CSRC]

@@ -14,8 +14,7 @@
  *     gate (tests/test_gpu_dequant.py) checks it on every finite code x
  *     scale corners, including subnormal products.
  *   - EXACT: the same with the NaN codes replaced by +-480 (as the
- *     reference). Used when a matrix holds a 0x7F/0xFF code. The dequant
- *     entry's exact form is all integer (ghip_deq4_int).
+ *     reference). Used when a matrix holds a 0x7F/0xFF code.
  */
 #ifndef GHIP_DEVICE_H
 #define GHIP_DEVICE_H
@@ -57,6 +56,13 @@ __device__ __forceinline__ float ghip_e4m3_exact(uint32_t c) {
 
 typedef unsigned int ghip_u32x2 __attribute__((ext_vector_type(2)));
 
+/* v: the hardware convert of a code; sign: the code with its sign bit on top.
+ * The minimum picks 480 where v is a NaN (codes 0x7F and 0xFF). */
+__device__ __forceinline__ float ghip_e4m3_fix(float v, uint32_t sign) {
+    return __builtin_copysignf(__builtin_fminf(__builtin_fabsf(v), 480.0f),
+                               __uint_as_float(sign));
+}
+
 /* Four codes of one dword -> four dequantized bf16 packed in two dwords
  * (element j in bits [16*(j&1), +16) of dword j/2). EXACT: the hardware
  * convert gives a NaN for the two NaN codes only; the minimum of |value| and
@@ -69,14 +75,10 @@ __device__ __forceinline__ ghip_u32x2 ghip_deq4(uint32_t d, float s) {
     ghip_f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8((int)d, false);
     ghip_f32x2 b = __builtin_amdgcn_cvt_pk_f32_fp8((int)d, true);
     if (EXACT) {
-        auto fix = [](float v, uint32_t sign) {
-            return __builtin_copysignf(__builtin_fminf(__builtin_fabsf(v), 480.0f),
-                                       __uint_as_float(sign));
-        };
-        a[0] = fix(a[0], d << 24);
-        a[1] = fix(a[1], d << 16);
-        b[0] = fix(b[0], d << 8);
-        b[1] = fix(b[1], d);
+        a[0] = ghip_e4m3_fix(a[0], d << 24);
+        a[1] = ghip_e4m3_fix(a[1], d << 16);
+        b[0] = ghip_e4m3_fix(b[0], d << 8);
+        b[1] = ghip_e4m3_fix(b[1], d);
     }
     bf2 p, q;
     p[0] = (__bf16)(a[0] * s);
@@ -84,16 +86,6 @@ __device__ __forceinline__ ghip_u32x2 ghip_deq4(uint32_t d, float s) {
     q[0] = (__bf16)(b[0] * s);
     q[1] = (__bf16)(b[1] * s);
     return (ghip_u32x2){__builtin_bit_cast(uint32_t, p), __builtin_bit_cast(uint32_t, q)};
-}
-
-/* The same by the integer decode and the integer RNE narrow, which passes a
- * NaN product's bits through as the reference does. */
-__device__ __forceinline__ ghip_u32x2 ghip_deq4_int(uint32_t d, float s) {
-    uint32_t b0 = ghip_bf16_bits(ghip_e4m3_exact(d & 0xffu) * s);
-    uint32_t b1 = ghip_bf16_bits(ghip_e4m3_exact((d >> 8) & 0xffu) * s);
-    uint32_t b2 = ghip_bf16_bits(ghip_e4m3_exact((d >> 16) & 0xffu) * s);
-    uint32_t b3 = ghip_bf16_bits(ghip_e4m3_exact(d >> 24) * s);
-    return (ghip_u32x2){b0 | (b1 << 16), b2 | (b3 << 16)};
 }
 
 /* 16 codes (one 16-byte load) -> 8 dwords of packed bf16: lo holds codes

@@ -1,7 +1,5 @@
 /*
  * k_linear.hip — gfx950 kernels for the dense FP8-block path:
- *   K1  k_dequant16 / k_dequant_any : FP8-E4M3 + F32 128x128 scales -> BF16,
- *       bit-exact vs c/fp8blk.h:115-136 (apus_fp8blk_rows_scalar).
  *   K2  k_fp8_gemv_stream : decode / MTP-verify GEMV (M <= 4, many weight
  *       rows) with the dequant fused in registers and the k reduction on MFMA
  *       (v_mfma_f32_16x16x32_bf16), the composition of c/gdsa.h:525-534
@@ -23,52 +21,6 @@
 #include "ghip_device.h"
 #include <type_traits>
 #include "ghip_internal.h"
-
-/* ------------------------------------------------------------------------ */
-/* K1: dequant                                                              */
-/* ------------------------------------------------------------------------ */
-
-/* K % 16 == 0: one thread per 16 consecutive codes of a row (they share
- * one 128-block scale because 16 divides 128). */
-template <bool EXACT>
-__global__ __launch_bounds__(256) void k_dequant16(
-    const uint8_t *__restrict__ w, const float *__restrict__ s,
-    uint16_t *__restrict__ out, uint32_t O, uint32_t K, uint32_t nkb) {
-    const uint32_t cpr = K >> 4;                       /* chunks per row */
-    const size_t n = (size_t)O * cpr;
-    for (size_t c = (size_t)blockIdx.x * 256 + threadIdx.x; c < n;
-         c += (size_t)gridDim.x * 256) {
-        uint32_t o = (uint32_t)(c / cpr);
-        uint32_t k0 = (uint32_t)(c - (size_t)o * cpr) << 4;
-        float sc = s[(size_t)(o >> 7) * nkb + (k0 >> 7)];
-        ghip_u32x4 v = *(const ghip_u32x4 *)(w + (size_t)o * K + k0);
-        ghip_u32x4 r0, r1;
-        if (EXACT) {
-            const ghip_u32x2 a = ghip_deq4_int(v[0], sc), b = ghip_deq4_int(v[1], sc);
-            const ghip_u32x2 e = ghip_deq4_int(v[2], sc), f = ghip_deq4_int(v[3], sc);
-            r0 = (ghip_u32x4){a[0], a[1], b[0], b[1]};
-            r1 = (ghip_u32x4){e[0], e[1], f[0], f[1]};
-        } else {
-            ghip_deq16_u32<false>(v, sc, r0, r1);
-        }
-        ghip_u32x4 *dst = (ghip_u32x4 *)(out + (size_t)o * K + k0);
-        dst[0] = r0;
-        dst[1] = r1;
-    }
-}
-
-/* Any K: one thread per element, exact integer path. */
-__global__ __launch_bounds__(256) void k_dequant_any(
-    const uint8_t *__restrict__ w, const float *__restrict__ s,
-    uint16_t *__restrict__ out, uint32_t O, uint32_t K, uint32_t nkb) {
-    const size_t n = (size_t)O * K;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * 256) {
-        uint32_t o = (uint32_t)(i / K), k = (uint32_t)(i - (size_t)o * K);
-        float sc = s[(size_t)(o >> 7) * nkb + (k >> 7)];
-        out[i] = (uint16_t)ghip_bf16_bits(ghip_e4m3_exact(w[i]) * sc);
-    }
-}
 
 /* NaN-code scan: bytes whose low 7 bits are all ones (0x7F / 0xFF). */
 __global__ __launch_bounds__(256) void k_nan_scan(
@@ -141,31 +93,6 @@ static uint32_t grid_for(size_t items, size_t per_block, uint32_t cap) {
     if (g < 1) g = 1;
     if (g > cap) g = cap;
     return (uint32_t)g;
-}
-
-extern "C" hipError_t ghip_launch_dequant(const uint8_t *codes,
-                                          const float *scales, uint16_t *out,
-                                          size_t O, size_t K, int exact,
-                                          hipStream_t st) {
-    if (O == 0 || K == 0) return hipSuccess;
-    if (O > 0xffffffffu || K > 0xffffffffu) return hipErrorInvalidValue;
-    uint32_t nkb = (uint32_t)((K + 127) / 128);
-    bool aligned = (K % 16 == 0) && (((uintptr_t)codes & 15) == 0)
-                && (((uintptr_t)out & 15) == 0);
-    if (aligned) {
-        uint32_t g = grid_for(O * (K / 16), 256, 65536);
-        if (exact)
-            hipLaunchKernelGGL(k_dequant16<true>, dim3(g), dim3(256), 0, st,
-                               codes, scales, out, (uint32_t)O, (uint32_t)K, nkb);
-        else
-            hipLaunchKernelGGL(k_dequant16<false>, dim3(g), dim3(256), 0, st,
-                               codes, scales, out, (uint32_t)O, (uint32_t)K, nkb);
-    } else {
-        uint32_t g = grid_for(O * K, 256, 65536);
-        hipLaunchKernelGGL(k_dequant_any, dim3(g), dim3(256), 0, st, codes,
-                           scales, out, (uint32_t)O, (uint32_t)K, nkb);
-    }
-    return hipGetLastError();
 }
 
 extern "C" hipError_t ghip_launch_nan_scan(const uint8_t *codes, size_t n,
