@@ -52,6 +52,15 @@ typedef struct {
 
 #define GHIP_SCAN_SLOTS 4096
 
+/* Host transfers of up to GHIP_PIN_COPY bytes go through pinned memory and a
+ * copy kernel of the calls' stream: the runtime's copies of pageable memory
+ * cost ~5 us each on the host and wait for another queue (fp8blk_linear, q_a
+ * 1536 x 4096, M = 1: 31.9 -> 20.0 us, M = 16, 128 KB of x: 30.7 -> 25.5;
+ * 4096 x 16384, M = 4: 72.0 -> 30.9 with the one-pass kernel). Larger ones stay the runtime's:
+ * at M = 256, 2 MB of x, the host's own copy is what counts (148 us). */
+#define GHIP_PIN_COPY ((size_t)256 << 10)
+#define GHIP_PIN_BYTES (4 * GHIP_PIN_COPY)
+
 static struct {
     int inited, enabled, device;
     uint32_t n_cu;               /* CU count rounded up to the 8 XCDs */
@@ -60,6 +69,8 @@ static struct {
     /* grow-only staging (device) */
     void *d_w, *d_s, *d_x, *d_y;
     size_t cap_w, cap_s, cap_x, cap_y;
+    uint8_t *pin;                /* pinned host memory of the small transfers */
+    size_t pin_off;              /* its bytes in use until the next wait */
     uint32_t *d_flag;            /* ephemeral NaN-scan flag */
     uint32_t *d_flags;           /* pool of cached scan flags */
     int n_scan;
@@ -150,6 +161,7 @@ static int ghip_init(void) {
     /* the allocation-free prefill's scratch: its device address, taken once
      * here with the device current */
     HIPCHK(ghip_pf_scratch_init(dev));
+    HIPCHK(hipHostMalloc((void **)&G.pin, GHIP_PIN_BYTES, hipHostMallocCoherent));
     HIPCHK(hipMalloc((void **)&G.d_flag, 256));
     {
         /* word 0: the per-call NaN-scan flag; word 1: a constant 1 (the
@@ -325,9 +337,25 @@ uint64_t apus_ghip_bytes_d2h(void) { return G.d2h; }
 /* host-pointer entry points                                                */
 /* ------------------------------------------------------------------------ */
 
+/* A piece of the pinned memory for n bytes, or NULL if they are many, there is
+ * no room until the next wait, or the copy kernel cannot take the address. */
+static uint8_t *pin_take(const void *d, size_t n) {
+    const size_t r = (n + 15) & ~(size_t)15;
+    if (n > GHIP_PIN_COPY || r > GHIP_PIN_BYTES - G.pin_off || ((uintptr_t)d & 15)) return NULL;
+    uint8_t *p = G.pin + G.pin_off;
+    G.pin_off += r;
+    return p;
+}
+
 static int h2d(void *d, const void *h, size_t n) {
     if (n == 0) return 0;
-    HIPCHK(hipMemcpyAsync(d, h, n, hipMemcpyHostToDevice, G.stream));
+    uint8_t *p = pin_take(d, n);
+    if (p) {
+        memcpy(p, h, n);
+        HIPCHK(ghip_launch_copy16(d, p, n, G.stream));
+    } else {
+        HIPCHK(hipMemcpyAsync(d, h, n, hipMemcpyHostToDevice, G.stream));
+    }
     G.h2d += n;
     return 0;
 }
@@ -344,8 +372,12 @@ static const void *weight_dev(const void *h, size_t n, void **stage,
 }
 
 static int sync_out(void *h, const void *d, size_t n) {
-    HIPCHK(hipMemcpyAsync(h, d, n, hipMemcpyDeviceToHost, G.stream));
+    uint8_t *p = pin_take(d, n);
+    if (p) HIPCHK(ghip_launch_copy16(p, d, n, G.stream));
+    else HIPCHK(hipMemcpyAsync(h, d, n, hipMemcpyDeviceToHost, G.stream));
     HIPCHK(hipStreamSynchronize(G.stream));
+    if (p) memcpy(h, p, n);
+    G.pin_off = 0;
     G.d2h += n;
     return 0;
 }

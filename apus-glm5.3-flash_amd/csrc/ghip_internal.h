@@ -235,6 +235,7 @@ int ghip_container_layer(const char *dir, int layer, size_t slab_bytes,
 
 /* Fill n u32 words with value (a kernel, not a memset, so callers may
  * capture it in a graph). */
+hipError_t ghip_launch_copy16(void *dst, const void *src, size_t n, hipStream_t st);
 hipError_t ghip_launch_fill_u32(uint32_t *p, size_t n, uint32_t value,
                                 hipStream_t st);
 

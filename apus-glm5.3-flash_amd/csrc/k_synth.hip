@@ -91,6 +91,27 @@ extern "C" hipError_t ghip_launch_fill_u32(uint32_t *p, size_t n, uint32_t value
     return hipGetLastError();
 }
 
+/* n bytes, both sides 16-byte aligned, between device and pinned host memory:
+ * small host transfers stay kernels of the calls' own stream. Bound by the
+ * launch and one trip over the bus (256 threads a workgroup, 16 bytes each:
+ * every load of up to 64 KB is in flight at once). */
+__global__ __launch_bounds__(256) void k_copy16(const uint8_t *__restrict__ src,
+                                                uint8_t *__restrict__ dst, uint32_t n) {
+    const uint32_t n16 = n / 16u, i = blockIdx.x * 256u + threadIdx.x;
+    if (i < n16) ((uint4 *)dst)[i] = ((const uint4 *)src)[i];
+    const uint32_t j = n16 * 16u + threadIdx.x;
+    if (blockIdx.x == gridDim.x - 1u && j < n) dst[j] = src[j];
+}
+
+extern "C" hipError_t ghip_launch_copy16(void *dst, const void *src, size_t n, hipStream_t st) {
+    if (n == 0) return hipSuccess;
+    if ((((uintptr_t)dst | (uintptr_t)src) & 15) || n > ((size_t)1 << 30))
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_copy16, dim3((uint32_t)((n + 4095) / 4096)), dim3(256), 0, st,
+                       (const uint8_t *)src, (uint8_t *)dst, (uint32_t)n);
+    return hipGetLastError();
+}
+
 /* One wave that waits `ticks` of the constant-rate wall clock and exits:
  * holds a stream for a fixed time with no memory traffic (a bounded wait:
  * every launch ends). */
