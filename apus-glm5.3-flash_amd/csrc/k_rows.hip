@@ -266,7 +266,7 @@ static const RwCfg rw_fp8[] = {
     RW_CFG(false, 16, 1, 8, 1, 1, 0.85f), RW_CFG(false, 16, 2, 8, 2, 2, 1.30f),
     RW_CFG(false, 16, 2, 4, 2, 2, 1.30f), RW_CFG(false, 32, 1, 8, 1, 1, 1.30f),
     RW_CFG(false, 32, 2, 8, 1, 1, 1.70f), RW_CFG(false, 32, 2, 4, 1, 1, 1.70f),
-    RW_CFG(false, 64, 2, 4, 1, 1, 2.50f),
+    RW_CFG(false, 64, 2, 4, 1, 1, 2.20f),
 };
 static const RwCfg rw_bf16[] = {
     RW_CFG(true, 8, 1, 8, 2, 2, 0.50f),  RW_CFG(true, 8, 1, 4, 2, 2, 0.50f),
@@ -290,7 +290,17 @@ static float rw_estimate(const RwCfg &c, bool bf, size_t M, size_t N, size_t K, 
     const double rounds = (double)(size_t)((wgs + n_cu - 1) / n_cu);
     const double nc = (double)(size_t)((nch + c.ks - 1) / c.ks);
     const double hbm = (double)N * (double)(bf ? 2 * K : K) / 6.5e6;
-    const double t = rounds * nc * c.chunk;
+    /* A round's first loads and reduction: hidden under no other workgroup by
+     * the form of 64 rows (16384 x 1536: 13.4 us at M = 64 in one round, 25.4
+     * at 128 in two, where the MFMA GEMM takes 21.5), and past the first round
+     * of other FP8 forms with two or more blocks where a wave has few chunks
+     * (32768 x 1024: M = 48 in six rounds of 16 rows 37.9 us, M = 64 in four
+     * of 32 27.5, the GEMM 16.6 and 18; 16384 x 1536, M = 80, three rounds 22,
+     * the GEMM 20.5). */
+    const double over = c.mr > 32 ? 3.8 * rounds
+                        : !bf && c.mr * c.nt >= 32 && nc < 8.0 ? 2.0 * (rounds - 1.0)
+                                                         : 0.0;
+    const double t = rounds * nc * c.chunk + over;
     const double lds = t < hbm ? 0.0015 * hbm * c.mr * c.nt : 0.0;
     return (float)(2.3 + (t > hbm ? t + 0.1 * hbm : hbm + 0.1 * t) + lds);
 }
