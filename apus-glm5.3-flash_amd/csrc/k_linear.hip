@@ -6,9 +6,8 @@
  *       (dequant -> bf16 -> fp32-accumulated GEMM -> RNE bf16). Other row
  *       counts and shapes: k_rows.hip, k_moe_prefill.hip (k_fp8_gemm) and,
  *       for BF16 weights, k_rows.hip and k_gemm_bf16.hip.
- *   k_fp8_linear_any / k_bf16_linear_any : shape-general fallbacks (K not a
- *       multiple of 128 / 64, unaligned operands) with the exact integer
- *       decode.
+ *   k_linear_any : shape-general fallback (K not a multiple of 128 / 64,
+ *       unaligned operands) with the exact integer decode.
  *   k_nan_scan : flags the out-of-contract NaN codes 0x7F/0xFF so callers
  *       can select the exact decode for such weights.
  *
@@ -40,7 +39,7 @@ __global__ __launch_bounds__(256) void k_nan_scan(
 }
 
 /* ------------------------------------------------------------------------ */
-/* shape-general fallbacks: one wave per (row, m), exact decode             */
+/* shape-general fallback: exact decode                                     */
 /* ------------------------------------------------------------------------ */
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -48,40 +47,77 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-__global__ __launch_bounds__(256) void k_fp8_linear_any(
-    const uint8_t *__restrict__ W, const float *__restrict__ S,
+/* One wave per weight row and MR rows of x: the decode and the weight's loads
+ * serve all of them, and the loads of four k steps are in flight together. Each
+ * sum is its lanes' k = lane, lane + 64, ... in order and then the wave's, for
+ * any MR. Bound by issue (any alignment: loads of one element): 2000 x 2001, M
+ * = 64, FP8 73 us and BF16 46 (a wave a row of x 183 and 132); M = 1 8.4 and
+ * 3.7 (10.8 and 5.8, each load waited for). */
+template <bool BF, int MR>
+__global__ __launch_bounds__(256) void k_linear_any(
+    const void *__restrict__ W, const float *__restrict__ S,
     const uint16_t *__restrict__ X, uint16_t *__restrict__ Y, uint32_t M,
     uint32_t O, uint32_t K, uint32_t nkb) {
     const uint32_t lane = threadIdx.x & 63u;
     const size_t item = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (item >= (size_t)M * O) return;
-    const uint32_t m = (uint32_t)(item / O), o = (uint32_t)(item - (size_t)m * O);
-    const uint8_t *wr = W + (size_t)o * K;
-    const float *srow = S + (size_t)(o >> 7) * nkb;
-    const uint16_t *xr = X + (size_t)m * K;
-    float acc = 0.0f;
-    for (uint32_t k = lane; k < K; k += 64) {
-        float wv = ghip_bf16_round(ghip_e4m3_exact(wr[k]) * srow[k >> 7]);
-        acc += wv * ghip_bf16_f32(xr[k]);
+    const uint32_t mt = (M + MR - 1u) / MR;
+    if (item >= (size_t)mt * O) return;
+    const uint32_t m0 = (uint32_t)(item / O) * MR, o = (uint32_t)(item % O);
+    const uint8_t *wr = (const uint8_t *)W + (size_t)o * K * (BF ? 2u : 1u);
+    const float *srow = BF ? nullptr : S + (size_t)(o >> 7) * nkb;
+    const uint16_t *xr[MR];
+#pragma unroll
+    for (int i = 0; i < MR; i++) xr[i] = X + (size_t)min(m0 + i, M - 1u) * K;
+    auto weight = [&](uint32_t k) -> float {
+        if (BF) return ghip_bf16_f32(((const uint16_t *)wr)[k]);
+        return ghip_bf16_round(ghip_e4m3_exact(wr[k]) * srow[k >> 7]);
+    };
+    float acc[MR] = {};
+    for (uint32_t k0 = 0; k0 < K; k0 += 256u) {
+        float wv[4], xv[4][MR];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t k = k0 + 64u * j + lane, kc = min(k, K - 1u);
+            wv[j] = weight(kc);
+#pragma unroll
+            for (int i = 0; i < MR; i++) {
+                /* past K a lane adds +0 */
+                const float v = ghip_bf16_f32(xr[i][kc]);
+                xv[j][i] = k < K ? v : 0.0f;
+            }
+            wv[j] = k < K ? wv[j] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int i = 0; i < MR; i++) acc[i] += wv[j] * xv[j][i];
     }
-    acc = wave_sum(acc);
-    if (lane == 0) Y[(size_t)m * O + o] = (uint16_t)ghip_bf16_bits(acc);
+#pragma unroll
+    for (int i = 0; i < MR; i++) {
+        const float s = wave_sum(acc[i]);
+        if (lane == 0 && m0 + i < M) Y[(size_t)(m0 + i) * O + o] = (uint16_t)ghip_bf16_bits(s);
+    }
 }
 
-__global__ __launch_bounds__(256) void k_bf16_linear_any(
-    const uint16_t *__restrict__ W, const uint16_t *__restrict__ X,
-    uint16_t *__restrict__ Y, uint32_t M, uint32_t O, uint32_t K) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const size_t item = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (item >= (size_t)M * O) return;
-    const uint32_t m = (uint32_t)(item / O), o = (uint32_t)(item - (size_t)m * O);
-    const uint16_t *wr = W + (size_t)o * K;
-    const uint16_t *xr = X + (size_t)m * K;
-    float acc = 0.0f;
-    for (uint32_t k = lane; k < K; k += 64)
-        acc += ghip_bf16_f32(wr[k]) * ghip_bf16_f32(xr[k]);
-    acc = wave_sum(acc);
-    if (lane == 0) Y[(size_t)m * O + o] = (uint16_t)ghip_bf16_bits(acc);
+/* The most rows of x a wave (8, 4, 2) that leave 4096 waves, four a SIMD. */
+template <bool BF>
+static hipError_t launch_linear_any(const void *w, const float *s, const uint16_t *x, uint16_t *y,
+                                    size_t M, size_t O, size_t K, hipEvent_t ev0, hipEvent_t ev1,
+                                    hipStream_t st) {
+    if (M * O > 0xffffffffull * 4) return hipErrorInvalidValue;
+    const uint32_t nkb = (uint32_t)((K + 127) / 128);
+    size_t mr = 8;
+    while (mr > 1 && (mr > M || O * ((M + mr - 1) / mr) < 4096)) mr >>= 1;
+    const dim3 g((uint32_t)((O * ((M + mr - 1) / mr) + 3) / 4));
+#define LINEAR_ANY(R) \
+    GHIP_LAUNCH(ev0, ev1, (k_linear_any<BF, R>), g, dim3(256), 0, st, w, s, x, y, (uint32_t)M, \
+                (uint32_t)O, (uint32_t)K, nkb)
+    if (mr == 8) LINEAR_ANY(8);
+    else if (mr == 4) LINEAR_ANY(4);
+    else if (mr == 2) LINEAR_ANY(2);
+    else LINEAR_ANY(1);
+#undef LINEAR_ANY
+    return hipGetLastError();
 }
 
 /* ------------------------------------------------------------------------ */
@@ -297,13 +333,7 @@ extern "C" hipError_t ghip_launch_fp8_linear(const uint8_t *codes,
     /* timing events: start on the first launch, stop on the last */
     hipEvent_t ev0 = ev ? ev[0] : nullptr, ev1 = ev ? ev[1] : nullptr;
     if (!g_gs_ncu || !ghip_rows_fits(0, M, O, K, codes, x)) {
-        uint32_t nkb = (uint32_t)((K + 127) / 128);
-        size_t items = M * O;
-        if (items > 0xffffffffull * 4) return hipErrorInvalidValue;
-        GHIP_LAUNCH(ev0, ev1, k_fp8_linear_any, dim3((uint32_t)((items + 3) / 4)),
-                    dim3(256), 0, st, codes, scales, x, y, (uint32_t)M,
-                    (uint32_t)O, (uint32_t)K, nkb);
-        return hipGetLastError();
+        return launch_linear_any<false>(codes, scales, x, y, M, O, K, ev0, ev1, st);
     }
     /* up to 4 rows against enough weight rows that every wave holds a row
      * group for half of K: x staged once in LDS (16384 x 4096, M = 1: 11.6 us
@@ -346,11 +376,7 @@ extern "C" hipError_t ghip_launch_bf16_linear(const uint16_t *w,
             return ghip_launch_rows(1, w, nullptr, x, y, M, O, K, nullptr, g_gs_ncu, ev0, ev1,
                                     st);
     }
-    size_t items = M * O;
-    if (items > 0xffffffffull * 4) return hipErrorInvalidValue;
-    GHIP_LAUNCH(ev0, ev1, k_bf16_linear_any, dim3((uint32_t)((items + 3) / 4)),
-                dim3(256), 0, st, w, x, y, (uint32_t)M, (uint32_t)O, (uint32_t)K);
-    return hipGetLastError();
+    return launch_linear_any<true>(w, nullptr, x, y, M, O, K, ev0, ev1, st);
 }
 
 extern "C" hipError_t ghip_linear_init(uint32_t n_cu) {
