@@ -52,6 +52,16 @@ def test_spilling_kernel_fails_the_gate():
             b.check_resources(bad, required=())
 
 
+def test_sgpr_spill_limit():
+    """k_fp8_gemm may spill no SGPR: four of them made it 1-4% slower."""
+    b = _build_mod()
+    ok, _ = b.resource_usage(_remarks("_Z10k_fp8_gemmPKh", 0, 0, 0))
+    b.check_resources(ok, required=())
+    bad, _ = b.resource_usage(_remarks("_Z10k_fp8_gemmPKh", 0, 4, 0))
+    with pytest.raises(RuntimeError, match="k_fp8_gemm.*4 SGPR spills"):
+        b.check_resources(bad, required=())
+
+
 def test_gate_fails_without_remarks():
     """No parsed remarks, a required kernel without remarks, or a remark
     block without its spill and scratch figures fail the build: a gate that
