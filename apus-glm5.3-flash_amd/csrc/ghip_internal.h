@@ -35,6 +35,12 @@ hipError_t ghip_launch_fp8_linear(const uint8_t *codes, const float *scales,
                                   size_t O, size_t K, const uint32_t *exact_dev,
                                   const hipEvent_t *ev, hipStream_t st);
 
+/* The kernel that an FP8 linear takes (host only; no device needed): any shape
+ * by k_linear_any, k_fp8_gemv_stream, k_rows_gemm or k_fp8_gemm. */
+enum { GHIP_ROUTE_ANY, GHIP_ROUTE_GEMV, GHIP_ROUTE_ROWS, GHIP_ROUTE_GEMM };
+int ghip_fp8_linear_route(const void *codes, const void *x, const void *y, size_t M, size_t O,
+                          size_t K, uint32_t n_cu);
+
 /* BF16-weight GEMV/GEMM: y[M,O] = x[M,K] . W[O,K]^T. Any shape. ev: NULL or
  * two timing events (start on the first launch, stop on the last). */
 hipError_t ghip_launch_bf16_linear(const uint16_t *w, const uint16_t *x,
@@ -56,7 +62,7 @@ hipError_t ghip_bf16_gemm_init(void);
 /* Weight-streaming linear for a few activation rows: bf != 0 BF16 weights (K
  * % 64 == 0), else FP8 codes (K % 128 == 0) with scales and exact_dev as
  * ghip_launch_fp8_linear; 16-byte aligned w and x (ghip_rows_fits). One
- * launch, no workspace. e0/e1: NULL or timing events. The estimate is in
+ * launch (several past 65535 row tiles), no workspace. e0/e1: NULL or timing events. The estimate is in
  * microseconds. */
 int ghip_rows_fits(int bf, size_t M, size_t N, size_t K, const void *w, const void *x);
 float ghip_rows_estimate(int bf, size_t M, size_t N, size_t K, uint32_t n_cu);

@@ -320,6 +320,22 @@ static float fp8_gemm_estimate(size_t M, size_t O, size_t K) {
     return 11.0f + (float)((double)O * (double)K / 6.0e6) + 0.04f * (float)M;
 }
 
+/* The kernel of an FP8 linear on n_cu CUs. */
+extern "C" int ghip_fp8_linear_route(const void *codes, const void *x, const void *y, size_t M,
+                                     size_t O, size_t K, uint32_t n_cu) {
+    const bool rows = n_cu && ghip_rows_fits(0, M, O, K, codes, x);
+    /* up to 4 rows against enough weight rows that every wave holds a row
+     * group for half of K: x staged once in LDS (16384 x 4096, M = 1: 11.6 us
+     * against 12.0 with x streamed beside the weights; 16384 x 1536: 5.9
+     * against 6.2; below that many rows the streamed form is as good or
+     * better, 7000 x 2048 4.9 against 6.0) */
+    if (rows && M <= 4 && (O + 63) / 64 >= n_cu && M * K * 2 <= GS_X_MAX) return GHIP_ROUTE_GEMV;
+    if (n_cu && M >= GHIP_GEMM_MIN_M && ghip_fp8_gemm_fits(M, O, K, codes, x, y)
+        && (M >= 256 || !rows || fp8_gemm_estimate(M, O, K) < ghip_rows_estimate(0, M, O, K, n_cu)))
+        return GHIP_ROUTE_GEMM;
+    return rows ? GHIP_ROUTE_ROWS : GHIP_ROUTE_ANY;
+}
+
 extern "C" hipError_t ghip_launch_fp8_linear(const uint8_t *codes,
                                              const float *scales,
                                              const uint16_t *x, uint16_t *y,
@@ -332,27 +348,21 @@ extern "C" hipError_t ghip_launch_fp8_linear(const uint8_t *codes,
         return hipErrorInvalidValue;
     /* timing events: start on the first launch, stop on the last */
     hipEvent_t ev0 = ev ? ev[0] : nullptr, ev1 = ev ? ev[1] : nullptr;
-    if (!g_gs_ncu || !ghip_rows_fits(0, M, O, K, codes, x)) {
-        return launch_linear_any<false>(codes, scales, x, y, M, O, K, ev0, ev1, st);
-    }
-    /* up to 4 rows against enough weight rows that every wave holds a row
-     * group for half of K: x staged once in LDS (16384 x 4096, M = 1: 11.6 us
-     * against 12.0 with x streamed beside the weights; 16384 x 1536: 5.9
-     * against 6.2; below that many rows the streamed form is as good or
-     * better, 7000 x 2048 4.9 against 6.0) */
-    if (M <= 4 && (O + 63) / 64 >= g_gs_ncu && M * K * 2 <= GS_X_MAX) {
+    switch (ghip_fp8_linear_route(codes, x, y, M, O, K, g_gs_ncu)) {
+    case GHIP_ROUTE_GEMV:
         switch (M) {
         case 4: return launch_gemv_m<4>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
         case 3: return launch_gemv_m<3>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
         case 2: return launch_gemv_m<2>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
         default: return launch_gemv_m<1>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
         }
+    case GHIP_ROUTE_GEMM:
+        return ghip_launch_fp8_gemm(codes, scales, x, y, M, O, K, exact_dev, g_gs_ncu, ev, st);
+    case GHIP_ROUTE_ROWS:
+        return ghip_launch_rows(0, codes, scales, x, y, M, O, K, exact_dev, g_gs_ncu, ev0, ev1,
+                                st);
+    default: return launch_linear_any<false>(codes, scales, x, y, M, O, K, ev0, ev1, st);
     }
-    if (M >= GHIP_GEMM_MIN_M && ghip_fp8_gemm_fits(M, O, K, codes, x, y)
-        && (M >= 256 || fp8_gemm_estimate(M, O, K) < ghip_rows_estimate(0, M, O, K, g_gs_ncu)))
-        return ghip_launch_fp8_gemm(codes, scales, x, y, M, O, K, exact_dev, g_gs_ncu, ev,
-                                    st);
-    return ghip_launch_rows(0, codes, scales, x, y, M, O, K, exact_dev, g_gs_ncu, ev0, ev1, st);
 }
 
 extern "C" hipError_t ghip_launch_bf16_linear(const uint16_t *w,

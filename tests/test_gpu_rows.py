@@ -93,3 +93,17 @@ def test_rows_not_finite(ghip):
     x[4, 9] = 0x7F80
     y = O.bf16_to_f32(run_fp8(ghip, codes, scales, x, 0))
     assert np.all(np.isposinf(y[4])) and np.all(np.isfinite(y[:4]))
+
+
+def test_rows_several_launches(ghip):
+    """More rows than one launch's 65535 row tiles hold, whatever the tile:
+    every row is computed once, from its own x."""
+    M, N, K, period = 65535 * 64 + 5, 20, 128, 1009
+    codes, scales, x = fp8_inputs(period, N, K, False)
+    w = O.dequant(codes, scales, threads=8)
+    floor = 2.0 ** -8 * (np.abs(O.bf16_to_f32(x)) @ np.abs(O.bf16_to_f32(w)).T)
+    got = run_fp8(ghip, codes, scales, np.resize(x, (M, K)), 0)
+    assert_close(got[:period], O.gemm(w, x, threads=16), floor, "first rows")
+    whole = M // period * period
+    assert (got[:whole].reshape(-1, period, N) == got[:period]).all()
+    assert np.array_equal(got[whole:], got[:M - whole])

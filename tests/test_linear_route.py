@@ -1,0 +1,47 @@
+"""Which kernel a linear takes (csrc/k_linear.hip), asked of the library's own
+dispatch: host code, so no device and no buffers of these sizes are needed."""
+import ctypes
+
+import pytest
+
+ANY, GEMV, ROWS, GEMM = range(4)
+NCU = 256
+P = ctypes.c_void_p(1 << 20)
+
+
+def fp8(pkg, M, N, K, codes=P, x=P, y=P, ncu=NCU):
+    f = pkg.load().ghip_fp8_linear_route
+    f.restype = ctypes.c_int
+    f.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_size_t] * 3 + [ctypes.c_uint32]
+    return f(codes, x, y, M, N, K, ncu)
+
+
+# the most rows that 65535 row tiles of 16 rows hold, and more than 65535
+# tiles of any height
+EDGE = 65535 * 16
+
+
+@pytest.mark.parametrize("M", [EDGE, EDGE + 1, 1300000])
+def test_fp8_very_many_rows_stay_on_the_gemm(pkg, M):
+    """What the MFMA GEMM takes (N % 256 == 0, 2 M K under 4 GiB) goes there
+    at any number of rows."""
+    assert fp8(pkg, M, 16384, 1536) == GEMM
+    assert fp8(pkg, M, 256, 128) == GEMM
+
+
+@pytest.mark.parametrize("M", [EDGE, EDGE + 1, 65535 * 64 + 1, 0x7FFFFFFF])
+def test_fp8_very_many_rows_off_the_gemm(pkg, M):
+    """What it does not take is streamed, in as many launches as its row tiles
+    need, and never falls to the kernel of any shape."""
+    assert fp8(pkg, M, 300, 128) == ROWS
+    assert fp8(pkg, M, 16384, 4096) == ROWS          # 2 M K over 4 GiB
+
+
+def test_fp8_other_shapes(pkg):
+    off = ctypes.c_void_p(P.value + 2)
+    assert fp8(pkg, 1, 16384, 4096) == GEMV and fp8(pkg, 4, 16384, 1536) == GEMV
+    assert fp8(pkg, 5, 16384, 4096) == ROWS and fp8(pkg, 1, 512, 4096) == ROWS
+    assert fp8(pkg, 256, 512, 4096) == GEMM and fp8(pkg, 256, 500, 4096) == ROWS
+    assert fp8(pkg, 1, 512, 4095) == ANY and fp8(pkg, 300, 512, 4096, codes=off) == ANY
+    assert fp8(pkg, 300, 512, 4096, x=off) == ANY and fp8(pkg, 300, 512, 4096, y=off) == ROWS
+    assert fp8(pkg, 300, 512, 4096, ncu=0) == ANY
