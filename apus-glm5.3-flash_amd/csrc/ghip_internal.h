@@ -16,11 +16,19 @@
 extern "C" {
 #endif
 
+/* The most threads along x of one launch: the runtime refuses 2^32 and, past
+ * it, launches the remainder of the count without an error. */
+#define GHIP_MAX_THREADS ((size_t)0xffffffffu)
+
 /* K1: out[O,K] bf16 = bf16(e4m3(codes) * scale of the 128x128 block).
  * exact != 0 selects the integer decode (required for NaN codes). */
 hipError_t ghip_launch_dequant(const uint8_t *codes, const float *scales,
                                uint16_t *out, size_t O, size_t K, int exact,
                                hipStream_t st);
+
+/* Rows of one launch of the chunked dequant kernel: O, or a whole number of
+ * scale blocks; 0 when no 128 rows of K codes fit. */
+size_t ghip_dequant_rows(size_t O, size_t K);
 
 /* Scan codes for the NaN codes 0x7F/0xFF: *flag (device u32) |= 1 when any
  * is present. The caller zeroes *flag first. */
@@ -62,7 +70,7 @@ hipError_t ghip_bf16_gemm_init(void);
 /* Weight-streaming linear for a few activation rows: bf != 0 BF16 weights (K
  * % 64 == 0), else FP8 codes (K % 128 == 0) with scales and exact_dev as
  * ghip_launch_fp8_linear; 16-byte aligned w and x (ghip_rows_fits). One
- * launch (several past 65535 row tiles), no workspace. e0/e1: NULL or timing events. The estimate is in
+ * launch (several past 65535 row tiles or 2^32 threads), no workspace. e0/e1: NULL or timing events. The estimate is in
  * microseconds. */
 int ghip_rows_fits(int bf, size_t M, size_t N, size_t K, const void *w, const void *x);
 float ghip_rows_estimate(int bf, size_t M, size_t N, size_t K, uint32_t n_cu);

@@ -126,6 +126,11 @@ __global__ __launch_bounds__(256) void k_dequant_any(
     }
 }
 
+extern "C" size_t ghip_dequant_rows(size_t O, size_t K) {
+    const size_t most = GHIP_MAX_THREADS / 256u * (DQ_U * 256u * DQ_CHUNK);
+    return O <= most / K ? O : most / K / 128u * 128u;
+}
+
 extern "C" hipError_t ghip_launch_dequant(const uint8_t *codes,
                                           const float *scales, uint16_t *out,
                                           size_t O, size_t K, int exact,
@@ -133,26 +138,34 @@ extern "C" hipError_t ghip_launch_dequant(const uint8_t *codes,
     if (O == 0 || K == 0) return hipSuccess;
     if (O > 0xffffffffu || K > 0xffffffffu) return hipErrorInvalidValue;
     const uint32_t nkb = (uint32_t)((K + 127) / 128);
-    const size_t n = O * K, per = DQ_U * 256u * DQ_CHUNK, blocks = (n + per - 1) / per;
+    const size_t per = DQ_U * 256u * DQ_CHUNK, rows = ghip_dequant_rows(O, K);
     /* rows of under 8 codes could end twice in a chunk; the sums of a
      * workgroup's k and of its blocks stay within 32 bits */
-    if (K >= DQ_CHUNK && K <= 0x7fffffffu && blocks <= 0x7fffffffu
-        && ((uintptr_t)codes & 7) == 0 && ((uintptr_t)out & 15) == 0) {
-        const dim3 g((uint32_t)blocks);
-        /* the fast decode is for K % 16 == 0 and 16-byte aligned codes only:
-         * elsewhere NaN codes have their numbers whatever `exact` says */
-        if (K % 8)
-            hipLaunchKernelGGL((k_dequant<true, true>), g, dim3(256), 0, st, codes,
-                               scales, out, (uint32_t)O, (uint32_t)K, nkb);
-        else if (exact || K % 16 || ((uintptr_t)codes & 15))
-            hipLaunchKernelGGL((k_dequant<true, false>), g, dim3(256), 0, st, codes,
-                               scales, out, (uint32_t)O, (uint32_t)K, nkb);
-        else
-            hipLaunchKernelGGL((k_dequant<false, false>), g, dim3(256), 0, st, codes,
-                               scales, out, (uint32_t)O, (uint32_t)K, nkb);
-        return hipGetLastError();
+    if (K >= DQ_CHUNK && K <= 0x7fffffffu && rows && ((uintptr_t)codes & 7) == 0
+        && ((uintptr_t)out & 15) == 0) {
+        for (size_t r = 0; r < O; r += rows) {
+            const size_t n = O - r < rows ? O - r : rows;
+            const dim3 g((uint32_t)((n * K + per - 1) / per));
+            const uint8_t *w = codes + r * K;
+            const float *s = scales + (r / 128) * nkb;
+            uint16_t *o = out + r * K;
+            /* the fast decode is for K % 16 == 0 and 16-byte aligned codes only:
+             * elsewhere NaN codes have their numbers whatever `exact` says */
+            if (K % 8)
+                hipLaunchKernelGGL((k_dequant<true, true>), g, dim3(256), 0, st, w, s, o,
+                                   (uint32_t)n, (uint32_t)K, nkb);
+            else if (exact || K % 16 || ((uintptr_t)codes & 15))
+                hipLaunchKernelGGL((k_dequant<true, false>), g, dim3(256), 0, st, w, s, o,
+                                   (uint32_t)n, (uint32_t)K, nkb);
+            else
+                hipLaunchKernelGGL((k_dequant<false, false>), g, dim3(256), 0, st, w, s, o,
+                                   (uint32_t)n, (uint32_t)K, nkb);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
     }
-    size_t g = (n + 255) / 256;
+    size_t g = (O * K + 255) / 256;
     if (g > 65536) g = 65536;
     hipLaunchKernelGGL(k_dequant_any, dim3((uint32_t)g), dim3(256), 0, st, codes,
                        scales, out, (uint32_t)O, (uint32_t)K, nkb);

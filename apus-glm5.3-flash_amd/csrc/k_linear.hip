@@ -57,9 +57,9 @@ template <bool BF, int MR>
 __global__ __launch_bounds__(256) void k_linear_any(
     const void *__restrict__ W, const float *__restrict__ S,
     const uint16_t *__restrict__ X, uint16_t *__restrict__ Y, uint32_t M,
-    uint32_t O, uint32_t K, uint32_t nkb) {
+    uint32_t O, uint32_t K, uint32_t nkb, uint32_t blk0) {
     const uint32_t lane = threadIdx.x & 63u;
-    const size_t item = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const size_t item = ((size_t)blk0 + blockIdx.x) * 4 + (threadIdx.x >> 6);
     const uint32_t mt = (M + MR - 1u) / MR;
     if (item >= (size_t)mt * O) return;
     const uint32_t m0 = (uint32_t)(item / O) * MR, o = (uint32_t)(item % O);
@@ -108,16 +108,22 @@ static hipError_t launch_linear_any(const void *w, const float *s, const uint16_
     const uint32_t nkb = (uint32_t)((K + 127) / 128);
     size_t mr = 8;
     while (mr > 1 && (mr > M || O * ((M + mr - 1) / mr) < 4096)) mr >>= 1;
-    const dim3 g((uint32_t)((O * ((M + mr - 1) / mr) + 3) / 4));
+    const size_t blocks = (O * ((M + mr - 1) / mr) + 3) / 4, most = GHIP_MAX_THREADS / 256u;
 #define LINEAR_ANY(R) \
-    GHIP_LAUNCH(ev0, ev1, (k_linear_any<BF, R>), g, dim3(256), 0, st, w, s, x, y, (uint32_t)M, \
-                (uint32_t)O, (uint32_t)K, nkb)
-    if (mr == 8) LINEAR_ANY(8);
-    else if (mr == 4) LINEAR_ANY(4);
-    else if (mr == 2) LINEAR_ANY(2);
-    else LINEAR_ANY(1);
+    GHIP_LAUNCH(b == 0 ? ev0 : nullptr, b + n == blocks ? ev1 : nullptr, (k_linear_any<BF, R>), \
+                dim3((uint32_t)n), dim3(256), 0, st, w, s, x, y, (uint32_t)M, (uint32_t)O, \
+                (uint32_t)K, nkb, (uint32_t)b)
+    for (size_t b = 0; b < blocks; b += most) {
+        const size_t n = blocks - b < most ? blocks - b : most;
+        if (mr == 8) LINEAR_ANY(8);
+        else if (mr == 4) LINEAR_ANY(4);
+        else if (mr == 2) LINEAR_ANY(2);
+        else LINEAR_ANY(1);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
 #undef LINEAR_ANY
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 /* ------------------------------------------------------------------------ */

@@ -31,7 +31,10 @@
 
 #define RW_NW 8                  /* waves per workgroup */
 #define RW_LDS_MAX (160u * 1024u)
-#define RW_MAX_TILES ((size_t)65535)  /* row tiles a launch */
+/* a launch's row tiles (grid y) and workgroups along the weight rows (grid x:
+ * under 2^32 threads); more take several launches */
+#define RW_MAX_TILES ((size_t)65535)
+#define RW_MAX_BLOCKS (GHIP_MAX_THREADS / (RW_NW * 64))
 
 /* LDS: each wave's SL slots of x and weights; the partial sums reuse it */
 template <bool BF, int MR, int NT, int SL>
@@ -49,7 +52,7 @@ template <bool BF, int MR, int NT, int KS, int NA, int SL>
 __global__ __launch_bounds__(RW_NW * 64, 1) void k_rows_gemm(
     const uint8_t *__restrict__ W, const float *__restrict__ S, const uint16_t *__restrict__ X,
     uint16_t *__restrict__ Y, uint32_t M, uint32_t O, uint32_t K,
-    const uint32_t *__restrict__ exact_flag, uint32_t tile0) {
+    const uint32_t *__restrict__ exact_flag, uint32_t blk0, uint32_t tile0) {
     constexpr uint32_t GPP = RW_NW / KS;                 /* row groups per workgroup */
     constexpr uint32_t MT = MR < 16 ? 1 : MR / 16;
     constexpr uint32_t XI = BF ? (MR < 8 ? 1 : MR / 8) : MR / 4;  /* x loads per chunk */
@@ -67,7 +70,7 @@ __global__ __launch_bounds__(RW_NW * 64, 1) void k_rows_gemm(
     const uint32_t nch = KB >> 7, nkb = K >> 7;
     const uint32_t part = wv % KS, slot = wv / KS;
     const uint32_t c0 = part * nch / KS, c1 = (part + 1u) * nch / KS, nc = c1 - c0;
-    const uint32_t grp = blockIdx.x * GPP + slot, row0 = grp * (16u * NT);
+    const uint32_t blk = blk0 + blockIdx.x, grp = blk * GPP + slot, row0 = grp * (16u * NT);
     const uint32_t m0 = (tile0 + blockIdx.y) * MR;
     const uint32_t mrows = min(M - m0, (uint32_t)MR);
     ghip_f32x4 acc[MT][NT];
@@ -223,7 +226,7 @@ __global__ __launch_bounds__(RW_NW * 64, 1) void k_rows_gemm(
     for (uint32_t v = tid; v < GPP * MR * 16u * NT; v += RW_NW * 64u) {
         const uint32_t sl = v / (MR * 16u * NT), e = v - sl * (MR * 16u * NT);
         const uint32_t m = e / (16u * NT), c = e - m * (16u * NT);
-        const uint32_t o = (blockIdx.x * GPP + sl) * (16u * NT) + c;
+        const uint32_t o = (blk * GPP + sl) * (16u * NT) + c;
         if (m < mrows && o < O) {
             float s = 0.0f;
 #pragma unroll
@@ -242,15 +245,16 @@ struct RwCfg {
     uint32_t lds;
     void (*launch)(dim3, uint32_t, hipStream_t, hipEvent_t, hipEvent_t, const uint8_t *,
                    const float *, const uint16_t *, uint16_t *, uint32_t, uint32_t, uint32_t,
-                   const uint32_t *, uint32_t);
+                   const uint32_t *, uint32_t, uint32_t);
 };
 
 template <bool BF, int MR, int NT, int KS, int NA, int SL>
 static void rw_run(dim3 grid, uint32_t lds, hipStream_t st, hipEvent_t e0, hipEvent_t e1,
                    const uint8_t *w, const float *s, const uint16_t *x, uint16_t *y, uint32_t M,
-                   uint32_t O, uint32_t K, const uint32_t *exact, uint32_t tile0) {
+                   uint32_t O, uint32_t K, const uint32_t *exact, uint32_t blk0,
+                   uint32_t tile0) {
     GHIP_LAUNCH(e0, e1, (k_rows_gemm<BF, MR, NT, KS, NA, SL>), grid, dim3(RW_NW * 64), lds, st, w,
-                s, x, y, M, O, K, exact, tile0);
+                s, x, y, M, O, K, exact, blk0, tile0);
 }
 
 #define RW_CFG(BF, MR, NT, KS, NA, SL, T)                                                  \
@@ -340,16 +344,20 @@ extern "C" hipError_t ghip_launch_rows(int bf, const void *w, const float *scale
     if (!ghip_rows_fits(bf, M, N, K, w, x) || n_cu == 0) return hipErrorInvalidValue;
     float est = 0.0f;
     const RwCfg *c = rw_pick(bf != 0, M, N, K, n_cu, &est);
-    const size_t gpp = 16u * c->nt * (RW_NW / c->ks), tiles = (M + c->mr - 1) / c->mr;
-    /* a grid has at most 65535 row tiles: more rows take several launches */
-    for (size_t t0 = 0; t0 < tiles; t0 += RW_MAX_TILES) {
-        const size_t n = tiles - t0 < RW_MAX_TILES ? tiles - t0 : RW_MAX_TILES;
-        c->launch(dim3((uint32_t)((N + gpp - 1) / gpp), (uint32_t)n), c->lds, st,
-                  t0 == 0 ? e0 : nullptr, t0 + n == tiles ? e1 : nullptr, (const uint8_t *)w,
-                  scales, x, y, (uint32_t)M, (uint32_t)N, (uint32_t)K, exact_dev, (uint32_t)t0);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
+    const size_t gpp = 16u * c->nt * (RW_NW / c->ks), blocks = (N + gpp - 1) / gpp;
+    const size_t tiles = (M + c->mr - 1) / c->mr;
+    for (size_t t0 = 0; t0 < tiles; t0 += RW_MAX_TILES)
+        for (size_t b0 = 0; b0 < blocks; b0 += RW_MAX_BLOCKS) {
+            const size_t nt = tiles - t0 < RW_MAX_TILES ? tiles - t0 : RW_MAX_TILES;
+            const size_t nb = blocks - b0 < RW_MAX_BLOCKS ? blocks - b0 : RW_MAX_BLOCKS;
+            c->launch(dim3((uint32_t)nb, (uint32_t)nt), c->lds, st,
+                      t0 == 0 && b0 == 0 ? e0 : nullptr,
+                      t0 + nt == tiles && b0 + nb == blocks ? e1 : nullptr, (const uint8_t *)w,
+                      scales, x, y, (uint32_t)M, (uint32_t)N, (uint32_t)K, exact_dev,
+                      (uint32_t)b0, (uint32_t)t0);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
     return hipSuccess;
 }
 

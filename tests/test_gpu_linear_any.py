@@ -42,3 +42,19 @@ def test_any_bf16(ghip, M, N, K):
     floor = 2.0 ** -8 * (np.abs(O.bf16_to_f32(x)) @ np.abs(O.bf16_to_f32(w)).T)
     assert_close(got, O.gemm(w, x, threads=16), floor, "bf16 M%d N%d K%d" % (M, N, K))
     assert np.array_equal(got[-1:], run(x[-1:].copy()))
+
+
+def test_any_several_launches(ghip):
+    """More waves than one launch holds (2^32 threads): every output is
+    written. K = 1, so an output is one product."""
+    M, N = 65541, 8200
+    assert -(-M // 8) * N * 64 > 1 << 32
+    rng = np.random.default_rng(4)
+    w = O.f32_to_bf16(rng.uniform(-4, 4, (N, 1)).astype(np.float32))
+    x = O.f32_to_bf16(rng.uniform(-4, 4, (M, 1)).astype(np.float32))
+    dw, dx, dy = G.dev(w), G.dev(x), G.empty(2 * M * N)
+    assert ghip.apus_ghip_bf16_gemm_dev(G.vp(dw), G.vp(dx), G.vp(dy), M, N, 1, G.stream()) == 0
+    got = G.host(dy, np.uint16, (M, N))
+    for m in range(0, M, 4096):
+        want = O.f32_to_bf16(O.bf16_to_f32(x[m:m + 4096]) * O.bf16_to_f32(w).T + np.float32(0))
+        assert np.array_equal(got[m:m + 4096], want), m

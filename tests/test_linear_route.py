@@ -45,3 +45,17 @@ def test_fp8_other_shapes(pkg):
     assert fp8(pkg, 1, 512, 4095) == ANY and fp8(pkg, 300, 512, 4096, codes=off) == ANY
     assert fp8(pkg, 300, 512, 4096, x=off) == ANY and fp8(pkg, 300, 512, 4096, y=off) == ROWS
     assert fp8(pkg, 300, 512, 4096, ncu=0) == ANY
+
+
+@pytest.mark.parametrize("O,K", [(1, 128), (16384, 4096), (1 << 24, 4096), ((1 << 24) - 1, 4096), (1 << 25, 4096),
+                                 (1 << 32, 16), (9000000, 8191), (130, 1 << 29), (130, (1 << 29) + 8)])
+def test_dequant_launches_stay_under_the_thread_limit(pkg, O, K):
+    """The rows of one launch: whole scale blocks, 2^32 threads or more in
+    none (8 codes a thread, 512 chunks of 8 a workgroup of 256)."""
+    f = pkg.load().ghip_dequant_rows
+    f.restype, f.argtypes = ctypes.c_size_t, [ctypes.c_size_t] * 2
+    rows = f(O, K)
+    assert rows == O or rows % 128 == 0
+    assert (rows * K + 4095) // 4096 * 256 < 1 << 32
+    # as many as fit: twice the rows (or a block more) would not
+    assert rows == O or ((rows + 128) * K + 4095) // 4096 * 256 >= 1 << 32
