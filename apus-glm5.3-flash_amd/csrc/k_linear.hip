@@ -73,24 +73,40 @@ __global__ __launch_bounds__(256) void k_linear_any(
         return ghip_bf16_round(ghip_e4m3_exact(wr[k]) * srow[k >> 7]);
     };
     float acc[MR] = {};
-    for (uint32_t k0 = 0; k0 < K; k0 += 256u) {
-        float wv[4], xv[4][MR];
+    /* U steps of 64 from k0; END: the last of them ends at K, and a lane past
+     * it adds +0 */
+    auto steps = [&](auto u_c, auto end_c, uint32_t k0) {
+        constexpr int U = decltype(u_c)::value;
+        constexpr bool END = decltype(end_c)::value;
+        float wv[U], xv[U][MR];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint32_t k = k0 + 64u * j + lane, kc = min(k, K - 1u);
+        for (int j = 0; j < U; j++) {
+            const bool last = END && j == U - 1;
+            const uint32_t k = k0 + 64u * j + lane, kc = last ? min(k, K - 1u) : k;
             wv[j] = weight(kc);
+            if (last) wv[j] = k < K ? wv[j] : 0.0f;
 #pragma unroll
             for (int i = 0; i < MR; i++) {
-                /* past K a lane adds +0 */
                 const float v = ghip_bf16_f32(xr[i][kc]);
-                xv[j][i] = k < K ? v : 0.0f;
+                xv[j][i] = last && k >= K ? 0.0f : v;
             }
-            wv[j] = k < K ? wv[j] : 0.0f;
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < U; j++)
 #pragma unroll
             for (int i = 0; i < MR; i++) acc[i] += wv[j] * xv[j][i];
+    };
+    using ST = std::true_type;
+    using SF = std::false_type;
+    uint32_t k0 = 0;
+    for (; K - k0 > 256u; k0 += 256u) steps(std::integral_constant<int, 4>{}, SF{}, k0);
+    /* no more steps than K has: four for 1 of 257 cost up to a fifth (2000 x
+     * 257, M = 3, FP8: 5.5 us against 4.7) */
+    switch ((K - k0 + 63u) >> 6) {
+    case 4: steps(std::integral_constant<int, 4>{}, ST{}, k0); break;
+    case 3: steps(std::integral_constant<int, 3>{}, ST{}, k0); break;
+    case 2: steps(std::integral_constant<int, 2>{}, ST{}, k0); break;
+    default: steps(std::integral_constant<int, 1>{}, ST{}, k0); break;
     }
 #pragma unroll
     for (int i = 0; i < MR; i++) {

@@ -1,6 +1,7 @@
 """The shape-general linear (K no multiple of 128 or 64), which takes 1, 2, 4
-or 8 rows of x a wave: row remainders at each, K under one wave's step, ends of
-its steps of 256, and scale blocks crossed inside one; against the oracle to
+or 8 rows of x a wave: row remainders at each, K under one wave's step, one to
+four steps of 64 left after those of 256, full and partial, and scale blocks
+crossed inside one; against the oracle to
 the contract tolerance, and the same bits for a row whatever rows are beside
 it."""
 import numpy as np
@@ -14,7 +15,8 @@ from tolerance import assert_close
 pytestmark = pytest.mark.gpu
 
 SIZES = [(1, 5, 1), (1, 4097, 63), (2, 4100, 65), (3, 2050, 255), (4, 5000, 257), (7, 4099, 100),
-         (8, 4096, 191), (9, 2100, 449), (17, 1500, 330), (64, 700, 1025), (33, 64, 500)]
+         (8, 4096, 191), (9, 2100, 449), (17, 1500, 330), (64, 700, 1025), (33, 64, 500),
+         (3, 2000, 257), (5, 300, 447), (6, 300, 576 + 32), (2, 500, 1216 + 32)]
 
 
 @pytest.mark.parametrize("M,N,K", SIZES)
