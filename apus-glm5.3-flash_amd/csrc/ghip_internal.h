@@ -232,6 +232,8 @@ hipError_t ghip_launch_fp8_gemm(const uint8_t *codes, const float *scales,
                                 const uint16_t *x, uint16_t *y, size_t M, size_t N,
                                 size_t K, const uint32_t *exact_dev, uint32_t n_cu,
                                 const hipEvent_t *ev, hipStream_t st);
+/* Its estimated time in microseconds below 256 rows (the dispatch compares it). */
+float ghip_fp8_gemm_estimate(size_t M, size_t N, size_t K, uint32_t n_cu);
 
 /* One expert slab record of a converted v2 container's apus.index.json
  * (c/gcache.h:896-930): the shard file name and the slab's file offset. */

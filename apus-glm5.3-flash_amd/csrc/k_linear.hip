@@ -334,14 +334,6 @@ static hipError_t launch_gemv_m(const uint8_t *codes, const float *scales, const
 /* Rows of X from which the MFMA GEMM (N % 256 == 0) is considered. */
 #define GHIP_GEMM_MIN_M 16
 
-/* Estimated microseconds of ghip_launch_fp8_gemm below 256 rows (two
- * launches, K split): 11 + the weights at 6 TB/s + 0.04 a row. Measured q_a
- * 1536 x 4096 14.6 us at M = 64, o_proj 4096 x 16384 22.2 at 16 and 31.4 at
- * 128, q_b 16384 x 1536 20.5 at 96. */
-static float fp8_gemm_estimate(size_t M, size_t O, size_t K) {
-    return 11.0f + (float)((double)O * (double)K / 6.0e6) + 0.04f * (float)M;
-}
-
 /* The kernel of an FP8 linear on n_cu CUs. */
 extern "C" int ghip_fp8_linear_route(const void *codes, const void *x, const void *y, size_t M,
                                      size_t O, size_t K, uint32_t n_cu) {
@@ -352,9 +344,16 @@ extern "C" int ghip_fp8_linear_route(const void *codes, const void *x, const voi
      * against 6.2; below that many rows the streamed form is as good or
      * better, 7000 x 2048 4.9 against 6.0) */
     if (rows && M <= 4 && (O + 63) / 64 >= n_cu && M * K * 2 <= GS_X_MAX) return GHIP_ROUTE_GEMV;
-    if (n_cu && M >= GHIP_GEMM_MIN_M && ghip_fp8_gemm_fits(M, O, K, codes, x, y)
-        && (M >= 256 || !rows || fp8_gemm_estimate(M, O, K) < ghip_rows_estimate(0, M, O, K, n_cu)))
-        return GHIP_ROUTE_GEMM;
+    /* below 256 rows whichever is estimated faster, the GEMM where they are
+     * within 6% (8192 x 128, M = 100: rows 6.6 us, GEMM 4.6; 1536 x 4096, M =
+     * 64: rows 7.7, GEMM 16.5) */
+    if (n_cu && n_cu % 8 == 0 && M >= GHIP_GEMM_MIN_M
+        && ghip_fp8_gemm_fits(M, O, K, codes, x, y)) {
+        if (M >= 256 || !rows) return GHIP_ROUTE_GEMM;
+        /* no GEMM is estimated under 4.4 us: the smallest calls skip its plan */
+        const float r = 1.06f * ghip_rows_estimate(0, M, O, K, n_cu);
+        if (r > 4.4f && ghip_fp8_gemm_estimate(M, O, K, n_cu) < r) return GHIP_ROUTE_GEMM;
+    }
     return rows ? GHIP_ROUTE_ROWS : GHIP_ROUTE_ANY;
 }
 

@@ -1563,13 +1563,14 @@ static float *g_part;
 static size_t g_part_cap;
 #define GHIP_SPLITK_MAX_BYTES ((size_t)256 << 20)
 
-extern "C" hipError_t ghip_launch_fp8_gemm(const uint8_t *codes, const float *scales,
-                                           const uint16_t *x, uint16_t *y, size_t M,
-                                           size_t N, size_t K, const uint32_t *exact_dev,
-                                           uint32_t n_cu, const hipEvent_t *ev,
-                                           hipStream_t st) {
-    if (!ghip_fp8_gemm_fits(M, N, K, codes, x, y) || n_cu == 0 || n_cu % 8)
-        return hipErrorInvalidValue;
+/* How the launch divides M x N x K: tile height, K splits, XCD grid R x
+ * (8 / R), workgroups. */
+struct F8Plan {
+    uint32_t bm, S, R, grid;
+};
+
+/* (no loop over splits: the dispatch asks at every call of a few rows) */
+static F8Plan f8_plan(size_t M, size_t N, size_t K, uint32_t n_cu) {
     const size_t nblk = N / 256, nkb = K / 128;
     /* Tile height bm and K splits S: among bm in {256, 128, 64, 32} (no
      * taller than M needs) with the fewest splits that give 3/4 of the CUs
@@ -1579,7 +1580,8 @@ extern "C" hipError_t ghip_launch_fp8_gemm(const uint8_t *codes, const float *sc
      * blocks each. When no choice reaches 3/4 of the CUs, the one with the
      * most items. */
     const size_t want = (size_t)n_cu * 3 / 4;
-    uint32_t bm = 32, S = 1;
+    const size_t most = GHIP_SPLITK_MAX_BYTES / (M * N * sizeof(float));
+    F8Plan p = {32, 1, 0, 0};
     size_t items = 0;
     {
         double best = -1.0;
@@ -1588,10 +1590,10 @@ extern "C" hipError_t ghip_launch_fp8_gemm(const uint8_t *codes, const float *sc
         for (uint32_t b = PF_BM; b >= 32; b >>= 1) {
             if (b > 32 && b / 2 >= M) continue;
             const size_t tiles = (M + b - 1) / b, base = tiles * nblk;
-            size_t sp = 1;
-            while (base * sp < want && sp + 1 <= nkb / 2
-                   && (sp + 1) * M * N * sizeof(float) <= GHIP_SPLITK_MAX_BYTES)
-                sp++;
+            size_t sp = (want + base - 1) / base;
+            if (sp > nkb / 2) sp = nkb / 2;
+            if (sp > most) sp = most;
+            if (sp < 1) sp = 1;
             const size_t it = base * sp;
             const bool ok = it >= want;
             const double bytes = (double)nblk * tiles * b * K * 2 + (double)tiles * N * K
@@ -1602,14 +1604,71 @@ extern "C" hipError_t ghip_launch_fp8_gemm(const uint8_t *codes, const float *sc
                 best = bytes;
                 best_items = it;
                 best_ok = ok;
-                bm = b;
-                S = (uint32_t)sp;
+                p.bm = b;
+                p.S = (uint32_t)sp;
             }
         }
         items = best_items;
     }
-    if (S > 1) {
-        const size_t need = (size_t)S * M * N * sizeof(float);
+    /* XCD grid R x (8/R): fewest bytes into the 8 L2s, (8/R) |X| + R |W|,
+     * among the grids that give every XCD the same number of units and of
+     * column blocks (an uneven split would leave XCDs idle at the end) */
+    {
+        const size_t rows_u = ((M + p.bm - 1) / p.bm) * p.S;
+        const double xb = (double)((M + p.bm - 1) / p.bm) * p.bm * K * 2, wb = (double)N * K;
+        double best = -1.0;
+        for (uint32_t r = 1; r <= 8; r <<= 1) {
+            if (rows_u % r || nblk % (8 / r)) continue;
+            const double b = (8.0 / r) * xb + r * wb;
+            if (best < 0.0 || b < best) {
+                best = b;
+                p.R = r;
+            }
+        }
+        if (!p.R) p.R = nblk >= 8 ? 1u : 8u;    /* no even grid: whole column blocks
+                                                   or whole units per XCD */
+    }
+    p.grid = items < n_cu ? (uint32_t)((items + 7) & ~(size_t)7) : n_cu;
+    return p;
+}
+
+/* Estimated microseconds at fewer than 256 rows: rounds of the busiest XCD's
+ * workgroups, each an item's fill and store and its k blocks (f8_cost, by tile
+ * height 32, 64, 128, 256), the weights, and with splits a second launch that
+ * reads S partial sums in turn. Fitted to 1968 shapes, M = 16..255, N =
+ * 256..32768, K = 128..16384, operands from HBM: within 10% at nine of ten
+ * (16384 x 128, M = 100: 5.2 us; 1536 x 4096, M = 64 16.5; 4096 x 16384, M =
+ * 128 35). */
+static const struct {
+    double item[4], block[4];
+} f8_cost[2] = {{{0.86, 3.14, 5.72, 5.72}, {1.515, 1.23, 1.44, 1.98}},   /* S == 1 */
+                {{1.18, 3.72, 3.25, 3.02}, {1.19, 0.94, 1.08, 1.98}}};   /* S > 1 */
+
+extern "C" float ghip_fp8_gemm_estimate(size_t M, size_t N, size_t K, uint32_t n_cu) {
+    const F8Plan p = f8_plan(M, N, K, n_cu);
+    const uint32_t nblk = (uint32_t)(N / 256), C = 8u / p.R;
+    const uint32_t ru = (uint32_t)((M + p.bm - 1) / p.bm) * p.S;
+    /* XCD 0 has the most units and column blocks */
+    const uint32_t n = (ru + p.R - 1) / p.R * ((nblk + C - 1) / C), per = p.grid / 8u;
+    const double rounds = (double)((n + per - 1) / per);
+    const int h = p.bm > 128 ? 3 : p.bm > 64 ? 2 : p.bm > 32 ? 1 : 0;
+    const double kb = (double)((K / 128 + p.S - 1) / p.S), w = (double)N * (double)K * 1e-6;
+    const double t = rounds * (f8_cost[p.S > 1].item[h] + kb * f8_cost[p.S > 1].block[h]);
+    if (p.S == 1) return (float)(2.0 + t + 0.1 * w);
+    return (float)(4.54 + t + 0.051 * w + 0.188 * p.S
+                   + 1.68e-6 * p.S * (double)M * (double)N);
+}
+
+extern "C" hipError_t ghip_launch_fp8_gemm(const uint8_t *codes, const float *scales,
+                                           const uint16_t *x, uint16_t *y, size_t M,
+                                           size_t N, size_t K, const uint32_t *exact_dev,
+                                           uint32_t n_cu, const hipEvent_t *ev,
+                                           hipStream_t st) {
+    if (!ghip_fp8_gemm_fits(M, N, K, codes, x, y) || n_cu == 0 || n_cu % 8)
+        return hipErrorInvalidValue;
+    const F8Plan p = f8_plan(M, N, K, n_cu);
+    if (p.S > 1) {
+        const size_t need = (size_t)p.S * M * N * sizeof(float);
         if (need > g_part_cap) {
             if (g_part) (void)hipFree(g_part);
             g_part = nullptr;
@@ -1619,35 +1678,15 @@ extern "C" hipError_t ghip_launch_fp8_gemm(const uint8_t *codes, const float *sc
             g_part_cap = need;
         }
     }
-    /* XCD grid R x (8/R): fewest bytes into the 8 L2s, (8/R) |X| + R |W|,
-     * among the grids that give every XCD the same number of units and of
-     * column blocks (an uneven split would leave XCDs idle at the end) */
-    uint32_t R = 0;
-    {
-        const size_t rows_u = ((M + bm - 1) / bm) * S;
-        const double xb = (double)((M + bm - 1) / bm) * bm * K * 2, wb = (double)N * K;
-        double best = -1.0;
-        for (uint32_t r = 1; r <= 8; r <<= 1) {
-            if (rows_u % r || nblk % (8 / r)) continue;
-            const double b = (8.0 / r) * xb + r * wb;
-            if (best < 0.0 || b < best) {
-                best = b;
-                R = r;
-            }
-        }
-        if (!R) R = nblk >= 8 ? 1u : 8u;    /* no even grid: whole column blocks
-                                                or whole units per XCD */
-    }
-    uint32_t g = items < n_cu ? (uint32_t)((items + 7) & ~(size_t)7) : n_cu;
     hipEvent_t e0 = ev ? ev[0] : nullptr, e1 = ev ? ev[1] : nullptr;
-    GHIP_LAUNCH(e0, S > 1 ? nullptr : e1, k_fp8_gemm, dim3(g), dim3(256), PF_LDS, st, codes,
-                scales, x, y, g_part, (uint32_t)M, (uint32_t)N, (uint32_t)K, bm, S, R,
+    GHIP_LAUNCH(e0, p.S > 1 ? nullptr : e1, k_fp8_gemm, dim3(p.grid), dim3(256), PF_LDS, st, codes,
+                scales, x, y, g_part, (uint32_t)M, (uint32_t)N, (uint32_t)K, p.bm, p.S, p.R,
                 exact_dev);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess || S == 1) return e;
+    if (e != hipSuccess || p.S == 1) return e;
     const size_t n = M * N;                          /* N % 256 == 0: n % 4 == 0 */
     GHIP_LAUNCH(nullptr, e1, k_splitk_sum, dim3((uint32_t)((n / 4 + 255) / 256)), dim3(256),
-                0, st, g_part, S, n, y);
+                0, st, g_part, p.S, n, y);
     return hipGetLastError();
 }
 

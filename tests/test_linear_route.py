@@ -59,3 +59,15 @@ def test_dequant_launches_stay_under_the_thread_limit(pkg, O, K):
     assert (rows * K + 4095) // 4096 * 256 < 1 << 32
     # as many as fit: twice the rows (or a block more) would not
     assert rows == O or ((rows + 128) * K + 4095) // 4096 * 256 >= 1 << 32
+
+
+# (M, N, K), the faster kernel, by a tenth or more (measured on 256 CUs)
+FEW = [(100, 8192, 128, GEMM), (255, 12288, 128, GEMM), (160, 12288, 512, GEMM), (96, 16384, 256, GEMM),
+       (64, 32768, 256, GEMM), (255, 8192, 768, GEMM), (128, 16384, 1536, GEMM), (17, 32768, 128, GEMM),
+       (16, 16384, 1536, ROWS), (64, 1536, 4096, ROWS), (129, 1536, 4096, ROWS), (64, 512, 4096, ROWS),
+       (32, 16384, 4096, ROWS), (48, 2048, 2048, ROWS)]
+
+
+@pytest.mark.parametrize("M,N,K,want", FEW)
+def test_fp8_few_rows_take_the_faster_kernel(pkg, M, N, K, want):
+    assert fp8(pkg, M, N, K) == want
