@@ -164,8 +164,11 @@ hipError_t ghip_launch_moe_router(const uint16_t *x, const uint16_t *gate_w,
 #define PF_HDR_NTILES 0
 #define PF_HDR_NPAIRS 1
 #define PF_HDR_ERR 2
+#define PF_HDR_LONG 3         /* 1: a tile has more than PF_LONG_ROWS rows */
 #define PF_HDR_Q 16           /* 2 x 8 item-queue counters (GEMM, XCD) */
 #define PF_HDR_WORDS 32
+#define PF_BM 256             /* most rows of a tile */
+#define PF_LONG_ROWS 32       /* rows of an item of the weight streams */
 typedef struct {
     uint32_t *hdr;        /* PF_HDR_WORDS u32: tiles, kept pairs, error,
                              the GEMMs' per-XCD item counters; zeroed per call */
@@ -209,16 +212,23 @@ hipError_t ghip_launch_moe_prefill(const GhipBank *bank, const uint16_t *x,
                                    const GhipMoePrefillWs *ws,
                                    const hipEvent_t *ev, hipStream_t st);
 
+/* Which products a prefill of T tokens x topk slots over n_experts takes (the
+ * shared expert counted in both; host only, no device needed). */
+enum { GHIP_MOE_QUEUED, GHIP_MOE_FULL, GHIP_MOE_ROWS };
+int ghip_moe_prefill_form(uint32_t dim, uint32_t inter, uint32_t n_experts, uint32_t topk,
+                          size_t T);
+
 /* The products of a prefill whose tiles mostly hold a few rows: mode 0 gate/up
  * + SwiGLU (act = x, rows gathered by perm[s] / topk; out = H), mode 1 down
  * (act = H, out = O), over the tile list of the permutation. e0/e1: NULL or
  * timing events. fits: whether its 32-bit offsets hold T tokens, P pairs. */
-int ghip_moe_rows_fits(const GhipBank *bank, size_t T, size_t P);
+int ghip_moe_rows_fits(uint32_t dim, uint32_t inter, size_t T, size_t P);
 hipError_t ghip_launch_moe_rows(int mode, const GhipBank *bank, const uint16_t *act,
                                 const int32_t *perm, const uint32_t *tiles,
                                 const uint32_t *hdr, uint32_t topk, float limit,
                                 uint16_t *out, uint32_t n_cu, hipEvent_t e0,
                                 hipEvent_t e1, hipStream_t st);
+hipError_t ghip_moe_rows_init(void);
 
 /* Dense FP8-block GEMM on MFMA (the prefill tile body): Y [M, N] =
  * bf16(X [M, K] . dequant(W [N, K])^T). Shapes it takes: N % 256 == 0,

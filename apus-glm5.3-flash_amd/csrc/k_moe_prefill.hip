@@ -55,7 +55,6 @@
 typedef float ghip_f32x16 __attribute__((ext_vector_type(16)));
 
 #define PF_CHUNK 1024            /* pairs per permutation workgroup */
-#define PF_BM 256                /* rows per GEMM tile */
 #define PF_RB (PF_BM / 32)       /* 32-row MFMA blocks per tile */
 #define PF_BK 64                 /* k per pipeline stage */
 #define PF_A_STAGE (PF_BM * PF_BK * 2)          /* 32 KB activation tile */
@@ -183,6 +182,7 @@ __global__ __launch_bounds__(1024) void k_pf_scan(
             const uint32_t rows = tot - r0 < PF_BM ? tot - r0 : PF_BM;
             tiles[tb + i] = make_uint4(e, base + r0, rows, nanf);
         }
+        if (tot > PF_LONG_ROWS) hdr[PF_HDR_LONG] = 1u;
     }
     if (e == 1023) {
         hdr[PF_HDR_NTILES] = tb + nt;
@@ -236,11 +236,11 @@ __global__ __launch_bounds__(1024) void k_pf_permute(
     int32_t *__restrict__ perm, int32_t *__restrict__ pos, uint32_t *__restrict__ hdr,
     uint32_t *__restrict__ serr) {
     extern __shared__ uint32_t pm[];                    /* starts [Ep], counts [16][Ep] */
-    __shared__ uint32_t sh[16], bad;
+    __shared__ uint32_t sh[16], bad, lng;
     const uint32_t Ep = E + (topk_p - topk), tid = threadIdx.x, w = tid >> 6, lane = tid & 63u;
     uint32_t *start = pm, *wcnt = pm + Ep;
     for (uint32_t i = tid; i < 16u * Ep; i += 1024u) wcnt[i] = 0;
-    if (tid == 0) bad = 0;
+    if (tid == 0) bad = lng = 0;
     __syncthreads();
     /* ids as k_pf_count takes them: out of range flagged and dropped, a
      * repeat of an earlier slot of the token dropped */
@@ -284,19 +284,20 @@ __global__ __launch_bounds__(1024) void k_pf_permute(
     if (tid < Ep) {
         const uint32_t nanf = (nan_flags && nan_flags[tid] ? 1u : 0u) | (nt > 1u ? 2u : 0u);
         start[tid] = base;
+        if (tot > PF_LONG_ROWS) lng = 1;
         for (uint32_t i = 0; i < nt; i++) {
             const uint32_t r0 = i * PF_BM;
             tiles[tb + i] = make_uint4(tid, base + r0, tot - r0 < PF_BM ? tot - r0 : PF_BM, nanf);
         }
     }
+    __syncthreads();
     if (tid < PF_HDR_WORDS && tid != PF_HDR_NTILES && tid != PF_HDR_NPAIRS)
-        hdr[tid] = tid == PF_HDR_ERR ? bad : 0u;
+        hdr[tid] = tid == PF_HDR_ERR ? bad : tid == PF_HDR_LONG ? lng : 0u;
     if (tid == 1023) {
         hdr[PF_HDR_NTILES] = tb + nt;
         hdr[PF_HDR_NPAIRS] = base + tot;
     }
     if (tid == 0 && bad && serr) atomicOr(serr, 2u);
-    __syncthreads();
     if (e >= 0) {
         for (uint32_t v = 0; v < w; v++) rank += wcnt[v * Ep + e];
         const uint32_t s = start[e] + rank;
@@ -1453,6 +1454,28 @@ extern "C" size_t ghip_moe_prefill_chunks(size_t pairs) {
     return (pairs + PF_CHUNK - 1) / PF_CHUNK;
 }
 
+/* Tiles mostly full (on average at least half a 256-row tile per expert): the
+ * static full-tile form. Few rows an expert (on average 7/8, or little work in
+ * all): weight streams in small items, which the tile form's 1 MB items and
+ * long launches cannot match (288 experts of 4096/2048, top-8: T = 16 399
+ * against 426 us, T = 32 662 against 666, T = 36 731 against 725; 64 of
+ * 2048/1024, 6 + shared: T = 32, 2.8 GFLOP, 87 against 102 us, T = 64, 5.6
+ * GFLOP, 118 against 114). The streams read an expert's weights again for
+ * every 16 rows, which must not cost more where all tokens choose the same
+ * experts: at most 18 experts' weights then (top-8, all alike: T = 32, 16 of
+ * them, 88 against 91 us, T = 33, 24 of them, 123 against 92). Else the queued
+ * form. */
+extern "C" int ghip_moe_prefill_form(uint32_t dim, uint32_t inter, uint32_t n_experts,
+                                     uint32_t topk, size_t T) {
+    const size_t P = T * topk;
+    if (P >= (size_t)n_experts * (PF_BM / 2)) return GHIP_MOE_FULL;
+    if (ghip_moe_rows_fits(dim, inter, T, P)
+        && ((8 * P <= 7 * (size_t)n_experts && topk * ((T + 15) / 16) <= 18)
+            || 6.0 * (double)P * dim * inter <= 3e9))
+        return GHIP_MOE_ROWS;
+    return GHIP_MOE_QUEUED;
+}
+
 extern "C" hipError_t ghip_launch_moe_prefill(const GhipBank *bank,
                                               const uint16_t *x, size_t T,
                                               const int32_t *idx, const float *w,
@@ -1507,24 +1530,14 @@ extern "C" hipError_t ghip_launch_moe_prefill(const GhipBank *bank,
     const size_t lds = PF_LDS, lds8 = PF_LDS_WB;
     (void)mt;
     const uint32_t g0 = ws->n_cu, g1 = ws->n_cu;
-    /* Which products. Tiles mostly full (on average at least half a 256-row
-     * tile per expert): the static full-tile form. Few rows an expert (on
-     * average at most one, or little work in all): weight streams in small
-     * items, which the tile form's 1 MB items and long launches cannot match
-     * (288 experts of 4096/2048, top-8: T = 12 351 against 364 us, T = 32
-     * 698 against 691, T = 64 1000 against 979; 64 of 2048/1024, 6 + shared:
-     * T = 32, 2.8 GFLOP, 87 against 102 us, T = 64, 5.6 GFLOP, 118 against
-     * 114). Else the queued form. */
-    const bool full = P >= (size_t)Ep * (PF_BM / 2);
-    const bool few = !full && ghip_moe_rows_fits(bank, T, P)
-                  && (P <= Ep || 6.0 * (double)P * dim * inter <= 3e9);
-    if (few) {
+    const int form = ghip_moe_prefill_form(dim, inter, Ep, topk_p, T);
+    if (form == GHIP_MOE_ROWS) {
         if ((e = ghip_launch_moe_rows(0, bank, x, ws->perm, ws->tiles, ws->hdr, topk_p, limit,
                                       ws->h, ws->n_cu, e2, e3, st)) != hipSuccess
             || (e = ghip_launch_moe_rows(1, bank, ws->h, ws->perm, ws->tiles, ws->hdr, topk_p,
                                          limit, ws->o, ws->n_cu, e4, e5, st)) != hipSuccess)
             return e;
-    } else if (full) {
+    } else if (form == GHIP_MOE_FULL) {
         GHIP_LAUNCH(e2, e3, (k_pf_gemm<0, true>), dim3(g0), dim3(512), lds8, st, *bank,
                     x, ws->perm, (const uint4 *)ws->tiles, ws->hdr, inter / 128,
                     topk_p, limit, ws->h);
@@ -1764,5 +1777,5 @@ extern "C" hipError_t ghip_moe_prefill_init(void) {
                                            lds[i]);
         if (e != hipSuccess) return e;
     }
-    return hipSuccess;
+    return ghip_moe_rows_init();
 }

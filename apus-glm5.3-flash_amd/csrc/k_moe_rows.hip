@@ -3,15 +3,16 @@
  * SwiGLU and down products of expert tiles that mostly hold a few rows, as
  * weight streams (c/gmoe.h:210-227 per token in the reference).
  *
- * An item is one tile of the expert-sorted rows (k_moe_prefill.hip) against
+ * An item is rows of one tile of the expert-sorted rows (k_moe_prefill.hip) against
  * 16 gate and the same 16 up rows (MODE 0) or 64 down rows (MODE 1), 128 KB of
  * weights at dim 4096 / inter 2048. The 8 waves split K (8 ways, or 4 ways
  * over two groups of 32 down rows); a wave loads 128-wide k blocks of its 32
  * weight rows with that part of 16 activation rows (gathered by token in MODE
  * 0) into registers, passes both through a wave-private LDS area into the
  * layout of v_mfma_f32_16x16x32_bf16 and dequantizes each code once. The
- * partial sums meet in LDS in a fixed order. A tile of more rows takes its
- * item in passes of 16 (the weights come from L2 again).
+ * partial sums meet in LDS in a fixed order. An item takes up to 32 rows, in
+ * passes of 16 (the weights come from L2 again); a tile's further rows are
+ * items of their own.
  *
  * HBM bounds it: 6.2-6.3 TB/s at T = 12, top-8 of 288 (1.39 GB of gate/up in
  * 224 us, 0.69 GB of down in 110). Two workgroups a CU (64 KB of LDS, 128
@@ -26,6 +27,8 @@
 #define MR_NW 8
 #define MR_SLOT (4096u + 4096u)  /* x of 16 rows, two weight chunks */
 #define MR_LDS (MR_NW * MR_SLOT)
+#define MR_SUB ((uint32_t)PF_LONG_ROWS)  /* rows of an item */
+#define MR_LONG 512u             /* most tiles of more rows */
 
 /* One item for `rows` (1..16) sorted rows from row0. */
 template <int MODE, bool EXACT>
@@ -136,20 +139,55 @@ __device__ __forceinline__ void mr_body(const GhipBank &bank, const uint16_t *__
     __syncthreads();
 }
 
-/* Persistent: items of one size, dealt round-robin to two workgroups a CU. */
+/* Persistent, two workgroups a CU, items dealt round-robin. An item is MR_SUB
+ * rows at most: a tile's rows past that are items of their own, after the
+ * others', from a list of the longer tiles that every workgroup makes (so one
+ * expert with most of the rows keeps all CUs busy and not a few with 16
+ * passes each: 128 experts of 512/256, top-2, Zipf 1.1, T = 600 93 -> 51 us,
+ * T = 1500 110 -> 67; parts of 64 rows 58 and 73). An
+ * item's parts keep its column block, hence its XCD where nblk % 8 == 0. */
 template <int MODE>
 __global__ __launch_bounds__(MR_NW * 64, 4) void k_moe_rows(
     GhipBank bank, const uint16_t *__restrict__ act, const int32_t *__restrict__ perm,
     const uint4 *__restrict__ tiles, const uint32_t *__restrict__ hdr, uint32_t topk, float limit,
     uint16_t *__restrict__ out) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t mr_lds[];
+    uint16_t *longer = (uint16_t *)(mr_lds + MR_LDS);    /* tiles of more than MR_SUB rows */
     const uint32_t nblk = MODE == 0 ? bank.inter / 16u : bank.dim / 64u;
-    const uint32_t items = hdr[PF_HDR_NTILES] * nblk;
-    for (uint32_t it = blockIdx.x; it < items; it += gridDim.x) {
-        const uint32_t ti = it / nblk, nb = it - ti * nblk;
+    const uint32_t ntiles = hdr[PF_HDR_NTILES], items = ntiles * nblk;
+    uint32_t nlong = 0;
+    if (hdr[PF_HDR_LONG]) {
+        uint32_t *cnt = (uint32_t *)mr_lds;
+        const uint32_t tid = threadIdx.x, w = tid >> 6;
+        for (uint32_t t0 = 0; t0 < ntiles; t0 += MR_NW * 64u) {
+            const bool is = t0 + tid < ntiles && tiles[t0 + tid].z > MR_SUB;
+            const uint64_t m = __ballot(is);
+            if ((tid & 63u) == 0) cnt[w] = __popcll(m);
+            __syncthreads();
+            uint32_t at = nlong + __popcll(m & ((1ull << (tid & 63u)) - 1ull));
+            for (uint32_t v = 0; v < MR_NW; v++) {
+                if (v < w) at += cnt[v];
+                nlong += cnt[v];
+            }
+            if (is && at < MR_LONG) longer[at] = (uint16_t)(t0 + tid);
+            __syncthreads();
+        }
+        nlong = __builtin_amdgcn_readfirstlane(min(nlong, MR_LONG));
+    }
+    const uint32_t total = items + nlong * nblk * (PF_BM / MR_SUB - 1u);
+    for (uint32_t it = blockIdx.x; it < total; it += gridDim.x) {
+        uint32_t ti = it / nblk, from = 0;
+        const uint32_t nb = it - ti * nblk;
+        if (it >= items) {
+            const uint32_t j = ti - ntiles;              /* q-major: part 1 of every tile first */
+            const uint32_t q = j / nlong;
+            ti = __builtin_amdgcn_readfirstlane(longer[j - q * nlong]);
+            from = (q + 1u) * MR_SUB;
+        }
         const uint4 td = tiles[ti];
-        for (uint32_t m0 = 0; m0 < td.z; m0 += 16u) {
-            const uint32_t rows = min(td.z - m0, 16u), r0 = td.y + m0;
+        const uint32_t end = min(td.z, from + MR_SUB);
+        for (uint32_t m0 = from; m0 < end; m0 += 16u) {
+            const uint32_t rows = min(end - m0, 16u), r0 = td.y + m0;
             if (td.w & 1u)
                 mr_body<MODE, true>(bank, act, perm, td.x, r0, rows, nb, topk, limit, out, mr_lds);
             else
@@ -158,10 +196,10 @@ __global__ __launch_bounds__(MR_NW * 64, 4) void k_moe_rows(
     }
 }
 
-/* 32-bit activation offsets */
-extern "C" int ghip_moe_rows_fits(const GhipBank *bank, size_t T, size_t P) {
-    return bank->dim % 128 == 0 && bank->inter % 128 == 0 && T * bank->dim * 2 <= 0xffffffffull
-        && P * bank->inter * 2 <= 0xffffffffull;
+/* 32-bit activation offsets, and MR_LONG tiles of over MR_SUB rows at most */
+extern "C" int ghip_moe_rows_fits(uint32_t dim, uint32_t inter, size_t T, size_t P) {
+    return dim % 128 == 0 && inter % 128 == 0 && P <= (size_t)MR_LONG * MR_SUB
+        && T * dim * 2 <= 0xffffffffull && P * inter * 2 <= 0xffffffffull;
 }
 
 extern "C" hipError_t ghip_launch_moe_rows(int mode, const GhipBank *bank, const uint16_t *act,
@@ -174,10 +212,20 @@ extern "C" hipError_t ghip_launch_moe_rows(int mode, const GhipBank *bank, const
         return hipErrorInvalidValue;
     const dim3 grid(2u * n_cu), blk(MR_NW * 64);
     if (mode == 0)
-        GHIP_LAUNCH(e0, e1, k_moe_rows<0>, grid, blk, MR_LDS, st, *bank, act, perm,
+        GHIP_LAUNCH(e0, e1, k_moe_rows<0>, grid, blk, MR_LDS + MR_LONG * 2u, st, *bank, act, perm,
                     (const uint4 *)tiles, hdr, topk, limit, out);
     else
-        GHIP_LAUNCH(e0, e1, k_moe_rows<1>, grid, blk, MR_LDS, st, *bank, act, perm,
+        GHIP_LAUNCH(e0, e1, k_moe_rows<1>, grid, blk, MR_LDS + MR_LONG * 2u, st, *bank, act, perm,
                     (const uint4 *)tiles, hdr, topk, limit, out);
     return hipGetLastError();
+}
+
+extern "C" hipError_t ghip_moe_rows_init(void) {
+    const void *ks[2] = {(const void *)k_moe_rows<0>, (const void *)k_moe_rows<1>};
+    for (int i = 0; i < 2; i++) {
+        hipError_t e = hipFuncSetAttribute(ks[i], hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           MR_LDS + MR_LONG * 2);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }

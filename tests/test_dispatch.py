@@ -1,5 +1,6 @@
-"""Which kernel a linear takes (csrc/k_linear.hip), asked of the library's own
-dispatch: host code, so no device and no buffers of these sizes are needed."""
+"""Which kernel a linear or a prefill takes (csrc/k_linear.hip,
+csrc/k_moe_prefill.hip), asked of the library's own dispatch: host code, so no
+device and no buffers of these sizes are needed."""
 import ctypes
 
 import pytest
@@ -71,3 +72,19 @@ FEW = [(100, 8192, 128, GEMM), (255, 12288, 128, GEMM), (160, 12288, 512, GEMM),
 @pytest.mark.parametrize("M,N,K,want", FEW)
 def test_fp8_few_rows_take_the_faster_kernel(pkg, M, N, K, want):
     assert fp8(pkg, M, N, K) == want
+
+
+QUEUED, FULL, STREAMS = range(3)
+
+
+@pytest.mark.parametrize("dim,inter,experts,k,T,want", [
+    (4096, 2048, 288, 8, 12, STREAMS), (4096, 2048, 288, 8, 31, STREAMS), (4096, 2048, 289, 9, 28, STREAMS),
+    (4096, 2048, 288, 8, 64, QUEUED),
+    (4096, 2048, 288, 8, 4608, FULL), (64 * 32, 1024, 65, 7, 32, STREAMS), (512, 256, 128, 2, 1500, STREAMS),
+    # about one row an expert on average; the second: half a row, but 20 experts' weights where all tokens
+    # choose the same ones
+    (4096, 2048, 288, 8, 36, QUEUED), (4096, 2048, 600, 4, 75, QUEUED), (4096, 2048, 289, 9, 32, QUEUED)])
+def test_prefill_form(pkg, dim, inter, experts, k, T, want):
+    f = pkg.load().ghip_moe_prefill_form
+    f.argtypes = [ctypes.c_uint32] * 4 + [ctypes.c_size_t]
+    assert f(dim, inter, experts, k, T) == want

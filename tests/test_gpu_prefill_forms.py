@@ -3,7 +3,11 @@ csrc/k_moe_rows.hip) at the row counts where each can go wrong, every output
 against the oracle's per-token loop (tests/tolerance.py): the weight streams
 of few rows, the queued tile form's bodies (streams up to 16 rows, k split
 between the wave halves up to 128, row halves above), the one-launch
-permutation and its limits, and experts with NaN codes in each."""
+permutation and its limits, and experts with NaN codes in each. The form is
+asked of the library's own rule, so that a case that no longer reaches what it
+is for fails."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -16,8 +20,24 @@ from test_gpu_prefill import floor_of, prefill
 pytestmark = pytest.mark.gpu
 
 
+QUEUED, FULL, ROWS = range(3)
+
+
+def form(ghip, dim, inter, E, k, T):
+    return ghip.ghip_moe_prefill_form(dim, inter, E, k, ctypes.c_size_t(T))
+
+
 def routing_of(rows, rng):
-    """[T, k] ids that give expert e rows[e] rows (the rest repeats, dropped)."""
+    """[T, k] ids that give expert e rows[e] rows (the rest repeats, dropped).
+    Experts past 16 spread their rows over the tokens with the fewest."""
+    if len([r for r in rows if r]) > 16:
+        T = max(max(rows), sum(rows) // 12)
+        mine = [[] for _ in range(T)]
+        for e in sorted(range(len(rows)), key=lambda e: -rows[e]):
+            for t in sorted(range(T), key=lambda t: len(mine[t]))[:rows[e]]:
+                mine[t].append(e)
+        k = max(len(m) for m in mine)
+        return np.array([list(rng.permutation(m)) + [m[0]] * (k - len(m)) for m in mine], np.int32)
     T, k = max(rows), max(1, max(sum(r > t for r in rows) for t in range(max(rows))))
     idx = np.empty((T, k), np.int32)
     for t in range(T):
@@ -36,7 +56,7 @@ def floor(slabs, dim, inter, x, idx, w, eo):
                       O.moe_expert_floor(slabs, dim, inter, x, idx, w, threads=16))
 
 
-def check(ghip, dim, inter, rows, nan):
+def check(ghip, dim, inter, rows, nan, want_form):
     """One store and routing; k <= 16 slots a token."""
     E = len(rows)
     rng = np.random.default_rng(sum(rows) + dim)
@@ -47,7 +67,7 @@ def check(ghip, dim, inter, rows, nan):
             assert ghip.apus_ghip_store_put(s, e, O.ptr(sl), sl.nbytes) == 0
         idx = routing_of(rows, rng)
         T, k = idx.shape
-        assert k <= 16
+        assert k <= 16 and form(ghip, dim, inter, E, k, T) == want_form
         w = rng.uniform(0.02, 0.6, (T, k)).astype(np.float32)
         x = O.f32_to_bf16((rng.standard_normal((T, dim)) *
                            rng.uniform(0.5, 4.0, (T, 1))).astype(np.float32))
@@ -61,10 +81,14 @@ def check(ghip, dim, inter, rows, nan):
 
 @pytest.mark.parametrize("dim,inter,rows", [
     (256, 128, [1]), (512, 384, [1, 15, 16, 17, 0, 31, 32, 33, 48]),
-    (256, 256, [260, 3, 0, 16]), (1024, 128, [5] * 16)])
+    # parts of 32 rows: tiles of up to 256 rows and two tiles of an expert
+    (256, 256, [260, 3, 0, 16] + [0] * 8), (256, 128, [256, 64, 65, 255, 33, 32, 1, 95, 96, 97, 0, 300] + [0] * 16),
+    # every tile longer than one part, and longer ones past the 512th tile
+    (256, 128, [33] * 16), (256, 128, [1] * 600 + [70, 0, 2, 40]),
+    (1024, 128, [5] * 16)])
 def test_prefill_streams(ghip, dim, inter, rows):
     """Little work: the weight streams, in passes of 16 rows."""
-    check(ghip, dim, inter, rows, nan=(len(rows) - 1,))
+    check(ghip, dim, inter, rows, nan=(len(rows) - 1,), want_form=ROWS)
 
 
 @pytest.mark.parametrize("rows", [
@@ -79,7 +103,14 @@ def test_prefill_queued_bodies(ghip, rows):
     assert 6.0 * sum(rows) * dim * inter > 3e9 and sum(rows) > len(rows)
     T, k = routing_of(rows, np.random.default_rng(0)).shape
     assert T * k < 128 * len(rows) * 16
-    check(ghip, dim, inter, rows + [0] * max(0, (T * k) // 127 + 1 - len(rows)), nan=(1, 4, 13))
+    check(ghip, dim, inter, rows + [0] * max(0, (T * k) // 127 + 1 - len(rows)), nan=(1, 4, 13),
+          want_form=QUEUED)
+
+
+@pytest.mark.parametrize("rows", [[256, 255, 225, 224], [257, 130, 300, 129, 31], [193, 192, 160, 128]])
+def test_prefill_full_tiles(ghip, rows):
+    """Tiles mostly full: each body of the static form."""
+    check(ghip, 512, 256, rows, nan=(3,), want_form=FULL)
 
 
 def test_prefill_permutation_limit(ghip):
