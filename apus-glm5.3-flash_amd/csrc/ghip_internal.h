@@ -212,6 +212,10 @@ hipError_t ghip_launch_moe_prefill(const GhipBank *bank, const uint16_t *x,
                                    const GhipMoePrefillWs *ws,
                                    const hipEvent_t *ev, hipStream_t st);
 
+/* Tokens of one pass over the kernels, whose offsets into x and into h are of
+ * 32 bits: T, or a share of it (topk with the shared expert's slot; host only). */
+size_t ghip_moe_prefill_tokens(uint32_t dim, uint32_t inter, uint32_t topk, size_t T);
+
 /* Which products a prefill of T tokens x topk slots over n_experts takes (the
  * shared expert counted in both; host only, no device needed). */
 enum { GHIP_MOE_QUEUED, GHIP_MOE_FULL, GHIP_MOE_ROWS };

@@ -1476,6 +1476,18 @@ extern "C" int ghip_moe_prefill_form(uint32_t dim, uint32_t inter, uint32_t n_ex
     return GHIP_MOE_QUEUED;
 }
 
+extern "C" size_t ghip_moe_prefill_tokens(uint32_t dim, uint32_t inter, uint32_t topk, size_t T) {
+    const size_t rows = 0xffffffffu / 2u / dim, hrows = 0xffffffffu / 2u / inter / topk;
+    const size_t most = rows < hrows ? rows : hrows;
+    if (T <= most) return T;
+    const size_t n = (T + most - 1) / most;
+    return (T + n - 1) / n;
+}
+
+static hipError_t pf_launch(const GhipBank *bank, const uint16_t *x, size_t T, const int32_t *idx,
+                            const float *w, int topk, float limit, uint16_t *out,
+                            const GhipMoePrefillWs *ws, const hipEvent_t *ev, hipStream_t st);
+
 extern "C" hipError_t ghip_launch_moe_prefill(const GhipBank *bank,
                                               const uint16_t *x, size_t T,
                                               const int32_t *idx, const float *w,
@@ -1502,12 +1514,32 @@ extern "C" hipError_t ghip_launch_moe_prefill(const GhipBank *bank,
         || (bank->off_dw & 15) || (bank->off_gs & 3) || (bank->off_us & 3)
         || (bank->off_ds & 3))
         return hipErrorInvalidValue;
+    /* the kernels' activation offsets have 32 bits: more tokens go in slices,
+     * one after the other through the same workspace; the events span them */
+    const size_t Ts = ghip_moe_prefill_tokens(dim, inter, topk_p, T);
+    for (size_t t = 0; t < T; t += Ts) {
+        const size_t n = T - t < Ts ? T - t : Ts;
+        hipEvent_t se[8];
+        for (int i = 0; i < 8; i++)
+            se[i] = ev && (i & 1 ? t + n == T : t == 0) ? ev[i] : nullptr;
+        const hipError_t e = pf_launch(bank, x + t * dim, n, idx + t * topk, w + t * topk, topk,
+                                       limit, out + t * dim, ws, se, st);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+/* One slice, its arguments checked. */
+static hipError_t pf_launch(const GhipBank *bank, const uint16_t *x, size_t T, const int32_t *idx,
+                            const float *w, int topk, float limit, uint16_t *out,
+                            const GhipMoePrefillWs *ws, const hipEvent_t *ev, hipStream_t st) {
+    const uint32_t dim = bank->dim, inter = bank->inter, E = bank->n_experts;
+    const uint32_t sh = bank->has_shared ? 1u : 0u, Ep = E + sh;
+    const uint32_t topk_p = (uint32_t)topk + sh;
+    const size_t P = T * (size_t)topk_p;
     const uint32_t nch = (uint32_t)ghip_moe_prefill_chunks(P);
-    const size_t mt = ghip_moe_prefill_max_tiles(P, Ep);
-    hipEvent_t e0 = ev ? ev[0] : nullptr, e1 = ev ? ev[1] : nullptr;
-    hipEvent_t e2 = ev ? ev[2] : nullptr, e3 = ev ? ev[3] : nullptr;
-    hipEvent_t e4 = ev ? ev[4] : nullptr, e5 = ev ? ev[5] : nullptr;
-    hipEvent_t e6 = ev ? ev[6] : nullptr, e7 = ev ? ev[7] : nullptr;
+    hipEvent_t e0 = ev[0], e1 = ev[1], e2 = ev[2], e3 = ev[3];
+    hipEvent_t e4 = ev[4], e5 = ev[5], e6 = ev[6], e7 = ev[7];
     hipError_t e;
     if (P <= PF_CHUNK) {
         GHIP_LAUNCH(e0, e1, k_pf_permute, dim3(1), dim3(1024), 17 * Ep * 4, st, idx, (uint32_t)P,
@@ -1528,7 +1560,6 @@ extern "C" hipError_t ghip_launch_moe_prefill(const GhipBank *bank,
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     const size_t lds = PF_LDS, lds8 = PF_LDS_WB;
-    (void)mt;
     const uint32_t g0 = ws->n_cu, g1 = ws->n_cu;
     const int form = ghip_moe_prefill_form(dim, inter, Ep, topk_p, T);
     if (form == GHIP_MOE_ROWS) {

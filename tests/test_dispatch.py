@@ -88,3 +88,15 @@ def test_prefill_form(pkg, dim, inter, experts, k, T, want):
     f = pkg.load().ghip_moe_prefill_form
     f.argtypes = [ctypes.c_uint32] * 4 + [ctypes.c_size_t]
     assert f(dim, inter, experts, k, T) == want
+
+
+@pytest.mark.parametrize("dim,inter,k,T", [
+    (4096, 2048, 8, 8192), (4096, 2048, 8, 131071), (4096, 2048, 8, 131072), (4096, 2048, 9, 1 << 20), (256, 16384, 1, 131272),
+    (16384, 128, 1, 131071), (16384, 128, 1, 131072), (256, 128, 1, 1 << 25), (256, 128, 16, 1)])
+def test_prefill_slices_keep_offsets_in_32_bits(pkg, dim, inter, k, T):
+    f = pkg.load().ghip_moe_prefill_tokens
+    f.restype, f.argtypes = ctypes.c_size_t, [ctypes.c_uint32] * 3 + [ctypes.c_size_t]
+    n = f(dim, inter, k, T)
+    assert 1 <= n <= T and n * dim * 2 < 1 << 32 and n * k * inter * 2 < 1 << 32
+    fits = T * dim * 2 < 1 << 32 and T * k * inter * 2 < 1 << 32
+    assert (n == T) == fits

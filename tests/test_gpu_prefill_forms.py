@@ -134,3 +134,28 @@ def test_prefill_permutation_limit(ghip):
         assert_close_combined(b, want, floor([slab] * E, dim, inter, x, idx, w, eo), "1025 pairs")
     finally:
         ghip.apus_ghip_store_close(s)
+
+
+def test_prefill_activations_past_4_gib(ghip):
+    """h of more than 4 GiB: the tokens go in slices, and each reads its own
+    rows of x and h."""
+    dim, inter, E, T, period = 256, 16384, 2, 131272, 1009
+    assert T * inter * 2 > 1 << 32
+    rng = np.random.default_rng(9)
+    slabs = random_slabs(E, dim, inter, rng)
+    s = open_store(ghip, E, dim, inter)
+    try:
+        for e, sl in enumerate(slabs):
+            assert ghip.apus_ghip_store_put(s, e, O.ptr(sl), sl.nbytes) == 0
+        x = O.f32_to_bf16(rng.standard_normal((period, dim)).astype(np.float32))
+        idx = rng.integers(0, E, (period, 1)).astype(np.int32)
+        w = rng.uniform(0.02, 0.6, (period, 1)).astype(np.float32)
+        out = prefill(ghip, s, np.resize(x, (T, dim)), np.resize(idx, (T, 1)), np.resize(w, (T, 1)),
+                      host=False)
+        want, eo = O.moe_forward(slabs, dim, inter, x, idx, w, want_expert_out=True, threads=16)
+        assert_close_combined(out[:period], want, floor(slabs, dim, inter, x, idx, w, eo), "first tokens")
+        whole = T // period * period
+        assert (out[:whole].reshape(-1, period, dim) == out[:period]).all()
+        assert np.array_equal(out[whole:], out[:T - whole])
+    finally:
+        ghip.apus_ghip_store_close(s)
