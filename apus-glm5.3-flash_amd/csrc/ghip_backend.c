@@ -23,6 +23,7 @@
 #include <pthread.h>
 #include <semaphore.h>
 #include <stdarg.h>
+#include <stdatomic.h>
 #include <unistd.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -70,7 +71,7 @@ static struct {
     void *d_w, *d_s, *d_x, *d_y;
     size_t cap_w, cap_s, cap_x, cap_y;
     uint8_t *pin;                /* pinned host memory of the small transfers */
-    size_t pin_off;              /* its bytes in use until the next wait */
+    size_t pin_off;              /* its bytes in use */
     uint32_t *d_flag;            /* ephemeral NaN-scan flag */
     uint32_t *d_flags;           /* pool of cached scan flags */
     int n_scan;
@@ -337,11 +338,39 @@ uint64_t apus_ghip_bytes_d2h(void) { return G.d2h; }
 /* host-pointer entry points                                                */
 /* ------------------------------------------------------------------------ */
 
+/* The pinned memory belongs to one call at a time: to the first that takes a
+ * piece, until it has waited for the stream. A call of another thread
+ * meanwhile (decodes of two stores) has its copies made by the runtime. */
+static atomic_flag pin_busy = ATOMIC_FLAG_INIT;
+static _Thread_local int pin_mine;
+
+static void pin_release(void) {
+    if (!pin_mine) return;
+    pin_mine = 0;
+    atomic_flag_clear(&pin_busy);
+}
+
+/* In each entry point that copies: a return before sync_out has waited gives
+ * the memory back too, once no copy reads it. */
+static void pin_scope_end(const int *unused) {
+    (void)unused;
+    if (!pin_mine) return;
+    hipStreamSynchronize(G.stream);
+    pin_release();
+}
+#define PIN_SCOPE __attribute__((cleanup(pin_scope_end), unused)) const int pin_scope = 0
+
 /* A piece of the pinned memory for n bytes, or NULL if they are many, there is
- * no room until the next wait, or the copy kernel cannot take the address. */
+ * no room, another thread has it, or the copy kernel cannot take the address. */
 static uint8_t *pin_take(const void *d, size_t n) {
     const size_t r = (n + 15) & ~(size_t)15;
-    if (n > GHIP_PIN_COPY || r > GHIP_PIN_BYTES - G.pin_off || ((uintptr_t)d & 15)) return NULL;
+    if (n > GHIP_PIN_COPY || ((uintptr_t)d & 15)) return NULL;
+    if (!pin_mine) {
+        if (atomic_flag_test_and_set(&pin_busy)) return NULL;
+        pin_mine = 1;
+        G.pin_off = 0;
+    }
+    if (r > GHIP_PIN_BYTES - G.pin_off) return NULL;
     uint8_t *p = G.pin + G.pin_off;
     G.pin_off += r;
     return p;
@@ -377,7 +406,7 @@ static int sync_out(void *h, const void *d, size_t n) {
     else HIPCHK(hipMemcpyAsync(h, d, n, hipMemcpyDeviceToHost, G.stream));
     HIPCHK(hipStreamSynchronize(G.stream));
     if (p) memcpy(h, p, n);
-    G.pin_off = 0;
+    pin_release();
     G.d2h += n;
     return 0;
 }
@@ -396,6 +425,7 @@ static int check_sizes(size_t M, size_t O, size_t K) {
 
 int apus_ghip_bf16_gemm(const uint16_t *w, const uint16_t *x, uint16_t *y,
                         size_t M, size_t O, size_t K) {
+    PIN_SCOPE;
     if (ghip_init() || check_sizes(M, O, K)) return 1;
     const void *dw = weight_dev(w, O * K * 2, &G.d_w, &G.cap_w);
     if (!dw) return 1;
@@ -413,6 +443,7 @@ int apus_ghip_bf16_gemm(const uint16_t *w, const uint16_t *x, uint16_t *y,
 int apus_ghip_fp8blk_linear(const uint8_t *codes, const float *scales,
                             const uint16_t *x, uint16_t *y,
                             size_t M, size_t O, size_t K) {
+    PIN_SCOPE;
     if (ghip_init() || check_sizes(M, O, K)) return 1;
     size_t nsb = ((O + 127) / 128) * ((K + 127) / 128) * sizeof(float);
     int reg = region_find(codes, O * K) != NULL;
@@ -440,6 +471,7 @@ int apus_ghip_fp8blk_linear(const uint8_t *codes, const float *scales,
 
 int apus_ghip_fp8blk_dequant(const uint8_t *codes, const float *scales,
                              uint16_t *out, size_t O, size_t K) {
+    PIN_SCOPE;
     if (ghip_init() || check_sizes(1, O, K)) return 1;
     size_t nsb = ((O + 127) / 128) * ((K + 127) / 128) * sizeof(float);
     const void *dc = weight_dev(codes, O * K, &G.d_w, &G.cap_w);
@@ -982,6 +1014,7 @@ int apus_ghip_store_synth(ApusGhipStore *s, uint64_t seed, int bank,
 
 int apus_ghip_store_expert_bf16(ApusGhipStore *s, int expert,
                                 uint16_t *payload) {
+    PIN_SCOPE;
     if (!s || expert < 0 || expert >= s->n_experts) {
         ghip_seterr("store_expert_bf16: bad expert %d", expert);
         return 1;
@@ -1158,6 +1191,7 @@ int apus_ghip_moe_router_dev(const uint16_t *x, const uint16_t *gate_w,
 int apus_ghip_moe_decode(ApusGhipStore *s, const uint16_t *x,
                          const int32_t *idx, const float *w, int topk,
                          uint16_t *out) {
+    PIN_SCOPE;
     if (!s) { ghip_seterr("moe_decode: no store"); return 1; }
     if (topk <= 0 || topk > GHIP_MAX_TOPK) {
         ghip_seterr("moe_decode: topk %d outside 1..%d", topk, GHIP_MAX_TOPK);
@@ -1325,6 +1359,7 @@ int apus_ghip_moe_prefill_dev_noalloc(ApusGhipStore *s, const uint16_t *x, size_
 int apus_ghip_moe_prefill(ApusGhipStore *s, const uint16_t *x, size_t T,
                           const int32_t *idx, const float *w, int topk,
                           uint16_t *out) {
+    PIN_SCOPE;
     if (!s) { ghip_seterr("moe_prefill: no store"); return 1; }
     if (topk <= 0 || topk > GHIP_MAX_TOPK) {
         ghip_seterr("moe_prefill: topk %d outside 1..%d", topk, GHIP_MAX_TOPK);
