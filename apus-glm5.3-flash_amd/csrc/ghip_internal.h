@@ -49,6 +49,10 @@ enum { GHIP_ROUTE_ANY, GHIP_ROUTE_GEMV, GHIP_ROUTE_ROWS, GHIP_ROUTE_GEMM };
 int ghip_fp8_linear_route(const void *codes, const void *x, const void *y, size_t M, size_t O,
                           size_t K, uint32_t n_cu);
 
+/* ... and a BF16 one. */
+int ghip_bf16_linear_route(const void *w, const void *x, size_t M, size_t O, size_t K,
+                           uint32_t n_cu);
+
 /* BF16-weight GEMV/GEMM: y[M,O] = x[M,K] . W[O,K]^T. Any shape. ev: NULL or
  * two timing events (start on the first launch, stop on the last). */
 hipError_t ghip_launch_bf16_linear(const uint16_t *w, const uint16_t *x,

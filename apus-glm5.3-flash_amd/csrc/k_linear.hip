@@ -1,11 +1,12 @@
 /*
  * k_linear.hip — gfx950 kernels for the dense FP8-block path:
- *   K2  k_fp8_gemv_stream : decode / MTP-verify GEMV (M <= 4, many weight
- *       rows) with the dequant fused in registers and the k reduction on MFMA
- *       (v_mfma_f32_16x16x32_bf16), the composition of c/gdsa.h:525-534
- *       (dequant -> bf16 -> fp32-accumulated GEMM -> RNE bf16). Other row
- *       counts and shapes: k_rows.hip, k_moe_prefill.hip (k_fp8_gemm) and,
- *       for BF16 weights, k_rows.hip and k_gemm_bf16.hip.
+ *   K2  k_fp8_gemv_stream : decode / MTP-verify GEMV (M <= 4) of many FP8
+ *       weight rows, with the dequant fused in registers and the k reduction
+ *       on MFMA (v_mfma_f32_16x16x32_bf16), the composition of
+ *       c/gdsa.h:525-534 (dequant -> bf16 -> fp32-accumulated GEMM -> RNE
+ *       bf16), and of few long BF16 ones (c/bf16.h:712-767). Other row counts
+ *       and shapes: k_rows.hip, k_moe_prefill.hip (k_fp8_gemm) and, for BF16
+ *       weights, k_gemm_bf16.hip.
  *   k_linear_any : shape-general fallback (K not a multiple of 128 / 64,
  *       unaligned operands) with the exact integer decode.
  *   k_nan_scan : flags the out-of-contract NaN codes 0x7F/0xFF so callers
@@ -163,35 +164,37 @@ extern "C" hipError_t ghip_launch_nan_scan(const uint8_t *codes, size_t n,
 }
 
 /* ------------------------------------------------------------------------ */
-/* K2: persistent FP8 GEMV, M <= 4, x staged once, weights streamed         */
+/* K2: persistent GEMV, M <= 4, x staged once, weights streamed             */
 /* ------------------------------------------------------------------------ */
 
 #define GS_NW 8                  /* waves per workgroup */
-/* LDS chunk slots per wave: a chunk is written from registers and read
- * back in the MFMA layout while the next one is in flight (measured on
+/* chunks in flight and LDS slots of a wave: a chunk is written from registers
+ * and read back in the MFMA layout while the next ones are in flight (FP8,
  * 16384 x 4096: one 13.8 us, two 12.3, three 12.6) */
-#define GS_R 2
-#define GS_X_MAX (48u * 1024u)   /* most bytes of x staged (K <= 6144 at M = 4) */
+#define GS_NA(BF) ((BF) ? 3u : 2u)
+#define GS_X_MAX (48u * 1024u)   /* FP8: most bytes of x staged (K <= 6144 at M = 4) */
 #define GS_LDS (144u * 1024u)    /* dynamic LDS limit of the streaming GEMV */
 
 /* Y[m, rows] for M <= 4 token rows. A row group (16 weight rows) is split
- * over two waves along K; a workgroup pass covers 4 row groups, passes run
- * over the groups persistently (one workgroup per CU). Each wave streams its
- * chunks (16 rows x 128 codes, one scale block) through registers: two
- * 16-byte loads per lane in a whole-line pattern (load i: rows 8i + lane /
- * 8, piece lane % 8), two chunks in flight, each chunk written to a
- * wave-private LDS slot (lane l's bytes at 16 l, piece p of row r at p ^
- * ((r >> 1) & 7)) and read back in the MFMA layout, dequantized in registers
- * and reduced on MFMA with the token rows of x (staged once per workgroup)
- * as the A operand: A row i = lane % 16 is token min(i, M-1), rows past M
- * feed output rows that are discarded. The two partial sums of a group are
- * added in LDS in a fixed order (deterministic). */
-template <int M>
+ * over KS waves along K (FP8 2, BF16 8); a workgroup pass covers 8 / KS row
+ * groups, passes run over the groups persistently (at most one workgroup per
+ * CU). Each wave streams its chunks (16 rows x 128 bytes: 128 codes, one scale
+ * block, or 64 BF16 weights) through registers: two 16-byte loads per lane in
+ * a whole-line pattern (load i: rows 8i + lane / 8, piece lane % 8), NA chunks
+ * in flight, each chunk written to a wave-private LDS slot (lane l's bytes at
+ * 16 l, piece p of row r at p ^ ((r >> 1) & 7)) and read back in the MFMA
+ * layout, dequantized in registers (FP8) and reduced on MFMA with the token
+ * rows of x (staged once per workgroup) as the A operand: A row i = lane % 16
+ * is token min(i, M-1), rows past M feed output rows that are discarded. The
+ * KS partial sums of a group are added in LDS in a fixed order
+ * (deterministic). */
+template <int M, int KS, bool BF>
 __global__ __launch_bounds__(GS_NW * 64, 1) void k_fp8_gemv_stream(
     const uint8_t *__restrict__ W, const float *__restrict__ S,
     const uint16_t *__restrict__ X, uint16_t *__restrict__ Y, uint32_t O,
     uint32_t K, const uint32_t *__restrict__ exact_flag) {
-    constexpr uint32_t KS = 2, GPP = GS_NW / KS;     /* K splits, row groups per pass */
+    constexpr uint32_t GPP = GS_NW / KS;             /* row groups per pass */
+    constexpr uint32_t NA = GS_NA(BF);               /* chunks in flight, LDS slots */
     extern __shared__ __attribute__((aligned(1024))) uint8_t gsl[];
     __shared__ float red[GPP][KS][M][16];
     uint16_t *xs = (uint16_t *)gsl;
@@ -199,34 +202,40 @@ __global__ __launch_bounds__(GS_NW * 64, 1) void k_fp8_gemv_stream(
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t n = lane & 15u, g = lane >> 4;
     uint8_t *ring = gsl + (((size_t)M * K * 2u + 1023u) & ~(size_t)1023u) +
-                    wv * (GS_R * 2048u);
-    const uint32_t nch = K >> 7, nkb = K >> 7;
+                    wv * (NA * 2048u);
+    /* chunk = 128 bytes of each of 16 rows; row stride in bytes */
+    const uint32_t KB = BF ? 2u * K : K;
+    const uint32_t nch = KB >> 7, nkb = K >> 7;
     const uint32_t part = wv % KS, slot = wv / KS;
     const uint32_t c0 = part * nch / KS, c1 = (part + 1) * nch / KS, nc = c1 - c0;
     const uint32_t groups = (O + 15) / 16, passes = (groups + GPP - 1) / GPP;
-    const uint16_t *xa = xs + (size_t)min(n, (uint32_t)M - 1u) * K + 32u * g;
+    const uint16_t *xa = xs + (size_t)min(n, (uint32_t)M - 1u) * K + (BF ? 16u : 32u) * g;
     /* pass ps's row group of this wave: its rows and load offsets (a
      * partial last group re-reads row O-1, outputs discarded) */
     auto rows_of = [&](uint32_t ps) {
-        return W + (size_t)(ps * GPP + slot) * 16u * K;
+        return W + (size_t)(ps * GPP + slot) * 16u * KB;
     };
     auto offs_of = [&](uint32_t ps) {
-        return ghip_cdma_offsets(lane, K, min(15u, O - 1u - (ps * GPP + slot) * 16u));
+        return ghip_cdma_offsets(lane, KB, min(15u, O - 1u - (ps * GPP + slot) * 16u));
     };
-    /* two chunks in flight: chunk t's two 16-byte pieces in register set t % 2
-     * ((ra0, ra1), (rb0, rb1)) and LDS slot t % 2 */
-    ghip_u32x4 ra0, ra1, rb0, rb1;
-    /* the first two chunks of a pass, always both loaded (chunk indices
+    /* chunk t's two 16-byte pieces in register set t % NA ((ra0, ra1), (rb0,
+     * rb1), (rc0, rc1)) and LDS slot t % NA */
+    ghip_u32x4 ra0, ra1, rb0, rb1, rc0, rc1;
+    /* the first NA chunks of a pass, always all loaded (chunk indices
      * clamped): a fixed count of loads in flight, in a fixed order */
     auto prefetch = [&](const uint8_t *rows, const ghip_cdma &d) {
         ghip_rl_load(rows, d, min(c0, nch - 1u), ra0, ra1);
         __builtin_amdgcn_sched_barrier(0);
         ghip_rl_load(rows, d, min(c0 + 1u, nch - 1u), rb0, rb1);
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (NA == 3u) {
+            ghip_rl_load(rows, d, min(c0 + 2u, nch - 1u), rc0, rc1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
     /* x into LDS without delaying the weight stream: x goes by direct DMA
      * (1 K pieces dealt to the waves, lanes past x re-read its last vector
-     * into the 1 K-rounded x region) ahead of the first pass's four chunk
+     * into the 1 K-rounded x region) ahead of the first pass's 2 NA chunk
      * loads, so waiting until no more than those are in flight means this
      * wave's x pieces have landed */
     {
@@ -234,62 +243,91 @@ __global__ __launch_bounds__(GS_NW * 64, 1) void k_fp8_gemv_stream(
         for (uint32_t c = wv; c < nxc; c += GS_NW)
             ghip_dma16(X + (size_t)min(c * 64u + lane, nvec - 1u) * 8u, gsl + c * 1024u);
         const uint32_t grp0 = min(blockIdx.x * GPP + slot, groups - 1u);
-        prefetch(W + (size_t)grp0 * 16u * K,
-               ghip_cdma_offsets(lane, K, min(15u, O - 1u - grp0 * 16u)));
-        GHIP_VMCNT(4);
+        prefetch(W + (size_t)grp0 * 16u * KB,
+               ghip_cdma_offsets(lane, KB, min(15u, O - 1u - grp0 * 16u)));
+        GHIP_VMCNT(2 * NA);
     }
     /* a bare barrier: __syncthreads() would also wait for the chunk loads
      * (its workgroup-scope release waits for every load in flight) */
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    const bool exact = exact_flag != nullptr && *exact_flag != 0u;
+    const bool exact = !BF && exact_flag != nullptr && *exact_flag != 0u;
     for (uint32_t ps = blockIdx.x; ps < passes; ps += gridDim.x) {
         const uint32_t grp = ps * GPP + slot;
         const bool live = grp < groups;
         if (live) {
-            /* a wave with no chunks (K < 256) contributes zeros */
+            /* a wave with no chunks contributes zeros */
             const uint32_t row0 = grp * 16;
             const uint8_t *rows = rows_of(ps);
             const ghip_cdma d = offs_of(ps);
-            const float *srow = S + (size_t)(row0 >> 7) * nkb;
+            const float *srow = BF ? nullptr : S + (size_t)(row0 >> 7) * nkb;
             if (ps != blockIdx.x) prefetch(rows, d);
             ghip_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            /* chunk t: its registers into LDS slot t % 2, the registers
-             * refilled with chunk t + 2 (REFILL), the chunk read back in
+            /* chunk t: its registers into LDS slot t % NA, the registers
+             * refilled with chunk t + NA (REFILL), the chunk read back in
              * the MFMA layout with this lane's activations and the scale */
             auto step = [&](auto refill_c, uint32_t t, ghip_u32x4 &v0, ghip_u32x4 &v1,
                             uint8_t *buf) {
                 ghip_rl_store(buf, lane, v0, v1);
                 if constexpr (decltype(refill_c)::value) {
                     __builtin_amdgcn_sched_barrier(0);
-                    ghip_rl_load(rows, d, c0 + t + 2u, v0, v1);
+                    ghip_rl_load(rows, d, c0 + t + NA, v0, v1);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 const uint32_t c = c0 + t;
                 const ghip_chunk cw = ghip_cdma_read(buf, n, g);
-                ghip_bf16x8 a4[4];
-                ghip_read_a4(xa + c * 128u, a4);
-                const float sc = ghip_sload(srow, c);
-                if (exact) ghip_chunk_mfma_a<true>(cw, sc, a4, acc);
-                else ghip_chunk_mfma_a<false>(cw, sc, a4, acc);
+                if constexpr (BF) {
+                    const ghip_bf16x8 *a = (const ghip_bf16x8 *)(xa + c * 64u);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        a[0], __builtin_bit_cast(ghip_bf16x8, cw.lo), acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        a[1], __builtin_bit_cast(ghip_bf16x8, cw.hi), acc, 0, 0, 0);
+                } else {
+                    ghip_bf16x8 a4[4];
+                    ghip_read_a4(xa + c * 128u, a4);
+                    const float sc = ghip_sload(srow, c);
+                    if (exact) ghip_chunk_mfma_a<true>(cw, sc, a4, acc);
+                    else ghip_chunk_mfma_a<false>(cw, sc, a4, acc);
+                }
             };
             using RF = std::true_type;
             using NR = std::false_type;
             uint32_t t = 0;
-            for (; t + 3u < nc; t += 2) {
-                step(RF{}, t, ra0, ra1, ring);
-                step(RF{}, t + 1u, rb0, rb1, ring + 2048u);
-            }
-            if (nc - t == 3u) {
-                step(RF{}, t, ra0, ra1, ring);
-                step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
-                step(NR{}, t + 2u, ra0, ra1, ring);
-            } else if (nc - t == 2u) {
-                step(NR{}, t, ra0, ra1, ring);
-                step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
-            } else if (nc - t == 1u) {
-                step(NR{}, t, ra0, ra1, ring);
+            if constexpr (NA == 2u) {
+                for (; t + 3u < nc; t += 2) {
+                    step(RF{}, t, ra0, ra1, ring);
+                    step(RF{}, t + 1u, rb0, rb1, ring + 2048u);
+                }
+                if (nc - t == 3u) {
+                    step(RF{}, t, ra0, ra1, ring);
+                    step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
+                    step(NR{}, t + 2u, ra0, ra1, ring);
+                } else if (nc - t == 2u) {
+                    step(NR{}, t, ra0, ra1, ring);
+                    step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
+                } else if (nc - t == 1u) {
+                    step(NR{}, t, ra0, ra1, ring);
+                }
+            } else {
+                for (; t + 5u < nc; t += 3) {
+                    step(RF{}, t, ra0, ra1, ring);
+                    step(RF{}, t + 1u, rb0, rb1, ring + 2048u);
+                    step(RF{}, t + 2u, rc0, rc1, ring + 4096u);
+                }
+                const uint32_t rem = nc - t;
+                if (rem > 3u) {
+                    step(RF{}, t, ra0, ra1, ring);
+                    if (rem > 4u) step(RF{}, t + 1u, rb0, rb1, ring + 2048u);
+                    else step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
+                    step(NR{}, t + 2u, rc0, rc1, ring + 4096u);
+                    step(NR{}, t + 3u, ra0, ra1, ring);
+                    if (rem > 4u) step(NR{}, t + 4u, rb0, rb1, ring + 2048u);
+                } else {
+                    if (rem > 0u) step(NR{}, t, ra0, ra1, ring);
+                    if (rem > 1u) step(NR{}, t + 1u, rb0, rb1, ring + 2048u);
+                    if (rem > 2u) step(NR{}, t + 2u, rc0, rc1, ring + 4096u);
+                }
             }
             if (g == 0) {
 #pragma unroll
@@ -317,18 +355,37 @@ __global__ __launch_bounds__(GS_NW * 64, 1) void k_fp8_gemv_stream(
 
 static uint32_t g_gs_ncu;                 /* CUs: the streaming grid bound */
 
-/* LDS the streaming GEMV needs for M token rows of length K */
-static size_t gs_lds(size_t M, size_t K) {
-    return ((M * K * 2 + 1023) & ~(size_t)1023) + (size_t)GS_NW * GS_R * 2048;
+/* LDS the streaming GEMV needs for M token rows of length K and `na` chunk
+ * slots a wave */
+static size_t gs_lds(size_t M, size_t K, size_t na) {
+    return ((M * K * 2 + 1023) & ~(size_t)1023) + (size_t)GS_NW * na * 2048;
 }
 
-template <int M>
-static hipError_t launch_gemv_m(const uint8_t *codes, const float *scales, const uint16_t *x,
-                                uint16_t *y, size_t O, size_t K, const uint32_t *exact_dev,
-                                hipEvent_t ev0, hipEvent_t ev1, hipStream_t st) {
-    GHIP_LAUNCH(ev0, ev1, k_fp8_gemv_stream<M>, dim3(g_gs_ncu), dim3(GS_NW * 64), gs_lds(M, K), st,
-                codes, scales, x, y, (uint32_t)O, (uint32_t)K, exact_dev);
+/* FP8: K over two waves, a workgroup per CU; BF16: K over all eight waves, a
+ * workgroup per row group. */
+template <int M, bool BF>
+static hipError_t launch_gemv_m(const void *w, const float *scales, const uint16_t *x, uint16_t *y,
+                                size_t O, size_t K, const uint32_t *exact_dev, hipEvent_t ev0,
+                                hipEvent_t ev1, hipStream_t st) {
+    constexpr int KS = BF ? 8 : 2;
+    const size_t groups = (O + 15) / 16;
+    const uint32_t grid = BF && groups < g_gs_ncu ? (uint32_t)groups : g_gs_ncu;
+    GHIP_LAUNCH(ev0, ev1, (k_fp8_gemv_stream<M, KS, BF>), dim3(grid), dim3(GS_NW * 64),
+                gs_lds(M, K, GS_NA(BF)), st, (const uint8_t *)w, scales, x, y, (uint32_t)O,
+                (uint32_t)K, exact_dev);
     return hipGetLastError();
+}
+
+template <bool BF>
+static hipError_t launch_gemv(const void *w, const float *scales, const uint16_t *x, uint16_t *y,
+                              size_t M, size_t O, size_t K, const uint32_t *exact_dev,
+                              hipEvent_t ev0, hipEvent_t ev1, hipStream_t st) {
+    switch (M) {
+    case 4: return launch_gemv_m<4, BF>(w, scales, x, y, O, K, exact_dev, ev0, ev1, st);
+    case 3: return launch_gemv_m<3, BF>(w, scales, x, y, O, K, exact_dev, ev0, ev1, st);
+    case 2: return launch_gemv_m<2, BF>(w, scales, x, y, O, K, exact_dev, ev0, ev1, st);
+    default: return launch_gemv_m<1, BF>(w, scales, x, y, O, K, exact_dev, ev0, ev1, st);
+    }
 }
 
 /* Rows of X from which the MFMA GEMM (N % 256 == 0) is considered. */
@@ -371,12 +428,7 @@ extern "C" hipError_t ghip_launch_fp8_linear(const uint8_t *codes,
     hipEvent_t ev0 = ev ? ev[0] : nullptr, ev1 = ev ? ev[1] : nullptr;
     switch (ghip_fp8_linear_route(codes, x, y, M, O, K, g_gs_ncu)) {
     case GHIP_ROUTE_GEMV:
-        switch (M) {
-        case 4: return launch_gemv_m<4>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
-        case 3: return launch_gemv_m<3>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
-        case 2: return launch_gemv_m<2>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
-        default: return launch_gemv_m<1>(codes, scales, x, y, O, K, exact_dev, ev0, ev1, st);
-        }
+        return launch_gemv<false>(codes, scales, x, y, M, O, K, exact_dev, ev0, ev1, st);
     case GHIP_ROUTE_GEMM:
         return ghip_launch_fp8_gemm(codes, scales, x, y, M, O, K, exact_dev, g_gs_ncu, ev, st);
     case GHIP_ROUTE_ROWS:
@@ -384,6 +436,28 @@ extern "C" hipError_t ghip_launch_fp8_linear(const uint8_t *codes,
                                 st);
     default: return launch_linear_any<false>(codes, scales, x, y, M, O, K, ev0, ev1, st);
     }
+}
+
+/* The kernel of a BF16 linear on n_cu CUs. */
+extern "C" int ghip_bf16_linear_route(const void *w, const void *x, size_t M, size_t O, size_t K,
+                                      uint32_t n_cu) {
+    if (!n_cu) return GHIP_ROUTE_ANY;
+    const bool rows = ghip_rows_fits(1, M, O, K, w, x);
+    /* up to 4 rows against few long weight rows, a chain of chunk round trips
+     * with most CUs idle: x staged once and three chunks in flight (288 x 8192,
+     * M = 1: 7.1 us against 7.5 with x streamed beside the weights, M = 4 7.5
+     * against 7.9; 288 x 4096 4.76 against 4.84, but 288 x 2048 3.63 against
+     * 3.56, and 4096 x 4096 7.2 against 7.0) */
+    if (rows && M <= 4 && K >= 4096 && O <= 8u * (size_t)n_cu
+        && gs_lds(M, K, GS_NA(true)) <= GS_LDS)
+        return GHIP_ROUTE_GEMV;
+    /* the weight-streaming form reads the weights once per row tile, the
+     * GEMM's tiles share them: whichever is estimated faster (4096 x 4096:
+     * 12.3 against 15.5 us at M = 64, 20.2 against 15.9 at 96) */
+    if (ghip_bf16_gemm_fits(M, O, K, w, x)
+        && (!rows || ghip_bf16_gemm_estimate(M, O, K, n_cu) < ghip_rows_estimate(1, M, O, K, n_cu)))
+        return GHIP_ROUTE_GEMM;
+    return rows ? GHIP_ROUTE_ROWS : GHIP_ROUTE_ANY;
 }
 
 extern "C" hipError_t ghip_launch_bf16_linear(const uint16_t *w,
@@ -394,27 +468,25 @@ extern "C" hipError_t ghip_launch_bf16_linear(const uint16_t *w,
     if (K == 0 || O > 0x7fffffffu || K > 0x7fffffffu || M > 0x7fffffffu)
         return hipErrorInvalidValue;
     hipEvent_t ev0 = ev ? ev[0] : nullptr, ev1 = ev ? ev[1] : nullptr;
-    if (g_gs_ncu) {
-        /* the weight-streaming form reads the weights once per row tile, the
-         * GEMM's tiles share them: whichever is estimated faster (4096 x
-         * 4096: 12.3 against 15.5 us at M = 64, 20.2 against 15.9 at 96) */
-        const bool rows = ghip_rows_fits(1, M, O, K, w, x);
-        if (ghip_bf16_gemm_fits(M, O, K, w, x)
-            && (!rows || ghip_bf16_gemm_estimate(M, O, K, g_gs_ncu)
-                             < ghip_rows_estimate(1, M, O, K, g_gs_ncu)))
-            return ghip_launch_bf16_gemm(w, x, y, M, O, K, g_gs_ncu, ev0, ev1, st);
-        if (rows)
-            return ghip_launch_rows(1, w, nullptr, x, y, M, O, K, nullptr, g_gs_ncu, ev0, ev1,
-                                    st);
+    switch (ghip_bf16_linear_route(w, x, M, O, K, g_gs_ncu)) {
+    case GHIP_ROUTE_GEMV:
+        return launch_gemv<true>(w, nullptr, x, y, M, O, K, nullptr, ev0, ev1, st);
+    case GHIP_ROUTE_GEMM:
+        return ghip_launch_bf16_gemm(w, x, y, M, O, K, g_gs_ncu, ev0, ev1, st);
+    case GHIP_ROUTE_ROWS:
+        return ghip_launch_rows(1, w, nullptr, x, y, M, O, K, nullptr, g_gs_ncu, ev0, ev1, st);
+    default: return launch_linear_any<true>(w, nullptr, x, y, M, O, K, ev0, ev1, st);
     }
-    return launch_linear_any<true>(w, nullptr, x, y, M, O, K, ev0, ev1, st);
 }
 
 extern "C" hipError_t ghip_linear_init(uint32_t n_cu) {
-    const void *ks[4] = {(const void *)k_fp8_gemv_stream<1>, (const void *)k_fp8_gemv_stream<2>,
-                         (const void *)k_fp8_gemv_stream<3>, (const void *)k_fp8_gemv_stream<4>};
+    const void *ks[8] = {
+        (const void *)k_fp8_gemv_stream<1, 2, false>, (const void *)k_fp8_gemv_stream<2, 2, false>,
+        (const void *)k_fp8_gemv_stream<3, 2, false>, (const void *)k_fp8_gemv_stream<4, 2, false>,
+        (const void *)k_fp8_gemv_stream<1, 8, true>, (const void *)k_fp8_gemv_stream<2, 8, true>,
+        (const void *)k_fp8_gemv_stream<3, 8, true>, (const void *)k_fp8_gemv_stream<4, 8, true>};
     hipError_t e;
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < 8; i++)
         if ((e = hipFuncSetAttribute(ks[i], hipFuncAttributeMaxDynamicSharedMemorySize, GS_LDS))
             != hipSuccess)
             return e;

@@ -74,6 +74,24 @@ def test_fp8_few_rows_take_the_faster_kernel(pkg, M, N, K, want):
     assert fp8(pkg, M, N, K) == want
 
 
+def bf16(pkg, M, N, K, w=P, x=P, ncu=NCU):
+    f = pkg.load().ghip_bf16_linear_route
+    f.restype, f.argtypes = ctypes.c_int, [ctypes.c_void_p] * 2 + [ctypes.c_size_t] * 3 + [ctypes.c_uint32]
+    return f(w, x, M, N, K, ncu)
+
+
+def test_bf16_routes(pkg):
+    off = ctypes.c_void_p(P.value + 2)
+    # few long weight rows: x staged once
+    assert all(bf16(pkg, M, N, K) == GEMV for M in (1, 2, 4) for N in (64, 288, 2048) for K in (4096, 8192))
+    assert bf16(pkg, 1, 288, 2048) == ROWS and bf16(pkg, 1, 4096, 4096) == ROWS and bf16(pkg, 5, 288, 8192) == ROWS
+    assert bf16(pkg, 4, 288, 12288) == GEMV and bf16(pkg, 4, 288, 12288 + 64) == ROWS    # x in LDS
+    assert bf16(pkg, 1, 154880, 4096) == ROWS and bf16(pkg, 600, 4096, 4096) == GEMM
+    assert bf16(pkg, 2048, 288, 4096) == GEMM and bf16(pkg, 65535 * 64 + 1, 48, 64) in (ROWS, GEMM)
+    assert bf16(pkg, 1, 288, 4095) == ANY and bf16(pkg, 1, 288, 4096, w=off) == ANY
+    assert bf16(pkg, 1, 288, 4096, x=off) == ANY and bf16(pkg, 1, 288, 4096, ncu=0) == ANY
+
+
 QUEUED, FULL, STREAMS = range(3)
 
 

@@ -84,6 +84,16 @@ def test_rows_bf16(ghip, M, N, K):
     assert np.array_equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 17, 4096), (4, 288, 4160), (3, 2048, 4672), (2, 100, 4096 + 64 * 21),
+                                   (4, 33, 12288), (1, 2041, 8192 + 64)])
+def test_few_long_bf16_rows(ghip, M, N, K):
+    """Few long weight rows (the streaming GEMV with x staged): every count of
+    chunks left after its loop of three, and row remainders."""
+    assert ghip.ghip_bf16_linear_route(ctypes.c_void_p(16), ctypes.c_void_p(16), ctypes.c_size_t(M), ctypes.c_size_t(N),
+                                       ctypes.c_size_t(K), 256) == 1
+    test_rows_bf16(ghip, M, N, K)
+
+
 def test_rows_not_finite(ghip):
     """An infinity in x reaches exactly its own row (rows past M re-read the
     last one and are not stored)."""
