@@ -68,6 +68,8 @@ hipError_t ghip_launch_bf16_gemm(const uint16_t *w, const uint16_t *x, uint16_t 
                                  hipEvent_t e1, hipStream_t st);
 /* Its estimated time in microseconds (the dispatch compares it). */
 float ghip_bf16_gemm_estimate(size_t M, size_t N, size_t K, uint32_t n_cu);
+/* The tile it picks, rows << 16 | columns (the tests hold their cases to it). */
+uint32_t ghip_bf16_gemm_form(size_t M, size_t N, uint32_t n_cu);
 /* Raise its dynamic-LDS limits (once per process). */
 hipError_t ghip_bf16_gemm_init(void);
 
@@ -78,6 +80,8 @@ hipError_t ghip_bf16_gemm_init(void);
  * microseconds. */
 int ghip_rows_fits(int bf, size_t M, size_t N, size_t K, const void *w, const void *x);
 float ghip_rows_estimate(int bf, size_t M, size_t N, size_t K, uint32_t n_cu);
+/* The form it picks, rows of x << 16 | weight groups << 8 | K splits. */
+uint32_t ghip_rows_form(int bf, size_t M, size_t N, size_t K, uint32_t n_cu);
 hipError_t ghip_launch_rows(int bf, const void *w, const float *scales, const uint16_t *x,
                             uint16_t *y, size_t M, size_t N, size_t K,
                             const uint32_t *exact_dev, uint32_t n_cu, hipEvent_t e0,
@@ -252,6 +256,8 @@ hipError_t ghip_launch_fp8_gemm(const uint8_t *codes, const float *scales,
                                 const hipEvent_t *ev, hipStream_t st);
 /* Its estimated time in microseconds below 256 rows (the dispatch compares it). */
 float ghip_fp8_gemm_estimate(size_t M, size_t N, size_t K, uint32_t n_cu);
+/* Its tile height << 16 | K splits. */
+uint32_t ghip_fp8_gemm_form(size_t M, size_t N, size_t K, uint32_t n_cu);
 
 /* One expert slab record of a converted v2 container's apus.index.json
  * (c/gcache.h:896-930): the shard file name and the slab's file offset. */

@@ -290,6 +290,12 @@ extern "C" float ghip_bf16_gemm_estimate(size_t M, size_t N, size_t K, uint32_t 
     return (float)(3.0 + (t > hbm ? t : hbm));
 }
 
+extern "C" uint32_t ghip_bf16_gemm_form(size_t M, size_t N, uint32_t n_cu) {
+    double est = 0.0;
+    const BgTile *t = bg_pick(M, N, n_cu, &est);
+    return t->bm << 16 | t->bn;
+}
+
 extern "C" hipError_t ghip_launch_bf16_gemm(const uint16_t *w, const uint16_t *x, uint16_t *y,
                                             size_t M, size_t N, size_t K, uint32_t n_cu,
                                             hipEvent_t e0, hipEvent_t e1, hipStream_t st) {

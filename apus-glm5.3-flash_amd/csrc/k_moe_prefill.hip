@@ -1703,6 +1703,11 @@ extern "C" float ghip_fp8_gemm_estimate(size_t M, size_t N, size_t K, uint32_t n
                    + 1.68e-6 * p.S * (double)M * (double)N);
 }
 
+extern "C" uint32_t ghip_fp8_gemm_form(size_t M, size_t N, size_t K, uint32_t n_cu) {
+    const F8Plan p = f8_plan(M, N, K, n_cu);
+    return p.bm << 16 | p.S;
+}
+
 extern "C" hipError_t ghip_launch_fp8_gemm(const uint8_t *codes, const float *scales,
                                            const uint16_t *x, uint16_t *y, size_t M,
                                            size_t N, size_t K, const uint32_t *exact_dev,

@@ -337,6 +337,12 @@ extern "C" float ghip_rows_estimate(int bf, size_t M, size_t N, size_t K, uint32
     return est;
 }
 
+extern "C" uint32_t ghip_rows_form(int bf, size_t M, size_t N, size_t K, uint32_t n_cu) {
+    float est = 0.0f;
+    const RwCfg *c = rw_pick(bf != 0, M, N, K, n_cu, &est);
+    return c->mr << 16 | c->nt << 8 | c->ks;
+}
+
 extern "C" hipError_t ghip_launch_rows(int bf, const void *w, const float *scales,
                                        const uint16_t *x, uint16_t *y, size_t M, size_t N,
                                        size_t K, const uint32_t *exact_dev, uint32_t n_cu,

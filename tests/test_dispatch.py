@@ -2,6 +2,7 @@
 csrc/k_moe_prefill.hip), asked of the library's own dispatch: host code, so no
 device and no buffers of these sizes are needed."""
 import ctypes
+import random
 
 import pytest
 
@@ -90,6 +91,40 @@ def test_bf16_routes(pkg):
     assert bf16(pkg, 2048, 288, 4096) == GEMM and bf16(pkg, 65535 * 64 + 1, 48, 64) in (ROWS, GEMM)
     assert bf16(pkg, 1, 288, 4095) == ANY and bf16(pkg, 1, 288, 4096, w=off) == ANY
     assert bf16(pkg, 1, 288, 4096, x=off) == ANY and bf16(pkg, 1, 288, 4096, ncu=0) == ANY
+
+
+def test_every_form_that_is_picked_has_a_gpu_case(pkg):
+    """The forms of the streaming kernel, the tiles of the BF16 GEMM and the
+    heights of the FP8 one that shapes drawn at random reach are those that
+    the GPU tests hold a case to."""
+    import test_gpu_bf16_gemm
+    import test_gpu_fp8_gemm
+    import test_gpu_rows
+    lib, rng, z = pkg.load(), random.Random(2), ctypes.c_size_t
+    seen = {ROWS: set(), "bf16": set(), GEMM: set(), "fp8": set()}
+    for _ in range(20000):
+        M, N = int(2 ** rng.uniform(0, 11.5)), int(2 ** rng.uniform(4, 17))
+        K = 128 * int(2 ** rng.uniform(0, 7.1))
+        if rng.random() < 0.5:
+            N = N // 256 * 256 + 256
+        r = fp8(pkg, M, N, K)
+        if r == ROWS:
+            f = lib.ghip_rows_form(0, z(M), z(N), z(K), NCU)
+            seen[ROWS].add((f >> 16, f >> 8 & 255, f & 255))
+        elif r == GEMM:
+            f = lib.ghip_fp8_gemm_form(z(M), z(N), z(K), NCU)
+            seen["fp8"].add((f >> 16, (f & 0xffff) > 1))
+        r = bf16(pkg, M, N, K // 2)
+        if r == ROWS:
+            f = lib.ghip_rows_form(1, z(M), z(N), z(K // 2), NCU)
+            seen["bf16"].add((f >> 16, f >> 8 & 255, f & 255))
+        elif r == GEMM:
+            f = lib.ghip_bf16_gemm_form(z(M), z(N), NCU)
+            seen[GEMM].add((f >> 16, f & 0xffff))
+    assert seen[ROWS] <= set(test_gpu_rows.FP8.values())
+    assert seen["bf16"] <= set(test_gpu_rows.BF16.values())
+    assert seen[GEMM] <= set(test_gpu_bf16_gemm.SHAPES.values())
+    assert seen["fp8"] <= {(h, s > 1) for h, s in test_gpu_fp8_gemm.SHAPES.values()}
 
 
 QUEUED, FULL, STREAMS = range(3)

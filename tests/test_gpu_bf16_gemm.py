@@ -14,14 +14,22 @@ from tolerance import assert_close
 
 pytestmark = pytest.mark.gpu
 
-# (M, N, K): the tile the launcher picks on 256 CUs
-SHAPES = [(65, 8000, 64), (250, 2005, 128), (130, 4100, 1088),  # 64 x 64
-          (64, 20000, 192), (320, 4000, 448),                 # 64 x 128
-          (600, 4096, 320),                                   # 192 x 64
-          (1023, 4095, 128), (1024, 4096, 704),               # 128 x 128
-          (1100, 4104, 256),                                  # 192 x 128
-          (2047, 4096, 320),                                  # 256 x 128
-          (2048, 8185, 192)]                                  # 256 x 256
+# (M, N, K): the tile the library picks on 256 CUs, to which each case is held
+SHAPES = {(65, 8000, 64): (64, 64), (250, 2050, 128): (64, 64), (130, 4100, 1088): (64, 64),
+          (64, 20000, 192): (64, 128), (320, 4000, 448): (64, 128),
+          (600, 4096, 320): (192, 64),
+          (1023, 4095, 128): (128, 128), (1024, 4096, 704): (128, 128),
+          (1100, 4104, 256): (192, 128),
+          (2047, 4096, 320): (256, 128),
+          (2048, 8185, 192): (256, 256)}
+GEMM = 3                                                            # the route's number (ghip_internal.h)
+
+
+def on_gemm(ghip, M, N, K):
+    p, z = ctypes.c_void_p(1 << 20), [ctypes.c_size_t(v) for v in (M, N, K)]
+    assert ghip.ghip_bf16_linear_route(p, p, *z, 256) == GEMM
+    form = ghip.ghip_bf16_gemm_form(z[0], z[1], 256)
+    return form >> 16, form & 0xffff
 
 
 def run(ghip, w, x, pad):
@@ -39,6 +47,7 @@ def run(ghip, w, x, pad):
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
 def test_bf16_gemm_tiles(ghip, M, N, K):
+    assert on_gemm(ghip, M, N, K) == SHAPES[M, N, K]
     rng = np.random.default_rng(M * 31 + N * 7 + K)
     w = O.f32_to_bf16(rng.uniform(-4, 4, (N, K)).astype(np.float32))
     x = O.f32_to_bf16(rng.uniform(-4, 4, (M, K)).astype(np.float32))
@@ -51,6 +60,7 @@ def test_bf16_gemm_tiles(ghip, M, N, K):
 def test_bf16_gemm_unaligned_y(ghip):
     """y two bytes off a 16-byte boundary: the same values by 2-byte stores."""
     rng = np.random.default_rng(11)
+    on_gemm(ghip, 250, 2056, 256)
     w = O.f32_to_bf16(rng.uniform(-4, 4, (2056, 256)).astype(np.float32))
     x = O.f32_to_bf16(rng.uniform(-4, 4, (250, 256)).astype(np.float32))
     assert np.array_equal(run(ghip, w, x, 1), run(ghip, w, x, 8))
@@ -61,6 +71,7 @@ def test_bf16_gemm_not_finite(ghip):
     M and N re-read the last one and are not stored)."""
     rng = np.random.default_rng(12)
     M, N, K = 250, 2050, 128
+    on_gemm(ghip, M, N, K)
     w = O.f32_to_bf16(rng.uniform(1, 4, (N, K)).astype(np.float32))
     x = O.f32_to_bf16(rng.uniform(1, 4, (M, K)).astype(np.float32))
     x[M - 1, 5], w[N - 1, 7] = 0x7F80, 0x7FC0                       # +inf, NaN

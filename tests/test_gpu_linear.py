@@ -96,12 +96,11 @@ def test_fp8_battery(ghip, M, N, K):
                  floor_linear(codes, scales, x), "M%d N%d K%d" % (M, N, K))
 
 
-# prefill-sized M: the MFMA GEMM path (M >= 16, N % 256 == 0, K % 128 == 0),
-# incl. ragged row tiles, K = 128 and K = 16384 (o_proj), the DSA shapes of
-# c/gdsa.h:599-611,660-661 at M = s; M = 15 stays on the GEMV passes. Most
-# small-M shapes run split-K (fp32 partials summed in a fixed order):
-# (16, 256, 16384) with 64 splits of 2 k blocks, (64, 4096, 16384) with 12,
-# (2048, 512, 4096) with 6 on 128-row tiles; (513, 256, 128) cannot split
+# prefill-sized M, incl. ragged row counts, K = 128 and K = 16384 (o_proj), the
+# DSA shapes of c/gdsa.h:599-611,660-661 at M = s. On 256 CUs (300, 2048, 1536),
+# (256, 4096, 16384), (513, 256, 128), (64, 4096, 16384) and (2048, 512, 4096)
+# take the MFMA GEMM (test_gpu_fp8_gemm.py holds its bodies to their shapes),
+# the others the weight-streaming kernel
 GEMM = [(16, 512, 4096), (100, 1536, 4096), (300, 2048, 1536), (40, 16384, 1536),
         (256, 4096, 16384), (513, 256, 128), (15, 512, 1024), (17, 300, 512),
         (16, 256, 16384), (64, 4096, 16384), (2048, 512, 4096)]
@@ -123,10 +122,17 @@ def test_fp8_gemm_prefill_shapes(ghip, M, N, K):
     assert np.array_equal(got, gpu_linear(ghip, codes, scales, x))   # deterministic
 
 
+def routed(ghip, M, N, K, y=1 << 20):
+    """The FP8 linear's kernel on 256 CUs (ghip_internal.h's numbers)."""
+    p = ctypes.c_void_p(1 << 20)
+    return ghip.ghip_fp8_linear_route(p, p, ctypes.c_void_p(y), *[ctypes.c_size_t(v) for v in (M, N, K)], 256)
+
+
 def test_fp8_gemm_nan_codes_exact_decode(ghip):
     """Every code incl. 0x7F/0xFF through the GEMM path (the NaN scan
-    selects the exact integer decode)."""
-    M, N, K = 48, 512, 1024
+    selects the exact decode)."""
+    M, N, K = 300, 512, 1024
+    assert routed(ghip, M, N, K) == 3
     codes = (np.arange(N * K) & 0xFF).astype(np.uint8).reshape(N, K)
     rng = np.random.default_rng(5)
     scales = np.exp2(rng.uniform(-10, -4, (O.nblocks(N), O.nblocks(K)))).astype(np.float32)
@@ -162,11 +168,12 @@ def test_linear_dev_entry(ghip, pkg):
 
 
 def test_linear_dev_unaligned_y(ghip, pkg):
-    """The GEMM path (M >= 16) stores 16-byte vectors, so it needs a 16-byte
-    aligned y; a y two bytes off goes to the streaming GEMV (4 rows per
-    launch, 2-byte stores) instead. Checked at M = 32 against the oracle,
-    with the elements either side of y left untouched."""
-    M, N, K = 32, 1024, 2048
+    """The GEMM stores 16-byte vectors, so it needs a 16-byte aligned y; a y
+    two bytes off goes to the weight-streaming kernel instead (2-byte stores).
+    Checked at M = 300 against the oracle, with the elements either side of y
+    left untouched."""
+    M, N, K = 300, 1024, 2048
+    assert routed(ghip, M, N, K) == 3 and routed(ghip, M, N, K, (1 << 20) + 2) == 2
     c, s, x = synth_linear(pkg.load(), 0x53, M, N, K)
     want = O.fp8_linear(c, s, x, threads=8)
     guard = np.full(M * N + 16, 0x7E57, np.uint16)
@@ -177,7 +184,7 @@ def test_linear_dev_unaligned_y(ghip, pkg):
     got = G.host(dy, np.uint16, guard.shape)
     assert got[0] == 0x7E57 and np.all(got[1 + M * N:] == 0x7E57), "wrote outside y"
     assert_close(got[1:1 + M * N].reshape(M, N), want, floor_linear(c, s, x),
-                 "unaligned y, M=32")
+                 "unaligned y, M=300")
 
 
 def test_deterministic(ghip, pkg):
@@ -197,7 +204,7 @@ def test_bf16_gemm_golden(ghip, fx, man):
 
 
 def test_bf16_gemm_real_shapes(ghip):
-    """Real shapes (streaming MFMA GEMV, M in groups of <= 4) and ragged
+    """Real shapes (the streaming kernels) and ragged
     ones: O % 16 != 0, K = 64, K % 64 != 0 (the generic kernel)."""
     rng = np.random.default_rng(3)
     for (Oo, K) in [(2048, 4096), (4096, 2048), (288, 4096), (300, 64), (129, 200)]:
@@ -263,7 +270,7 @@ def test_fp8_hook_through_table_floors(ghip):
     M, the hook declines (nonzero: the engine runs its CPU kernel) and the
     offload counter does not move; the direct entry ignores the floors;
     without floors the hook runs, moves offload_fp8blk by one, and meets
-    the tolerance. Both the GEMV (M = 1) and GEMM (M = 32) paths."""
+    the tolerance. Both M = 1 and M = 32."""
     hooks = (ctypes.c_void_p * 2).in_dll(ghip, "apus_ghip_hooks")
     HookFp8 = ctypes.CFUNCTYPE(ctypes.c_int, *([ctypes.c_void_p] * 4 + [ctypes.c_size_t] * 3))
     rng = np.random.default_rng(0xF8)

@@ -15,21 +15,31 @@ from tolerance import assert_close
 
 pytestmark = pytest.mark.gpu
 
-# (M, N, K), the form picked on 256 CUs as rows of x / weight groups / K splits
-FP8 = [(1, 100, 128), (4, 6000, 512),                       # 4/1/4
-       (3, 4096, 16384), (4, 1000, 1152), (2, 33, 256),     # 4/1/8: x over 48 KB; 9 chunks; one
-       (8, 15000, 384), (5, 9000, 640),                     # 8/1/2
-       (7, 1000, 1024),                                     # 8/1/8
-       (13, 16383, 512),                                    # 16/2/4
-       (17, 1000, 896),                                     # 16/1/8, two row tiles
-       (16, 7000, 1024), (50, 2000, 1024),                  # 16/2/8
-       (24, 16383, 384), (33, 7000, 640),                   # 32/2/4
-       (64, 16380, 384), (65, 16001, 128),                  # 64/2/4
-       (300, 500, 256)]                                     # column remainder at prefill rows
-BF16 = [(1, 288, 1024), (8, 500, 64), (3, 20000, 192),      # 8/1/8, one chunk; 8/1/4
-        (12, 8200, 512), (9, 300, 128), (30, 2000, 576),    # 16/1/8
-        (16, 20000, 256),                                   # 16/2/4
-        (60, 2000, 1024)]                                   # 32/1/8
+# (M, N, K): the form the library picks on 256 CUs as rows of x, weight groups, K splits, to which each case is held
+FP8 = {(1, 100, 128): (4, 1, 8), (2, 33, 256): (4, 1, 8), (4, 1000, 1152): (4, 1, 8),    # one chunk; 9 chunks
+       (3, 4096, 16384): (4, 1, 8),                                                    # x over 48 KB
+       (3, 9001, 384): (4, 1, 4), (4, 6000, 512): (4, 1, 4), (1, 8551, 128): (4, 1, 2),
+       (7, 1000, 1024): (8, 1, 8), (5, 4285, 384): (8, 1, 4), (8, 15000, 384): (8, 1, 2), (5, 9000, 640): (8, 1, 2),
+       (17, 1000, 896): (16, 1, 8), (16, 7000, 1024): (16, 2, 8), (50, 2000, 1024): (16, 2, 8),
+       (13, 16383, 512): (16, 2, 4), (300, 500, 256): (16, 2, 4),
+       (1040, 99, 640): (32, 1, 8), (17, 4115, 640): (32, 2, 8), (24, 16383, 384): (32, 2, 4),
+       (33, 7000, 640): (32, 2, 4), (64, 16380, 384): (32, 2, 4), (65, 16001, 128): (32, 2, 4),
+       (33, 24854, 128): (64, 2, 4), (67, 7582, 640): (64, 2, 4), (100, 5569, 640): (64, 2, 4)}
+BF16 = {(1, 288, 1024): (8, 1, 8), (8, 500, 64): (8, 1, 8), (3, 20000, 192): (8, 1, 4),
+        (9, 300, 128): (16, 1, 8), (30, 2000, 576): (16, 1, 8), (17, 2188, 64): (16, 1, 4),
+        (40, 2100, 64): (16, 1, 4), (12, 8200, 512): (16, 2, 4), (16, 20000, 256): (16, 2, 4),
+        (60, 2000, 1024): (32, 1, 8), (17, 4140, 320): (32, 2, 8), (33, 4000, 320): (32, 2, 8),
+        (17, 8417, 128): (32, 2, 4), (31, 9000, 192): (32, 2, 4)}
+ROWS = 2                                                            # the route's number (ghip_internal.h)
+
+
+def held_to_form(ghip, bf, M, N, K, form):
+    """The dispatch's choices are host code over estimates: a changed one must
+    not take a form's cases away unseen."""
+    p, z = ctypes.c_void_p(1 << 20), [ctypes.c_size_t(v) for v in (M, N, K)]
+    route = ghip.ghip_bf16_linear_route(p, p, *z, 256) if bf else ghip.ghip_fp8_linear_route(p, p, p, *z, 256)
+    got = ghip.ghip_rows_form(bf, *z, 256)
+    assert route == ROWS and (got >> 16, got >> 8 & 255, got & 255) == form
 
 
 def guarded(ghip, call, M, N, pad):
@@ -60,6 +70,7 @@ def fp8_inputs(M, N, K, nan_codes):
 @pytest.mark.parametrize("M,N,K", FP8)
 def test_rows_fp8(ghip, M, N, K):
     """Clean codes: both decodes give the same bits; then NaN codes."""
+    held_to_form(ghip, 0, M, N, K, FP8[M, N, K])
     for nan_codes in (False, True):
         codes, scales, x = fp8_inputs(M, N, K, nan_codes)
         w = O.dequant(codes, scales, threads=8)
@@ -73,6 +84,11 @@ def test_rows_fp8(ghip, M, N, K):
 
 @pytest.mark.parametrize("M,N,K", BF16)
 def test_rows_bf16(ghip, M, N, K):
+    held_to_form(ghip, 1, M, N, K, BF16[M, N, K])
+    check_bf16(ghip, M, N, K)
+
+
+def check_bf16(ghip, M, N, K):
     rng = np.random.default_rng(M * 1013 + N * 17 + K)
     w = O.f32_to_bf16(rng.uniform(-4, 4, (N, K)).astype(np.float32))
     x = O.f32_to_bf16(rng.uniform(-4, 4, (M, K)).astype(np.float32))
@@ -91,7 +107,7 @@ def test_few_long_bf16_rows(ghip, M, N, K):
     chunks left after its loop of three, and row remainders."""
     assert ghip.ghip_bf16_linear_route(ctypes.c_void_p(16), ctypes.c_void_p(16), ctypes.c_size_t(M), ctypes.c_size_t(N),
                                        ctypes.c_size_t(K), 256) == 1
-    test_rows_bf16(ghip, M, N, K)
+    check_bf16(ghip, M, N, K)
 
 
 def test_rows_not_finite(ghip):
