@@ -21,7 +21,7 @@ extern "C" {
 #define GHIP_MAX_THREADS ((size_t)0xffffffffu)
 
 /* K1: out[O,K] bf16 = bf16(e4m3(codes) * scale of the 128x128 block).
- * exact != 0 selects the integer decode (required for NaN codes). */
+ * exact != 0 selects the exact decode (required for NaN codes). */
 hipError_t ghip_launch_dequant(const uint8_t *codes, const float *scales,
                                uint16_t *out, size_t O, size_t K, int exact,
                                hipStream_t st);
@@ -118,7 +118,8 @@ typedef struct {
     float *w_out;
 } GhipRouterArgs;
 
-/* Streaming GEMV set-up (dynamic-LDS limits, persistent grid bound). */
+/* Set-up of the linear kernels (dynamic-LDS limits, the CU count of their
+ * grids and routes). */
 hipError_t ghip_linear_init(uint32_t n_cu);
 
 /* Raise the decode kernel's dynamic-LDS limit (once per process). */
@@ -273,9 +274,12 @@ typedef struct {
 int ghip_container_layer(const char *dir, int layer, size_t slab_bytes,
                          GhipSlabRec **out, int *n_out, char *err, size_t errcap);
 
+/* Copy n bytes (at most 1 GiB) between 16-byte aligned addresses, either of
+ * them in pinned host memory, by a kernel. */
+hipError_t ghip_launch_copy16(void *dst, const void *src, size_t n, hipStream_t st);
+
 /* Fill n u32 words with value (a kernel, not a memset, so callers may
  * capture it in a graph). */
-hipError_t ghip_launch_copy16(void *dst, const void *src, size_t n, hipStream_t st);
 hipError_t ghip_launch_fill_u32(uint32_t *p, size_t n, uint32_t value,
                                 hipStream_t st);
 

@@ -52,8 +52,8 @@ __device__ __forceinline__ float wave_sum(float v) {
  * serve all of them, and the loads of four k steps are in flight together. Each
  * sum is its lanes' k = lane, lane + 64, ... in order and then the wave's, for
  * any MR. Bound by issue (any alignment: loads of one element): 2000 x 2001, M
- * = 64, FP8 73 us and BF16 46 (a wave a row of x 183 and 132); M = 1 8.4 and
- * 3.7 (10.8 and 5.8, each load waited for). */
+ * = 64, weights from HBM, FP8 52 us and BF16 37 (a wave a row of x 222 and
+ * 147), M = 3 15.0 and 5.9 (22.7 and 12.5, each load waited for). */
 template <bool BF, int MR>
 __global__ __launch_bounds__(256) void k_linear_any(
     const void *__restrict__ W, const float *__restrict__ S,

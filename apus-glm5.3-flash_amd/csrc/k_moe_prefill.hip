@@ -1107,8 +1107,10 @@ __device__ __forceinline__ void pf_rows_tile(const PfTile &t, uint8_t *lds) {
  * holds a backlog; tiles of up to 128 rows split each stage's k between the
  * wave halves instead of the rows, which dequantizes every weight once, and
  * tiles of up to 16 rows are weight streams. Against one wave per SIMD over
- * all rows (288 experts, top-8): T = 512 1381 -> 1269 us, T = 2048 1712 ->
- * 1651 and, Zipf 1.1, 1867 -> 1773, T = 4096 2311 -> 2240.
+ * all rows (288 experts, top-8): T = 512 1381 -> 1307 us, T = 2048 1783 ->
+ * 1714 and, Zipf 1.1, 1956 -> 1849, T = 4096 2418 -> 2306; but T = 1024, tiles
+ * of 17 to 32 rows, 1457 -> 1477 (weight streams of 32 rows took 1560 there,
+ * row halves 1807).
  * A grab past a queue's end moves on to the next queue, so every workgroup
  * leaves the loop after at most one failed grab per queue. */
 template <int MODE, bool FULL>
@@ -1265,8 +1267,7 @@ __global__ __launch_bounds__(512, 1) void k_pf_gemm(
  * (mod 8/R), so each XCD's L2 holds 1/R of X's rows and (R/8) of the
  * weights; the launcher picks R to minimize the bytes fetched into the
  * L2s, (8/R) |X| + R |W|. exact_dev: NULL or a device flag, nonzero when W
- * holds a NaN code (0x7F/0xFF) and the exact integer decode must be
- * used. */
+ * holds a NaN code (0x7F/0xFF) and the exact decode must be used. */
 __global__ __launch_bounds__(256, 1) void k_fp8_gemm(
     const uint8_t *__restrict__ codes, const float *__restrict__ scales,
     const uint16_t *__restrict__ x, uint16_t *__restrict__ y, float *__restrict__ part,

@@ -15,11 +15,12 @@
  * items of their own.
  *
  * HBM bounds it: 6.2-6.3 TB/s at T = 12, top-8 of 288 (1.39 GB of gate/up in
- * 224 us, 0.69 GB of down in 110). Two workgroups a CU (64 KB of LDS, 128
+ * 224 us, 0.69 GB of down in 110; by the counters the bytes fetched are the
+ * weights' and the matrix cores are busy 9% of the cycles). Two workgroups a CU (64 KB of LDS, 128
  * registers a lane) keep loads in flight across items, and small items keep
  * all CUs busy from the first token on, where the tile GEMM's 1 MB items and
- * ~25 us a launch do not: T = 2 133 -> 82 us, T = 12 412 -> 350, 16 experts
- * of 1024/512 at T = 16 66 -> 22.
+ * ~25 us a launch do not: T = 2 135 -> 79 us, T = 12 426 -> 345, 16 experts
+ * of 1024/512 at T = 16 66 -> 20.
  */
 #include "ghip_device.h"
 #include "ghip_internal.h"

@@ -132,16 +132,18 @@ int apus_ghip_fp8blk_dequant(const uint8_t *codes, const float *scales,
 
 /* Device-pointer variants (asynchronous on `stream`, a hipStream_t; NULL =
  * the null stream). exact: 0 = fast decode (caller guarantees no 0x7F/0xFF
- * code), 1 = exact integer decode, -1 = scan the codes first and pick.
+ * code), 1 = exact decode (those two codes +-480), -1 = scan the codes first
+ * and pick.
  * These share process-wide device state: the NaN-scan flag (exact = -1),
  * the exact-decode flag word and the split-K partial buffer of the FP8 GEMM
  * path (M >= 16). Calls must therefore not overlap in time: issue them on
  * one stream, and do not run them concurrently with the host-pointer
  * entry points (which use the backend's own stream).
  * Alignment: with 16-byte aligned codes (w) and x and K % 128 == 0 (K % 64
- * == 0 for BF16 weights) the weights are read once per up to 64 rows of x
- * (the streaming kernels), or once per row tile (the MFMA GEMMs, at more
- * rows; for FP8 weights N % 256 == 0 and a 16-byte aligned y too); other
+ * == 0 for BF16 weights) the weights are read once per up to 64 rows of x (32
+ * for BF16 weights; the streaming kernels), or once per row tile (the MFMA
+ * GEMMs, at more rows or with little K; for FP8 weights N % 256 == 0 and a
+ * 16-byte aligned y too); other
  * shapes and alignments take a slow general kernel (same results within the
  * tolerance). */
 int apus_ghip_fp8blk_dequant_dev(const uint8_t *codes, const float *scales,
