@@ -359,7 +359,7 @@ def test_config4_two_layers(ghip, pkg):
         cnt = np.bincount(runs[0][1].ravel(), minlength=E)
         print("config4 rows per expert: min %d mean %.1f max %d" % (cnt.min(), cnt.mean(),
                                                                    cnt.max()))
-        assert cnt.sum() >= E * 128           # the full-tile (8-wave) bodies
+        assert cnt.sum() >= E * 128           # the full-tile form
         for s, (x, idx, w, dx, di, dw, do) in zip(stores, runs):
             assert ghip.apus_ghip_moe_prefill_dev(s, G.vp(dx), T, G.vp(di), G.vp(dw), k,
                                                   G.vp(do), G.stream()) == 0, \

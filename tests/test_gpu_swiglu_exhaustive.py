@@ -17,11 +17,15 @@ without a non-finite x, which would turn every row's 0 * x into NaN.
   g = -inf                 h = -inf * 0 = NaN: its own token, all NaN
   g = NaN (254 codes)      x[0] = NaN: its own token, all outputs NaN
 
-Paths: the decode (one launch per token) and both prefill kernels (all
-tokens in one call; one expert of a 3-expert bank takes the one-wave-per-
-SIMD bodies, of a 1-expert bank the two-waves-per-SIMD bodies: 256-row
-and 31-row tiles). Every finite output is compared bitwise and the
-mismatches are recorded per path."""
+Paths: the decode (one launch per token) and every form of the prefill
+(all experts of a bank hold the same weights, so the tokens may be spread
+over them): full tiles, queued tiles with more than 128 rows, with 17 to
+128 rows (each stage's k split between the wave halves) and with at most
+16 (weight streams without a ring), and the weight streams of calls with
+few rows. Every finite output is compared bitwise and the mismatches are
+recorded per path."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -29,6 +33,7 @@ import oracle as O
 from tolerance import record
 from test_gpu_moe import open_store
 from test_gpu_prefill import prefill
+from test_gpu_prefill_forms import FULL, QUEUED, ROWS
 
 pytestmark = pytest.mark.gpu
 
@@ -142,17 +147,28 @@ def test_swiglu_exhaustive_decode(ghip, case):
         ghip.apus_ghip_store_close(s)
 
 
-@pytest.mark.parametrize("E,body", [(3, "4wave"), (1, "8wave")])
-def test_swiglu_exhaustive_prefill(ghip, case, E, body):
+# bank, tokens a call (0: all 287), experts they are spread over, the form
+@pytest.mark.parametrize("E,step,spread,form", [
+    pytest.param(1, 0, 1, FULL, id="full"),
+    pytest.param(3, 0, 1, QUEUED, id="queued"),
+    pytest.param(4, 0, 4, QUEUED, id="queued_72_rows"),
+    pytest.param(24, 0, 24, QUEUED, id="queued_12_rows"),
+    pytest.param(3, 48, 3, ROWS, id="streams")])
+def test_swiglu_exhaustive_prefill(ghip, case, E, step, spread, form, request):
     slab, x, what, want = case
     T = x.shape[0]
-    assert (T >= E * 128) == (body == "8wave")      # the launcher's body choice
+    step = step or T
     s = open_store(ghip, E, DIM, INTER, LIMIT)
     try:
         for e in range(E):
             assert ghip.apus_ghip_store_put(s, e, O.ptr(slab), slab.nbytes) == 0
-        idx = np.zeros((T, 1), np.int32)
-        w = np.ones((T, 1), np.float32)
-        compare(prefill(ghip, s, x, idx, w), want, what, "prefill_" + body)
+        got = []
+        for t in range(0, T, step):
+            xt = np.ascontiguousarray(x[t:t + step])
+            n = len(xt)
+            assert ghip.ghip_moe_prefill_form(DIM, INTER, E, 1, ctypes.c_size_t(n)) == form
+            idx = (np.arange(n, dtype=np.int32) % spread).reshape(n, 1)
+            got.append(prefill(ghip, s, xt, idx, np.ones((n, 1), np.float32)))
+        compare(np.concatenate(got), want, what, "prefill_" + request.node.callspec.id)
     finally:
         ghip.apus_ghip_store_close(s)
