@@ -429,8 +429,17 @@ extern "C" hipError_t ghip_launch_fp8_linear(const uint8_t *codes,
     switch (ghip_fp8_linear_route(codes, x, y, M, O, K, g_gs_ncu)) {
     case GHIP_ROUTE_GEMV:
         return launch_gemv<false>(codes, scales, x, y, M, O, K, exact_dev, ev0, ev1, st);
-    case GHIP_ROUTE_GEMM:
-        return ghip_launch_fp8_gemm(codes, scales, x, y, M, O, K, exact_dev, g_gs_ncu, ev, st);
+    case GHIP_ROUTE_GEMM: {
+        const hipError_t e =
+            ghip_launch_fp8_gemm(codes, scales, x, y, M, O, K, exact_dev, g_gs_ncu, ev, st);
+        /* no memory for the K splits, or a capture that would have to allocate
+         * it: below 256 rows the form that needs none runs */
+        if ((e != hipErrorOutOfMemory && e != hipErrorStreamCaptureUnsupported) || M >= 256
+            || !ghip_rows_fits(0, M, O, K, codes, x))
+            return e;
+        (void)hipGetLastError();
+    }
+    /* fall through */
     case GHIP_ROUTE_ROWS:
         return ghip_launch_rows(0, codes, scales, x, y, M, O, K, exact_dev, g_gs_ncu, ev0, ev1,
                                 st);

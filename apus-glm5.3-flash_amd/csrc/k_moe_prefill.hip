@@ -1603,10 +1603,39 @@ extern "C" int ghip_fp8_gemm_fits(size_t M, size_t N, size_t K, const void *code
 }
 
 /* split-K partials: one device buffer, grown on demand, kept for the
- * process (launches on one device are stream-ordered users of it) */
+ * process (launches on one device are stream-ordered users of it). A graph
+ * that captured a launch replays into the buffer it saw, so from then on that
+ * one is never freed: growth takes another of at least twice its size, and
+ * all of them together stay under twice the largest. */
 static float *g_part;
 static size_t g_part_cap;
+static bool g_part_captured;
 #define GHIP_SPLITK_MAX_BYTES ((size_t)256 << 20)
+
+/* Makes g_part hold `need` bytes for a launch on st. A capturing stream cannot
+ * allocate: hipErrorStreamCaptureUnsupported, the capture left as it was. */
+static hipError_t f8_part(size_t need, hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(st, &cs);
+    if (e != hipSuccess) (void)hipGetLastError();        /* the launch reports it */
+    const bool captures = e == hipSuccess && cs != hipStreamCaptureStatusNone;
+    if (need > g_part_cap) {
+        if (captures) return hipErrorStreamCaptureUnsupported;
+        size_t n = need;
+        if (g_part_captured) {
+            if (n < 2 * g_part_cap) n = 2 * g_part_cap;
+        } else if (g_part) {
+            (void)hipFree(g_part);
+        }
+        g_part = nullptr;
+        g_part_cap = 0;
+        g_part_captured = false;
+        if ((e = hipMalloc((void **)&g_part, n)) != hipSuccess) return e;
+        g_part_cap = n;
+    }
+    if (captures) g_part_captured = true;
+    return hipSuccess;
+}
 
 /* How the launch divides M x N x K: tile height, K splits, XCD grid R x
  * (8 / R), workgroups. */
@@ -1717,22 +1746,13 @@ extern "C" hipError_t ghip_launch_fp8_gemm(const uint8_t *codes, const float *sc
     if (!ghip_fp8_gemm_fits(M, N, K, codes, x, y) || n_cu == 0 || n_cu % 8)
         return hipErrorInvalidValue;
     const F8Plan p = f8_plan(M, N, K, n_cu);
-    if (p.S > 1) {
-        const size_t need = (size_t)p.S * M * N * sizeof(float);
-        if (need > g_part_cap) {
-            if (g_part) (void)hipFree(g_part);
-            g_part = nullptr;
-            g_part_cap = 0;
-            hipError_t e = hipMalloc((void **)&g_part, need);
-            if (e != hipSuccess) return e;
-            g_part_cap = need;
-        }
-    }
+    hipError_t e;
+    if (p.S > 1 && (e = f8_part((size_t)p.S * M * N * sizeof(float), st)) != hipSuccess) return e;
     hipEvent_t e0 = ev ? ev[0] : nullptr, e1 = ev ? ev[1] : nullptr;
     GHIP_LAUNCH(e0, p.S > 1 ? nullptr : e1, k_fp8_gemm, dim3(p.grid), dim3(256), PF_LDS, st, codes,
                 scales, x, y, g_part, (uint32_t)M, (uint32_t)N, (uint32_t)K, p.bm, p.S, p.R,
                 exact_dev);
-    hipError_t e = hipGetLastError();
+    e = hipGetLastError();
     if (e != hipSuccess || p.S == 1) return e;
     const size_t n = M * N;                          /* N % 256 == 0: n % 4 == 0 */
     GHIP_LAUNCH(nullptr, e1, k_splitk_sum, dim3((uint32_t)((n / 4 + 255) / 256)), dim3(256),

@@ -138,7 +138,10 @@ int apus_ghip_fp8blk_dequant(const uint8_t *codes, const float *scales,
  * the exact-decode flag word and the split-K partial buffer of the FP8 GEMM
  * path (M >= 16). Calls must therefore not overlap in time: issue them on
  * one stream, and do not run them concurrently with the host-pointer
- * entry points (which use the backend's own stream).
+ * entry points (which use the backend's own stream). A capture cannot grow
+ * the partial buffer: below 256 rows it then takes the kernel that needs none;
+ * from 256 rows on it fails unless an earlier call of the size has run. A
+ * captured call's buffer is kept until the process ends.
  * Alignment: with 16-byte aligned codes (w) and x and K % 128 == 0 (K % 64
  * == 0 for BF16 weights) the weights are read once per up to 64 rows of x (32
  * for BF16 weights; the streaming kernels), or once per row tile (the MFMA
